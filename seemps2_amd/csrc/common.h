@@ -147,10 +147,9 @@ int64_t polar_svd_bytes(int64_t Lg, int64_t l);
 int polar_svd(int64_t Lg, int64_t l, const double2* W, int64_t ldw, double2* U, double* S,
               double2* VH, const int64_t** tiny_dev, const int** conv_dev, void* work,
               int64_t work_bytes, hipStream_t stream);
-int qr_factor(double2* A, int64_t len, int64_t ncol, int nb_max, double2* Vall, double2* Tall,
-              double2* tau, double2* Z, double2* ks, int64_t ks_elems, hipStream_t stream);
-int qr_apply_q(double2* Y, int64_t len, int64_t ny, int64_t ncol, int nb_max, const double2* Vall,
-               const double2* Tall, double2* Z, double2* ks, int64_t ks_elems,
-               hipStream_t stream);
+int qr_factor(double2* A, int64_t len, int64_t ncol, double2* Vall, double2* tau,
+              hipStream_t stream);
+int qr_apply_q(double2* Y, int64_t len, int64_t ny, int64_t ncol, const double2* Vall,
+               const double2* tau, hipStream_t stream);
 
 }  // namespace seemps

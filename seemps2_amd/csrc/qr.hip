@@ -1,358 +1,437 @@
-// Blocked Householder QR of a column-major working matrix (FP64 complex), used
-// to precondition the one-sided Jacobi SVD (Jacobi on R^H converges in a few
-// sweeps even for strongly graded spectra, where Jacobi on A needs tens).
+// Householder QR of a column-major working matrix (FP64 complex), used to
+// precondition the one-sided Jacobi SVD (Jacobi on R^H converges in a few
+// sweeps even for strongly graded spectra, where Jacobi on A needs tens) and
+// to orthonormalise sketches.
 //
 // Storage: A_cm holds ncol columns of length len (len >= ncol), column c at
-// A_cm + c * len.  After qr_factor, column c holds R[0..c, c] in rows 0..c and
-// the Householder vector v_c (implicit leading 1) in rows c+1..len-1.  Each
-// panel of NB columns keeps an explicit copy of its vectors (Vp, NB x L with
-// L = len - j0, unit diagonal, zeros above) and the compact-WY factor T
-// (NB x NB upper triangular) so that H_j0 ... H_j0+NB-1 = I - V T V^H.
-// The panel is factorised by one workgroup; trailing updates and the
-// application of Q are complex GEMMs on the FP64 matrix cores.
+// A_cm + c * len.  qr_factor leaves R[0..c, c] in rows 0..c of column c (the
+// rows below are scratch), tau, and the reflectors explicitly: row c of Vall
+// (length len) is v_c, zeros above row c included.
 //
-// Reflector convention (LAPACK zlarfg): H = I - tau v v^H with
-// H^H [alpha; x] = [beta; 0], beta real.
+// Both kernels keep columns in registers, one column's rows spread over the 64
+// lanes of a wavefront, so a dot product is a few FMAs per lane and one
+// wavefront reduction (wave.h).  A panel is one workgroup of 16 wavefronts
+// with one barrier per column; the trailing columns then take the panel's
+// reflectors one after the other in one launch, every column by itself (no
+// compact-WY factor, no GEMMs).
+//
+// Reflector convention: H = I - tau v v^H with H^H [alpha; x] = [beta; 0], beta
+// real of the sign opposite to Re alpha, v = [alpha - beta; x] (not scaled to a
+// leading 1: that needs a division per column and nothing reads it) and
+// tau = -1 / (beta conj(alpha - beta)).
 #include <cmath>
 
-#include "common.h"
+#include "jacobi_inner.h"
+#include "wave.h"
 
 namespace seemps {
 namespace {
 
-constexpr int QR_THREADS = 256;
+struct Reflector {
+  double beta;
+  double2 d, tau;  // alpha - beta, tau
+  bool any;        // false: H = I
+};
 
-__device__ double2 block_reduce_sum(double2 v, double2* red) {
-  for (int off = 32; off > 0; off >>= 1) {
-    v.x += __shfl_down(v.x, off, 64);
-    v.y += __shfl_down(v.y, off, 64);
+// A column of squared norm below 1e-300 (the squares lose their digits there)
+// gets no reflector; NaN does, and spreads.
+__device__ __forceinline__ Reflector make_reflector(double2 alpha, double xnorm2) {
+  Reflector h;
+  h.beta = alpha.x;
+  h.d = h.tau = make_double2(0.0, 0.0);
+  const double s = cabs2(alpha) + xnorm2;
+  h.any = !(xnorm2 == 0.0 && alpha.y == 0.0) && !(s < 1e-300);
+  if (h.any) {
+    const double r = jac::rsqrt_nr(s), sg = (alpha.x >= 0.0) ? -1.0 : 1.0;
+    h.beta = sg * (s * r);
+    h.d = make_double2(alpha.x - h.beta, alpha.y);
+    const double q = jac::rcp_nr(cabs2(h.d)), ib = -sg * r;  // 1 / |d|^2, -1 / beta
+    h.tau = make_double2((h.d.x * ib) * q, (h.d.y * ib) * q);
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double2 s = make_double2(0.0, 0.0);
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s = cadd(s, red[w]);
-    red[8] = s;
+  return h;
+}
+
+// Panel of nb <= NW CPW columns from j0 on, L = len - j0 <= 64 RPT rows.
+// Wavefront w holds columns w, w + NW, ... (CPW of them), lane l rows l,
+// l + 64, ... (RPT).  Step j: the unscaled column j is in LDS (published by its
+// owner at the end of the step before); every wavefront forms its norm below
+// the diagonal and its dot products with the wavefront's own later columns,
+// derives the reflector (redundantly, the same arithmetic everywhere) and
+// updates those columns in registers; the owner of column j + 1 publishes it.
+// One barrier per column.
+//
+// Bound by instruction issue on one CU, half of it the reductions (14
+// instructions a column against 8 FMAs a row and column).  64 columns of 64
+// rows take 80 us, 16 of 512 rows 23 us; with the panel in LDS instead (every
+// update a read and a write there) 16 columns took 54 and 64 us.  Eight
+// wavefronts: each derives the reflector by itself, and 16 of them spent 125 us
+// on the 64 x 64 panel.
+template <int NW, int RPT, int CPW>
+__global__ __launch_bounds__(64 * NW) void qr_panel(double2* __restrict__ A, int64_t len,
+                                                             int64_t j0, int nb,
+                                                             double2* __restrict__ tau,
+                                                             double2* __restrict__ Vall) {
+  __shared__ double2 xs[2][64 * RPT];
+  __shared__ double2 s_tau[NW * CPW];
+  __shared__ double s_beta[NW * CPW];
+  const int L = (int)(len - j0);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double2 a[CPW][RPT];
+#pragma unroll
+  for (int i = 0; i < CPW; ++i) {
+    const int c = wv + NW * i;
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const int row = lane + 64 * r;
+      a[i][r] = (c < nb && row < L) ? A[(j0 + c) * len + j0 + row] : make_double2(0.0, 0.0);
+    }
+  }
+  if (wv == 0) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) xs[0][lane + 64 * r] = a[0][r];
   }
   __syncthreads();
-  const double2 s = red[8];
+#pragma unroll
+  for (int i = 0; i < CPW; ++i) {
+    for (int w = 0; w < NW; ++w) {
+      const int j = NW * i + w;
+      if (j >= nb) break;
+      const double2* xb = xs[j & 1];
+      double2 x[RPT];
+      double nn = 0.0;
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        x[r] = (lane + 64 * r > j) ? xb[lane + 64 * r] : make_double2(0.0, 0.0);
+        nn += cabs2(x[r]);
+      }
+      const double2 alpha = xb[j];
+      double2 d[CPW];
+#pragma unroll
+      for (int k = 0; k < CPW; ++k) {
+        d[k] = make_double2(0.0, 0.0);
+        if (k < i) continue;
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) d[k] = cfmac(x[r], a[k][r], d[k]);
+      }
+      nn = wave::sum(nn);
+#pragma unroll
+      for (int k = i; k < CPW; k += 2) {
+        if (k + 1 < CPW)
+          wave::sum4(d[k], d[k + 1]);
+        else
+          d[k] = wave::sum2(d[k]);
+      }
+      const Reflector h = make_reflector(alpha, nn);
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+        if (lane + 64 * r == j) x[r] = h.d;  // x is v from here on
+      if (h.any) {
+        // c <- c - conj(tau) (v^H c) v,  v^H c = x^H c + conj(d) c[j]
+        const double2 ct = make_double2(h.tau.x, -h.tau.y);
+#pragma unroll
+        for (int k = i; k < CPW; ++k) {
+          if (k == i && wv <= w) continue;  // column j itself or an earlier one
+          const double2 cj = make_double2(wave::bcast(a[k][(NW * i) / 64].x, j & 63),
+                                          wave::bcast(a[k][(NW * i) / 64].y, j & 63));
+          const double2 f = cmul(ct, cfmac(h.d, cj, d[k]));
+          const double2 g = make_double2(-f.x, -f.y);
+#pragma unroll
+          for (int r = 0; r < RPT; ++r) a[k][r] = cfma(g, x[r], a[k][r]);
+        }
+      }
+      if (wv == w) {
+        // column j is done: R above the diagonal, the reflector from it on
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+          if (lane + 64 * r >= j) a[i][r] = x[r];
+        if (lane == 0) {
+          s_beta[j] = h.beta;
+          s_tau[j] = h.tau;
+        }
+      }
+      // the next column's owner publishes it
+      const int wn = (w + 1) % NW;
+      if (wv == wn) {
+        double2* nx = xs[(j + 1) & 1];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) {
+          if (w + 1 < NW)
+            nx[lane + 64 * r] = a[i][r];
+          else if (i + 1 < CPW)
+            nx[lane + 64 * r] = a[i + 1 < CPW ? i + 1 : i][r];
+        }
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < CPW; ++i) {
+    const int c = wv + NW * i;
+    if (c >= nb) continue;
+    double2* v = Vall + (j0 + c) * len;
+    for (int64_t row = lane; row < j0; row += 64) v[row] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const int row = lane + 64 * r;
+      if (row < L) v[j0 + row] = (row < c) ? make_double2(0.0, 0.0) : a[i][r];
+      if (row < L && row <= c)
+        A[(j0 + c) * len + j0 + row] = (row < c) ? a[i][r] : make_double2(s_beta[c], 0.0);
+    }
+    if (lane == 0) tau[j0 + c] = s_tau[c];
+  }
+}
+
+// Row q of a matrix with L double2 a row, as a buffer resource: reads past the
+// row's end give zero, so the lanes need no bounds tests (a test would put each
+// load behind a branch, and the loads ahead would wait for one another).
+__device__ __forceinline__ double2 row_load(__amdgpu_buffer_rsrc_t row, int elem) {
+  const auto w = __builtin_amdgcn_raw_buffer_load_b128(row, elem * 16, 0, 0);
+  return make_double2(__hiloint2double((int)w[1], (int)w[0]), __hiloint2double((int)w[3], (int)w[2]));
+}
+
+// Reflectors j1 - 1 .. j0 (FORWARD: j0 .. j1 - 1, adjoint) on the columns of Y
+// (ny of length len), rows r0 .. len - 1 (L <= 64 RPT; the reflectors are zero
+// above r0).  One wavefront per CW columns, its rows in registers; the next
+// reflectors are loaded while one is applied.  Bound by the chain of the dot
+// product, its reduction and the update: 0.31 us a reflector at 512 rows (8 us
+// for a panel's 16 on the trailing columns, 160 us for Q of 512 reflectors on
+// 512 columns; as compact-WY GEMMs three launches took 20 us a panel).
+template <int RPT, int CW, bool FORWARD>
+__global__ __launch_bounds__(64) void qr_reflect(double2* __restrict__ Y, int64_t len, int64_t ny,
+                                                 int64_t r0, int64_t j0, int64_t j1,
+                                                 const double2* __restrict__ tau,
+                                                 const double2* __restrict__ Vall) {
+  const int lane = threadIdx.x;
+  const int L = (int)(len - r0);
+  const int64_t c0 = (int64_t)blockIdx.x * CW;
+  // reflectors loaded ahead of the one applied (the registers hold no more of
+  // them at 1024 rows)
+  constexpr int AHEAD = RPT <= 8 ? 2 : 1;
+  double2 y[CW][RPT], v[AHEAD][RPT];
+  const int nq = (int)(j1 - j0);
+  const double2* vrow = Vall + (FORWARD ? j0 : j1 - 1) * len + r0;
+  const double2* trow = tau + (FORWARD ? j0 : j1 - 1);
+  auto load_v = [&](int q, double2* vq) {
+    const int64_t qq = q < nq ? q : nq - 1;
+    const auto row = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(vrow + (FORWARD ? qq : -qq) * len), 0, L * 16, 0x00027000);
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) vq[r] = row_load(row, lane + 64 * r);
+  };
+#pragma unroll
+  for (int p = 0; p < AHEAD; ++p) load_v(p, v[p]);
+#pragma unroll
+  for (int k = 0; k < CW; ++k)
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const int row = lane + 64 * r;
+      y[k][r] = (c0 + k < ny && row < L) ? Y[(c0 + k) * len + r0 + row] : make_double2(0.0, 0.0);
+    }
+  for (int qb = 0; qb < nq; qb += 64) {
+    // 64 tau in the lanes, one readlane each
+    const int ql = min(qb + lane, nq - 1);
+    double2 tl = trow[FORWARD ? ql : -ql];
+    if (FORWARD) tl.y = -tl.y;
+    // past the last reflector tau = 0 (H = I), so that no step is conditional
+    if (qb + lane >= nq) tl = make_double2(0.0, 0.0);
+    const int qe = min(64, nq - qb);
+    for (int q0 = 0; q0 < qe; q0 += AHEAD) {
+#pragma unroll
+      for (int p = 0; p < AHEAD; ++p) {
+        double2 u[RPT], d[CW];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) u[r] = v[p][r];
+        load_v(qb + q0 + p + AHEAD, v[p]);
+#pragma unroll
+        for (int k = 0; k < CW; ++k) {
+          d[k] = make_double2(0.0, 0.0);
+#pragma unroll
+          for (int r = 0; r < RPT; ++r) d[k] = cfmac(u[r], y[k][r], d[k]);
+        }
+        if (CW == 2)
+          wave::sum4(d[0], d[CW - 1]);
+        else
+          d[0] = wave::sum2(d[0]);
+        const double2 t = make_double2(wave::bcast(tl.x, q0 + p), wave::bcast(tl.y, q0 + p));
+#pragma unroll
+        for (int k = 0; k < CW; ++k) {
+          const double2 f = cmul(t, d[k]), g = make_double2(-f.x, -f.y);
+#pragma unroll
+          for (int r = 0; r < RPT; ++r) y[k][r] = cfma(g, u[r], y[k][r]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < CW; ++k)
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      const int row = lane + 64 * r;
+      if (c0 + k < ny && row < L) Y[(c0 + k) * len + r0 + row] = y[k][r];
+    }
+}
+
+// ---- columns longer than the registers hold (more than 64 REG_RPT rows) ------
+
+constexpr int REG_RPT = 16;
+constexpr int LONG_NB = 16;
+
+__device__ double2 block_sum(double2 v, double2* red) {
+  v = wave::sum2(v);
   __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double2 s = make_double2(0.0, 0.0);
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s = cadd(s, red[w]);
   return s;
 }
 
-// Factorise the panel of nb columns starting at j0; write Vp (nb x L) and T.
-__global__ __launch_bounds__(QR_THREADS) void qr_panel_kernel(double2* __restrict__ A, int64_t len,
-                                                              int64_t j0, int nb,
-                                                              double2* __restrict__ tau,
-                                                              double2* __restrict__ Vp,
-                                                              double2* __restrict__ T) {
+// y <- y - f (v^H y) v over rows [lo, len) by one workgroup, v and y in memory.
+__device__ void long_reflect(double2* __restrict__ y, const double2* __restrict__ v, int64_t lo,
+                             int64_t len, double2 f, double2* red) {
+  double2 d = make_double2(0.0, 0.0);
+  for (int64_t r = lo + threadIdx.x; r < len; r += blockDim.x) d = cfmac(v[r], y[r], d);
+  d = cmul(f, block_sum(d, red));
+  for (int64_t r = lo + threadIdx.x; r < len; r += blockDim.x) {
+    const double2 p = cmul(d, v[r]);
+    y[r] = make_double2(y[r].x - p.x, y[r].y - p.y);
+  }
+}
+
+// Panel of nb columns from j0 on, columns in memory, one workgroup.
+__global__ __launch_bounds__(1024) void qr_panel_long(double2* __restrict__ A, int64_t len,
+                                                      int64_t j0, int nb,
+                                                      double2* __restrict__ tau,
+                                                      double2* __restrict__ Vall) {
   __shared__ double2 red[16];
-  __shared__ double2 s_tau[32];
-  const int tid = threadIdx.x;
-  const int64_t L = len - j0;
   for (int j = 0; j < nb; ++j) {
     const int64_t c = j0 + j;
     double2* col = A + c * len;
+    double2* v = Vall + c * len;
+    __syncthreads();
     double2 acc = make_double2(0.0, 0.0);
-    for (int64_t r = c + 1 + tid; r < len; r += blockDim.x) acc.x += cabs2(col[r]);
-    const double xnorm2 = block_reduce_sum(acc, red).x;
-    const double2 alpha = col[c];
-    double2 t = make_double2(0.0, 0.0);
-    double beta = alpha.x;
-    double2 scal = make_double2(0.0, 0.0);
-    if (!(xnorm2 == 0.0 && alpha.y == 0.0)) {
-      const double nrm = sqrt(cabs2(alpha) + xnorm2);
-      beta = (alpha.x >= 0.0) ? -nrm : nrm;
-      t = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
-      // scal = 1 / (alpha - beta)
-      const double2 d = make_double2(alpha.x - beta, alpha.y);
-      const double dd = cabs2(d);
-      scal = make_double2(d.x / dd, -d.y / dd);
+    for (int64_t r = c + 1 + threadIdx.x; r < len; r += blockDim.x) acc.x += cabs2(col[r]);
+    const Reflector h = make_reflector(col[c], block_sum(acc, red).x);
+    __syncthreads();  // every thread has read col[c]
+    for (int64_t r = j0 + threadIdx.x; r < len; r += blockDim.x) {
+      v[r] = (r < c) ? make_double2(0.0, 0.0) : (r == c) ? h.d : col[r];
+      if (r == c) col[r] = make_double2(h.beta, 0.0);
     }
+    if (threadIdx.x == 0) tau[c] = h.tau;
+    if (!h.any) continue;
     __syncthreads();
-    if (!(t.x == 0.0 && t.y == 0.0)) {
-      for (int64_t r = c + 1 + tid; r < len; r += blockDim.x) col[r] = cmul(scal, col[r]);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      col[c] = make_double2(beta, 0.0);
-      tau[c] = t;
-      s_tau[j] = t;
-    }
-    __syncthreads();
-    // Apply H^H = I - conj(t) v v^H to the remaining panel columns.
-    if (!(t.x == 0.0 && t.y == 0.0)) {
-      for (int jj = j + 1; jj < nb; ++jj) {
-        double2* cc = A + (j0 + jj) * len;
-        const double2 ccc = cc[c];  // read before thread 0 rewrites it below
-        double2 a = make_double2(0.0, 0.0);
-        for (int64_t r = c + 1 + tid; r < len; r += blockDim.x) a = cfmac(col[r], cc[r], a);
-        double2 w = block_reduce_sum(a, red);
-        w = cadd(w, ccc);  // v[c] = 1
-        const double2 f = cmul(make_double2(t.x, -t.y), w);  // conj(t) * (v^H a)
-        if (tid == 0) cc[c] = make_double2(ccc.x - f.x, ccc.y - f.y);
-        for (int64_t r = c + 1 + tid; r < len; r += blockDim.x) {
-          const double2 p = cmul(f, col[r]);
-          cc[r] = make_double2(cc[r].x - p.x, cc[r].y - p.y);
-        }
-        __syncthreads();
-      }
-    }
+    for (int jj = j + 1; jj < nb; ++jj)
+      long_reflect(A + (j0 + jj) * len, v, c, len, make_double2(h.tau.x, -h.tau.y), red);
   }
-  // Explicit V (nb x L): unit diagonal, zeros above.
-  for (int64_t e = tid; e < (int64_t)nb * L; e += blockDim.x) {
-    const int j = (int)(e / L);
-    const int64_t rr = e % L;
-    double2 v;
-    if (rr < j)
-      v = make_double2(0.0, 0.0);
-    else if (rr == j)
-      v = make_double2(1.0, 0.0);
-    else
-      v = A[(j0 + j) * len + j0 + rr];
-    Vp[e] = v;
-  }
-  __syncthreads();
-  // T (zlarft, forward, columnwise): T[j][j] = tau_j,
-  // T[0:j, j] = -tau_j * T[0:j, 0:j] * (V[:, 0:j]^H v_j).
-  __shared__ double2 s_y[32];
-  __shared__ double2 s_T[32 * 32];
-  for (int e = tid; e < nb * nb; e += blockDim.x) s_T[e] = make_double2(0.0, 0.0);
-  __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    for (int i = 0; i < j; ++i) {
-      double2 a = make_double2(0.0, 0.0);
-      for (int64_t rr = j + tid; rr < L; rr += blockDim.x)
-        a = cfmac(Vp[(int64_t)i * L + rr], Vp[(int64_t)j * L + rr], a);
-      const double2 y = block_reduce_sum(a, red);
-      if (tid == 0) s_y[i] = y;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      const double2 tj = s_tau[j];
-      for (int i = 0; i < j; ++i) {
-        double2 acc2 = make_double2(0.0, 0.0);
-        for (int k = i; k < j; ++k) acc2 = cfma(s_T[i * nb + k], s_y[k], acc2);
-        const double2 v = cmul(tj, acc2);
-        s_T[i * nb + j] = make_double2(-v.x, -v.y);
-      }
-      s_T[j * nb + j] = tj;
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < nb * nb; e += blockDim.x) T[e] = s_T[e];
 }
 
-// Panel factorisation with the whole panel resident in LDS (nb <= 16 columns
-// of L <= QR_LDS_ROWS rows, one thread per row): one load, two barriers per
-// column (dot products and norm | reflector and updates, row by row), the T
-// factor from wavefront-parallel dot products, one write-back.  Same outputs
-// as qr_panel_kernel.
-constexpr int QR_LDS_THREADS = 1024;
-constexpr int QR_LDS_ROWS = 560;
-constexpr int QR_LDS_NB = 16;
+// Reflectors j0 .. j1 - 1 (adjoint, ascending) or j1 - 1 .. j0 on one column
+// of Y per workgroup, in memory.
+__global__ __launch_bounds__(256) void qr_reflect_long(double2* __restrict__ Y, int64_t len,
+                                                       int64_t j0, int64_t j1, int forward,
+                                                       const double2* __restrict__ tau,
+                                                       const double2* __restrict__ Vall) {
+  __shared__ double2 red[4];
+  double2* y = Y + (int64_t)blockIdx.x * len;
+  for (int64_t q = 0; q < j1 - j0; ++q) {
+    const int64_t j = forward ? j0 + q : j1 - 1 - q;
+    double2 t = tau[j];
+    if (forward) t.y = -t.y;
+    long_reflect(y, Vall + j * len, j, len, t, red);
+  }
+}
 
-__global__ __launch_bounds__(QR_LDS_THREADS) void qr_panel_lds_kernel(
-    double2* __restrict__ A, int64_t len, int64_t j0, int nb, double2* __restrict__ tau,
-    double2* __restrict__ Vp, double2* __restrict__ T) {
-  __shared__ double2 P[QR_LDS_NB * QR_LDS_ROWS];  // column j at P + j * L
-  __shared__ double2 s_T[QR_LDS_NB * QR_LDS_NB];
-  __shared__ double2 s_y[QR_LDS_NB * QR_LDS_NB];  // y[i][j] = V_i^H V_j, i < j
-  __shared__ double2 s_w[QR_LDS_NB];    // unscaled column-j dot products
-  __shared__ double2 s_ccj[QR_LDS_NB];  // trailing columns' row-j entries
-  __shared__ double2 s_tau[QR_LDS_NB];
-  __shared__ double2 s_alpha;
-  __shared__ double s_xn;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nwaves = QR_LDS_THREADS / 64;
-  const int L = (int)(len - j0);
-  for (int e = tid; e < nb * L; e += QR_LDS_THREADS) {
-    const int j = e / L, rr = e % L;
-    P[e] = A[(j0 + j) * len + j0 + rr];
+// Rows per lane of the smallest instantiation that holds L rows (0: none).
+inline int rows_per_lane(int64_t L) {
+  for (int r = 1; r <= REG_RPT; r <<= 1)
+    if (L <= 64 * r) return r;
+  return 0;
+}
+
+// Panel width of a register panel with r rows per lane: 64 columns up to 128
+// rows, 32 up to 256, 16 up to 512 (four, two, one columns on each of 16
+// wavefronts), 8 beyond (16 rows of two columns a lane do not fit the registers
+// of a full workgroup).
+inline int panel_width(int r) { return r <= 2 ? 64 : r <= 4 ? 32 : r <= 8 ? 16 : 8; }
+
+int panel(int r, double2* A, int64_t len, int64_t j0, int nb, double2* tau, double2* Vall,
+          hipStream_t stream) {
+  TimedLaunch timed("qr_panel", stream, 0.0);
+#define SEEMPS_PANEL(W, R, C)                                                             \
+  hipLaunchKernelGGL((qr_panel<W, R, C>), dim3(1), dim3(64 * W), 0, stream, A, len, j0, nb, tau, \
+                     Vall)
+  if (r == 1)
+    SEEMPS_PANEL(8, 1, 8);
+  else if (r == 2)
+    SEEMPS_PANEL(8, 2, 8);
+  else if (r == 4)
+    SEEMPS_PANEL(8, 4, 4);
+  else if (r == 8)
+    SEEMPS_PANEL(8, 8, 2);
+  else if (r == 16)
+    SEEMPS_PANEL(8, 16, 1);
+  else
+    hipLaunchKernelGGL(qr_panel_long, dim3(1), dim3(1024), 0, stream, A, len, j0, nb, tau, Vall);
+#undef SEEMPS_PANEL
+  return check_launch("qr_panel");
+}
+
+// Reflectors [j0, j1) on the ny columns of Y, rows r0 .. len - 1.
+template <bool FORWARD>
+int reflect(double2* Y, int64_t len, int64_t ny, int64_t r0, int64_t j0, int64_t j1,
+            const double2* tau, const double2* Vall, hipStream_t stream) {
+  if (ny <= 0 || j1 <= j0) return SEEMPS_OK;
+  TimedLaunch timed("qr_reflect", stream, 16.0 * (double)(len - r0) * ny * (j1 - j0));
+  // two columns per wavefront share each load of a reflector once one column
+  // each would put more than a wavefront on every SIMD
+  const bool two = ny > 1024;
+  const dim3 grid((unsigned)(two ? ceil_div(ny, 2) : ny)), wg(64);
+#define SEEMPS_REFLECT(R)                                                                       \
+  if (two)                                                                                      \
+    hipLaunchKernelGGL((qr_reflect<R, 2, FORWARD>), grid, wg, 0, stream, Y, len, ny, r0, j0, j1, \
+                       tau, Vall);                                                              \
+  else                                                                                          \
+    hipLaunchKernelGGL((qr_reflect<R, 1, FORWARD>), grid, wg, 0, stream, Y, len, ny, r0, j0, j1, \
+                       tau, Vall)
+  switch (rows_per_lane(len - r0)) {
+    case 1: SEEMPS_REFLECT(1); break;
+    case 2: SEEMPS_REFLECT(2); break;
+    case 4: SEEMPS_REFLECT(4); break;
+    case 8: SEEMPS_REFLECT(8); break;
+    case 16: SEEMPS_REFLECT(16); break;
+    default:
+      hipLaunchKernelGGL(qr_reflect_long, dim3((unsigned)ny), dim3(256), 0, stream, Y, len, j0, j1,
+                         (int)FORWARD, tau, Vall);
   }
-  __syncthreads();
-  // Two barriers per column.  Phase 1 only reads: wavefront q < nt forms the
-  // dot product of the unscaled column j with trailing column j + 1 + q (rows
-  // below j) and keeps that column's row-j entry; wavefront nt forms the norm
-  // of column j below the diagonal and keeps alpha = column j's row j.  Phase 2:
-  // thread rr owns row rr of the panel: it scales row rr of the reflector and
-  // applies every trailing column's update to row rr, so no two threads touch
-  // the same entry and nothing is read after being written.
-  for (int j = 0; j < nb; ++j) {
-    double2* col = P + j * L;
-    const int nt = nb - j - 1;  // trailing columns (<= 15 < nwaves)
-    if (wave < nt) {
-      const double2* cc = P + (j + 1 + wave) * L;
-      double2 a = make_double2(0.0, 0.0);
-      for (int rr = j + 1 + lane; rr < L; rr += 64) a = cfmac(col[rr], cc[rr], a);
-      for (int off = 32; off > 0; off >>= 1) {
-        a.x += __shfl_down(a.x, off, 64);
-        a.y += __shfl_down(a.y, off, 64);
-      }
-      if (lane == 0) {
-        s_w[wave] = a;
-        s_ccj[wave] = cc[j];
-      }
-    } else if (wave == nt) {
-      double acc = 0.0;
-      for (int rr = j + 1 + lane; rr < L; rr += 64) acc += cabs2(col[rr]);
-      for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-      if (lane == 0) {
-        s_xn = acc;
-        s_alpha = col[j];
-      }
-    }
-    __syncthreads();  // #1
-    const double2 alpha = s_alpha;
-    const double xnorm2 = s_xn;
-    double2 t = make_double2(0.0, 0.0);
-    double beta = alpha.x;
-    double2 scal = make_double2(0.0, 0.0);
-    const bool reflect = !(xnorm2 == 0.0 && alpha.y == 0.0);
-    if (reflect) {
-      const double nrm = sqrt(cabs2(alpha) + xnorm2);
-      beta = (alpha.x >= 0.0) ? -nrm : nrm;
-      t = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
-      const double2 d = make_double2(alpha.x - beta, alpha.y);
-      const double dd = cabs2(d);
-      scal = make_double2(d.x / dd, -d.y / dd);
-    }
-    const int rr = tid;
-    if (rr >= j && rr < L) {
-      if (reflect) {
-        // v = [1; scal col[j+1:]];  f_q = conj(t) v^H c_q = conj(t) (c_q[j] + conj(scal) w_q)
-        const double2 ct = make_double2(t.x, -t.y), cs = make_double2(scal.x, -scal.y);
-        const double2 v = (rr == j) ? make_double2(1.0, 0.0) : cmul(scal, col[rr]);
-        for (int q = 0; q < nt; ++q) {
-          const double2 f = cmul(ct, cadd(s_ccj[q], cmul(cs, s_w[q])));
-          double2* cc = P + (j + 1 + q) * L;
-          const double2 p = cmul(f, v);
-          cc[rr] = make_double2(cc[rr].x - p.x, cc[rr].y - p.y);
-        }
-        if (rr > j) col[rr] = v;
-      }
-      if (rr == j) {
-        col[j] = make_double2(beta, 0.0);
-        s_tau[j] = t;
-        tau[j0 + j] = t;
-      }
-    }
-    __syncthreads();  // #2
-  }
-  // y[i][j] = conj(V_i[j]) + sum_{rr > j} conj(V_i[rr]) V_j[rr], i < j
-  for (int q = wave; q < nb * nb; q += nwaves) {
-    const int i = q / nb, j = q % nb;
-    if (i >= j) continue;
-    const double2* ci = P + i * L;
-    const double2* cj = P + j * L;
-    double2 a = make_double2(0.0, 0.0);
-    for (int rr = j + 1 + lane; rr < L; rr += 64) a = cfmac(ci[rr], cj[rr], a);
-    for (int off = 32; off > 0; off >>= 1) {
-      a.x += __shfl_down(a.x, off, 64);
-      a.y += __shfl_down(a.y, off, 64);
-    }
-    if (lane == 0) s_y[i * QR_LDS_NB + j] = cadd(a, make_double2(ci[j].x, -ci[j].y));
-  }
-  for (int e = tid; e < QR_LDS_NB * QR_LDS_NB; e += QR_LDS_THREADS) s_T[e] = make_double2(0, 0);
-  __syncthreads();
-  // T (zlarft, forward, columnwise): T[j][j] = tau_j,
-  // T[0:j, j] = -tau_j * T[0:j, 0:j] * y[0:j, j].
-  for (int j = 0; j < nb; ++j) {
-    if (tid < j) {
-      const int i = tid;
-      double2 acc2 = make_double2(0.0, 0.0);
-      for (int k = i; k < j; ++k) acc2 = cfma(s_T[i * QR_LDS_NB + k], s_y[k * QR_LDS_NB + j], acc2);
-      const double2 v = cmul(s_tau[j], acc2);
-      s_T[i * QR_LDS_NB + j] = make_double2(-v.x, -v.y);
-    } else if (tid == j) {
-      s_T[j * QR_LDS_NB + j] = s_tau[j];
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < nb * nb; e += QR_LDS_THREADS)
-    T[e] = s_T[(e / nb) * QR_LDS_NB + e % nb];
-  for (int e = tid; e < nb * L; e += QR_LDS_THREADS) {
-    const int j = e / L, rr = e % L;
-    const double2 p = P[e];
-    A[(j0 + j) * len + j0 + rr] = p;
-    Vp[e] = (rr < j) ? make_double2(0.0, 0.0) : (rr == j) ? make_double2(1.0, 0.0) : p;
-  }
+#undef SEEMPS_REFLECT
+  return check_launch("qr_reflect");
 }
 
 }  // namespace
 
-// In-place blocked QR of A_cm (ncol columns of length len, len >= ncol).
-// Work: Vall (ncol * len complex), Tall (npanels * NB * NB), tau (ncol), Z (NB * ncol * 2),
-// ks (ks_elems complex, split-K partials of the NB-row products; may be 0).
-int qr_factor(double2* A, int64_t len, int64_t ncol, int nb_max, double2* Vall, double2* Tall,
-              double2* tau, double2* Z, double2* ks, int64_t ks_elems, hipStream_t stream) {
+// In-place QR of A_cm (ncol columns of length len, len >= ncol).
+// Work: Vall (ncol * len complex), tau (ncol).
+int qr_factor(double2* A, int64_t len, int64_t ncol, double2* Vall, double2* tau,
+              hipStream_t stream) {
   int st;
-  const double2 one = make_double2(1.0, 0.0), zero = make_double2(0.0, 0.0),
-                mone = make_double2(-1.0, 0.0);
-  for (int64_t j0 = 0, p = 0; j0 < ncol; j0 += nb_max, ++p) {
-    const int nb = (int)((ncol - j0) < nb_max ? (ncol - j0) : nb_max);
-    const int64_t L = len - j0;
-    double2* Vp = Vall + j0 * len;  // nb x L block (fits: nb * L <= nb * len)
-    double2* T = Tall + p * nb_max * nb_max;
-    if (L <= QR_LDS_ROWS && nb <= QR_LDS_NB) {
-      TimedLaunch timed("qr_panel_lds_kernel", stream, 0.0);
-      hipLaunchKernelGGL(qr_panel_lds_kernel, dim3(1), dim3(QR_LDS_THREADS), 0, stream, A, len,
-                         j0, nb, tau, Vp, T);
-      if ((st = check_launch("qr_panel_lds"))) return st;
-    } else {
-      TimedLaunch timed("qr_panel_kernel", stream, 0.0);
-      hipLaunchKernelGGL(qr_panel_kernel, dim3(1), dim3(QR_THREADS), 0, stream, A, len, j0, nb,
-                         tau, Vp, T);
-      if ((st = check_launch("qr_panel"))) return st;
-    }
-    const int64_t ntr = ncol - j0 - nb;
-    if (ntr <= 0) continue;
-    double2* At = A + (j0 + nb) * len + j0;  // ntr x L, row stride len
-    double2* Z1 = Z;                          // nb x ntr
-    double2* Z2 = Z + nb_max * ncol;          // nb x ntr
-    // Z1 = conj(Vp) At^T ; Z2 = T^H Z1 ; At -= Z2^T Vp
-    if ((st = zgemm_ws(SEEMPS_OP_C, SEEMPS_OP_T, nb, ntr, L, one, Vp, L, At, len, zero, Z1, ntr,
-                       ks, ks_elems, stream)))
+  for (int64_t j0 = 0; j0 < ncol;) {
+    const int r = rows_per_lane(len - j0);
+    const int64_t wide = r ? panel_width(r) : LONG_NB;
+    const int nb = (int)(ncol - j0 < wide ? ncol - j0 : wide);
+    if ((st = panel(r, A, len, j0, nb, tau, Vall, stream))) return st;
+    if ((st = reflect<true>(A + (j0 + nb) * len, len, ncol - j0 - nb, j0, j0, j0 + nb, tau, Vall,
+                            stream)))
       return st;
-    if ((st = zgemm(SEEMPS_OP_H, SEEMPS_OP_N, nb, ntr, nb, one, T, nb, 0, Z1, ntr, 0, zero, Z2, ntr,
-                    0, 1, stream)))
-      return st;
-    if ((st = zgemm(SEEMPS_OP_T, SEEMPS_OP_N, ntr, L, nb, mone, Z2, ntr, 0, Vp, L, 0, one, At, len,
-                    0, 1, stream)))
-      return st;
+    j0 += nb;
   }
   return SEEMPS_OK;
 }
 
-// Y <- Q Y for Y column-major (ny columns of length len), Q from qr_factor.
-int qr_apply_q(double2* Y, int64_t len, int64_t ny, int64_t ncol, int nb_max, const double2* Vall,
-               const double2* Tall, double2* Z, double2* ks, int64_t ks_elems,
-               hipStream_t stream) {
-  int st;
-  const double2 one = make_double2(1.0, 0.0), zero = make_double2(0.0, 0.0),
-                mone = make_double2(-1.0, 0.0);
-  const int64_t npan = ceil_div(ncol, nb_max);
-  for (int64_t p = npan - 1; p >= 0; --p) {
-    const int64_t j0 = p * nb_max;
-    const int nb = (int)((ncol - j0) < nb_max ? (ncol - j0) : nb_max);
-    const int64_t L = len - j0;
-    const double2* Vp = Vall + j0 * len;
-    const double2* T = Tall + p * nb_max * nb_max;
-    double2* Yt = Y + j0;  // ny x L, row stride len
-    double2* Z1 = Z;
-    double2* Z2 = Z + nb_max * (ny > ncol ? ny : ncol);
-    if ((st = zgemm_ws(SEEMPS_OP_C, SEEMPS_OP_T, nb, ny, L, one, Vp, L, Yt, len, zero, Z1, ny, ks,
-                       ks_elems, stream)))
-      return st;
-    if ((st = zgemm(SEEMPS_OP_N, SEEMPS_OP_N, nb, ny, nb, one, T, nb, 0, Z1, ny, 0, zero, Z2, ny, 0,
-                    1, stream)))
-      return st;
-    if ((st = zgemm(SEEMPS_OP_T, SEEMPS_OP_N, ny, L, nb, mone, Z2, ny, 0, Vp, L, 0, one, Yt, len, 0,
-                    1, stream)))
-      return st;
-  }
-  return SEEMPS_OK;
+// Y <- Q Y for Y column-major (ny columns of length len), Q from qr_factor with
+// ncol columns.
+int qr_apply_q(double2* Y, int64_t len, int64_t ny, int64_t ncol, const double2* Vall,
+               const double2* tau, hipStream_t stream) {
+  return reflect<false>(Y, len, ny, 0, 0, ncol, tau, Vall, stream);
 }
 
 }  // namespace seemps

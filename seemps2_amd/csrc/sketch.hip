@@ -139,11 +139,10 @@ unsigned grid_for(int64_t n) {
   return (unsigned)b;
 }
 
-constexpr int QRNB = 16;
 
 // Workspace layout of the sketch path (the fallback reuses the whole buffer).
 struct SketchWork {
-  double2 *Om, *Ycm, *Vall, *Tall, *tau, *Z, *ks, *Qcm, *Zcm, *B, *Ub, *VHb, *U, *red, *frob2,
+  double2 *Om, *Ycm, *Vall, *tau, *Qcm, *Zcm, *B, *Ub, *VHb, *U, *red, *frob2,
       *Rres, *resid2;
   double* S;
   int64_t* Ddev;
@@ -175,10 +174,7 @@ SketchWork sketch_carve(int64_t m, int64_t n, int64_t l, void* base) {
   w.Om = (double2*)take(l * n * 16);
   w.Ycm = (double2*)take(l * m * 16);
   w.Vall = (double2*)take(l * mx * 16);
-  w.Tall = (double2*)take(ceil_div(l, QRNB) * QRNB * QRNB * 16);
   w.tau = (double2*)take(l * 16);
-  w.Z = (double2*)take(2 * QRNB * (mx > l ? mx : l) * 16);
-  w.ks = (double2*)take(8 * QRNB * l * 16);
   w.Qcm = (double2*)take(l * m * 16);
   w.Zcm = (double2*)take(l * n * 16);
   w.B = (double2*)take(l * n * 16);
@@ -208,16 +204,15 @@ SketchWork sketch_carve(int64_t m, int64_t n, int64_t l, void* base) {
 
 // Orthonormal basis of the l columns (length len) of Xcm, written to Qout
 // (column-major, l columns of length len).  Xcm is overwritten.  WS supplies the
-// QR scratch (Vall, Tall, tau, Z, ks) sized for l columns of length len.
+// QR scratch (Vall, tau) sized for l columns of length len.
 template <class WS>
 int orthonormalize(double2* Xcm, int64_t len, int64_t l, double2* Qout, const WS& w,
                    hipStream_t stream) {
   int st;
-  if ((st = qr_factor(Xcm, len, l, QRNB, w.Vall, w.Tall, w.tau, w.Z, w.ks, 8 * QRNB * l, stream)))
-    return st;
+  if ((st = qr_factor(Xcm, len, l, w.Vall, w.tau, stream))) return st;
   hipLaunchKernelGGL(identity_cm, dim3(grid_for(len * l)), dim3(256), 0, stream, len, l, Qout);
   if ((st = check_launch("identity_cm"))) return st;
-  return qr_apply_q(Qout, len, l, l, QRNB, w.Vall, w.Tall, w.Z, w.ks, 8 * QRNB * l, stream);
+  return qr_apply_q(Qout, len, l, l, w.Vall, w.tau, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -323,7 +318,7 @@ __global__ __launch_bounds__(256) void expansion_rotation(int p, const double2* 
 // Workspace of the basis-sketched split: Lg x Sh working orientation (Lg = m,
 // Sh = n for side 0; Lg = n, Sh = m for side 1), l = k + p sketch columns.
 struct BasisWork {
-  double2 *G0t, *Yt, *Zt, *C, *Qz, *Vall, *Tall, *tau, *Z, *ks, *Oh, *W, *Uw, *VHw, *T, *red,
+  double2 *G0t, *Yt, *Zt, *C, *Qz, *Vall, *tau, *Oh, *W, *Uw, *VHw, *T, *red,
       *frob2, *Rres, *resid2, *G2, *Q2;
   double* S;
   int64_t* Ddev;
@@ -351,10 +346,7 @@ BasisWork basis_carve(int64_t Lg, int64_t Sh, int64_t k, int64_t p, void* base) 
   w.C = (double2*)take(pp * k * 16);
   w.Qz = (double2*)take(pp * Sh * 16);
   w.Vall = (double2*)take(pp * Sh * 16);
-  w.Tall = (double2*)take(ceil_div(pp, QRNB) * QRNB * QRNB * 16);
   w.tau = (double2*)take(pp * 16);
-  w.Z = (double2*)take(2 * QRNB * (Sh > pp ? Sh : pp) * 16);
-  w.ks = (double2*)take(8 * QRNB * pp * 16);
   w.Oh = (double2*)take(l * Sh * 16);
   w.W = (double2*)take(Lg * l * 16);
   w.Uw = (double2*)take(Lg * l * 16);

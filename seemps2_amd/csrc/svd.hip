@@ -51,7 +51,6 @@ constexpr int RMAX = 16;        // max row chunks per pair
 // Relative off-diagonal measure from which one more sweep is known to suffice
 // (quadratic convergence: the sweep leaves ~1e-18 against a target ~1e-13).
 constexpr double QUAD_STOP = 1e-9;
-constexpr int QRNB = 16;        // QR panel width
 constexpr int QR_MIN_COLS = 17; // use the QR preconditioner from this many columns
 constexpr int MAX_SWEEPS = 60;
 constexpr unsigned long long SPIN_LIMIT = 4000000ull;
@@ -81,11 +80,8 @@ struct SvdShape {
 struct SvdWork {
   double2* Acm;   // ncol x lenA (QR in place)
   double2* Vall;  // ncol x lenA (QR vectors)
-  double2* Tall;  // npanels x QRNB x QRNB
   double2* tau;   // ncol
-  double2* Z;     // 2 x QRNB x max(ncol, ncolp)
   double2* Y;     // ncol x lenA (Q V)
-  double2* ks;    // split-K partials of the QR panel products
   double2* W;     // ncolp x len
   double2* V;     // ncolp x ncolp
   double2* part;  // 2 x P x RMAX x PW x PW (partial Grams, by step parity)
@@ -156,18 +152,11 @@ SvdShape svd_shape(int64_t m, int64_t n, int num_cu, bool precondition = true) {
   return s;
 }
 
-// Split-K scratch of the NB-row products of the QR (factor and apply).
-// (Up to 8 slices of NB x ncol, enough for every panel's shape.)
-inline int64_t qr_ks_elems(const SvdShape& s) { return 8 * QRNB * s.ncol; }
-
 #define SEEMPS_SVD_REGIONS(X)                                         \
   X(Acm, s.use_qr ? s.ncol * s.lenA : 0, double2)                     \
   X(Vall, s.use_qr ? s.ncol * s.lenA : 0, double2)                    \
-  X(Tall, s.use_qr ? ceil_div(s.ncol, QRNB) * QRNB * QRNB : 0, double2) \
   X(tau, s.use_qr ? s.ncol : 0, double2)                              \
-  X(Z, s.use_qr ? 2 * QRNB * (s.ncolp > s.lenA ? s.ncolp : s.lenA) : 0, double2) \
   X(Y, s.use_qr ? s.ncol * s.lenA : 0, double2)                       \
-  X(ks, s.use_qr ? qr_ks_elems(s) : 0, double2)                       \
   X(W, s.ncolp * s.len, double2)                                      \
   X(V, s.ncolp * s.ncolp, double2)                                    \
   X(part, 2 * s.P * RMAX * PW * PW, double2)                          \
@@ -1102,9 +1091,7 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
     hipLaunchKernelGGL(load_colmajor, dim3(blocks_for(s.ncol * s.lenA)), dim3(256), 0, stream, s,
                        A, lda, w.Acm, s.ncol, (const int*)w.colperm);
     if ((st = check_launch("load_colmajor"))) return st;
-    if ((st = qr_factor(w.Acm, s.lenA, s.ncol, QRNB, w.Vall, w.Tall, w.tau, w.Z, w.ks,
-                        qr_ks_elems(s), stream)))
-      return st;
+    if ((st = qr_factor(w.Acm, s.lenA, s.ncol, w.Vall, w.tau, stream))) return st;
     hipLaunchKernelGGL(load_w_from_r, dim3(blocks_for(s.ncolp * s.len)), dim3(256), 0, stream, s,
                        w.Acm, w.W);
     if ((st = check_launch("load_w_from_r"))) return st;
@@ -1147,9 +1134,7 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
   if (s.use_qr) {
     hipLaunchKernelGGL(load_y, dim3(blocks_for(s.ncol * s.lenA)), dim3(256), 0, stream, s, w);
     if ((st = check_launch("load_y"))) return st;
-    if ((st = qr_apply_q(w.Y, s.lenA, s.ncol, s.ncol, QRNB, w.Vall, w.Tall, w.Z, w.ks,
-                         qr_ks_elems(s), stream)))
-      return st;
+    if ((st = qr_apply_q(w.Y, s.lenA, s.ncol, s.ncol, w.Vall, w.tau, stream))) return st;
   }
   const int64_t big = s.ncol * (s.len > s.lenA ? s.len : s.lenA);
   hipLaunchKernelGGL(svd_output, dim3(blocks_for(big)), dim3(256), 0, stream, s, w, U, S, VH);
