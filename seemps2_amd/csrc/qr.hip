@@ -287,12 +287,17 @@ __device__ double2 block_sum(double2 v, double2* red) {
 }
 
 // y <- y - f (v^H y) v over rows [lo, len) by one workgroup, v and y in memory.
+// A thread keeps the same rows (its index modulo the workgroup's size) whatever
+// lo is: what it reads of y it has written itself, with no barrier between
+// calls.
 __device__ void long_reflect(double2* __restrict__ y, const double2* __restrict__ v, int64_t lo,
                              int64_t len, double2 f, double2* red) {
+  const int64_t step = blockDim.x, tid = threadIdx.x;
+  const int64_t first = tid + (lo > tid ? ceil_div(lo - tid, step) * step : 0);
   double2 d = make_double2(0.0, 0.0);
-  for (int64_t r = lo + threadIdx.x; r < len; r += blockDim.x) d = cfmac(v[r], y[r], d);
+  for (int64_t r = first; r < len; r += step) d = cfmac(v[r], y[r], d);
   d = cmul(f, block_sum(d, red));
-  for (int64_t r = lo + threadIdx.x; r < len; r += blockDim.x) {
+  for (int64_t r = first; r < len; r += step) {
     const double2 p = cmul(d, v[r]);
     y[r] = make_double2(y[r].x - p.x, y[r].y - p.y);
   }
