@@ -11,8 +11,9 @@
 //   3. One-sided block Jacobi on the working matrix W (columns of X or B):
 //      column blocks of width BW, every pair of blocks visited once per sweep
 //      in a round-robin (circle) schedule; per pair the 2BW x 2BW Gram matrix is
-//      formed (partial sums over row chunks in different workgroups), an inner
-//      Hermitian Jacobi sweep accumulates Q, and W_pq <- W_pq Q, V_pq <- V_pq Q.
+//      formed (partial sums over row chunks in different workgroups), and the
+//      rotations of an inner Hermitian Jacobi sweep on it are applied to the
+//      pair's columns of W and V as they come.
 //      Stops when every normalised off-diagonal |G_ij| / sqrt(G_ii G_jj) seen in
 //      a sweep is below 32 sqrt(len) eps (relative orthogonality), when it was
 //      already below 1e-9 (quadratic convergence: that sweep's rotations leave
@@ -33,20 +34,18 @@
 #include <cmath>
 #include <cstdlib>
 
-#include "common.h"
 #include "jacobi_inner.h"
+#include "wave.h"
 
 namespace seemps {
 
 namespace {
 
 using jac::GP;
-using jac::inner_jacobi;
 using jac::PW;
 
 constexpr int BW = PW / 2;      // block width (columns); PW, GP from jacobi_inner.h
-constexpr int RT = 32;          // rows per LDS tile (the 2 x 2 blocked loops assume 32)
-constexpr int RTP = RT + 1;     // padded tile row length (complex)
+constexpr int RT = 64;          // rows per LDS tile: a row a lane
 constexpr int RMAX = 16;        // max row chunks per pair
 // Relative off-diagonal measure from which one more sweep is known to suffice
 // (quadratic convergence: the sweep leaves ~1e-18 against a target ~1e-13).
@@ -110,17 +109,10 @@ SvdShape svd_shape(int64_t m, int64_t n, int num_cu, bool precondition = true) {
   s.nb = nb;
   s.ncolp = nb * BW;
   s.P = nb / 2;
-  // Row chunks per pair: one workgroup per CU (cooperative residency caps the
-  // grid there).  The QR-preconditioned matrix takes about half that while
-  // at least 8 chunks remain: fewer, longer chunks shorten each step's
-  // reduction and waits, and on 512 columns (16 pairs) R = 8 beat R = 16 over
-  // whole DMRG sweeps; on the basis-sketched matrices R = 16 stayed ahead.
+  // Row chunks per pair: a tile each, as far as one workgroup per CU allows.
+  // The chunk's rotations then hide behind the inner rounds; a longer chunk
+  // replays them tile by tile.
   int64_t R = num_cu / s.P;
-  if (s.use_qr) {
-    int64_t half = num_cu / (2 * s.P);
-    if (half < 8) half = 8;
-    if (half < R) R = half;
-  }
   // tuning knob: cap on the row chunks per pair (SEEMPS_SVD_ROW_CHUNKS)
   static const int64_t r_cap = [] {
     const char* e = getenv("SEEMPS_SVD_ROW_CHUNKS");
@@ -151,6 +143,9 @@ SvdShape svd_shape(int64_t m, int64_t n, int num_cu, bool precondition = true) {
   s.cross_inner = s.nb > 2 ? inner_mode : 0;
   return s;
 }
+
+// Inner sweeps per step: a single pair (two blocks) has nothing to wait for.
+__host__ __device__ inline int inner_sweeps_of(const SvdShape& s) { return s.nb == 2 ? 3 : 1; }
 
 #define SEEMPS_SVD_REGIONS(X)                                         \
   X(Acm, s.use_qr ? s.ncol * s.lenA : 0, double2)                     \
@@ -354,70 +349,6 @@ __device__ __forceinline__ int64_t pair_col(int64_t bi, int64_t bj, int t) {
   return (t < BW) ? bi * BW + t : bj * BW + (t - BW);
 }
 
-// Rotate rows [w0, w1) of the pair's PW columns of W (column stride ldw) and
-// rows [v0, v1) of those of V (stride ldv) by Q: M_pq <- M_pq Q.  Both RT-row
-// tiles are staged in LDS together (tw, tv), so one load latency covers both.
-__device__ void rotate_rows(double2* __restrict__ W, int64_t ldw, int64_t w0, int64_t w1,
-                            double2* __restrict__ V, int64_t ldv, int64_t v0, int64_t v1,
-                            int64_t bi, int64_t bj, const double2* Q, double2* tw,
-                            double2* tv) {
-  const int tid = threadIdx.x;
-  const int64_t nw = ceil_div(w1 - w0, (int64_t)RT), nv = ceil_div(v1 - v0, (int64_t)RT);
-  const int64_t nblk = nw > nv ? nw : nv;
-  for (int64_t blk = 0; blk < nblk; ++blk) {
-    const int64_t rbw = w0 + blk * RT, rbv = v0 + blk * RT;
-    const int nrw = (blk < nw) ? (int)min((int64_t)RT, w1 - rbw) : 0;
-    const int nrv = (blk < nv) ? (int)min((int64_t)RT, v1 - rbv) : 0;
-    for (int e = tid; e < PW * RT; e += blockDim.x) {
-      const int t = e / RT, rr = e % RT;
-      tw[t * RTP + rr] = (rr < nrw) ? W[pair_col(bi, bj, t) * ldw + rbw + rr] : make_double2(0, 0);
-      tv[t * RTP + rr] = (rr < nrv) ? V[pair_col(bi, bj, t) * ldv + rbv + rr] : make_double2(0, 0);
-    }
-    __syncthreads();
-    {
-      // thread (jb, r0): columns jb, jb + 16 by rows r0, r0 + 16 of both tiles
-      const int jb = tid >> 4, r0 = tid & 15;
-      double2 w00 = make_double2(0.0, 0.0), w01 = w00, w10 = w00, w11 = w00;
-      double2 v00 = w00, v01 = w00, v10 = w00, v11 = w00;
-#pragma unroll 4
-      for (int k = 0; k < PW; ++k) {
-        const double2 q0 = Q[k * GP + jb], q1 = Q[k * GP + jb + 16];
-        const double2 x0 = tw[k * RTP + r0], x1 = tw[k * RTP + r0 + 16];
-        const double2 y0 = tv[k * RTP + r0], y1 = tv[k * RTP + r0 + 16];
-        w00 = cfma(x0, q0, w00);
-        w01 = cfma(x1, q0, w01);
-        w10 = cfma(x0, q1, w10);
-        w11 = cfma(x1, q1, w11);
-        v00 = cfma(y0, q0, v00);
-        v01 = cfma(y1, q0, v01);
-        v10 = cfma(y0, q1, v10);
-        v11 = cfma(y1, q1, v11);
-      }
-      double2* W0 = W + pair_col(bi, bj, jb) * ldw + rbw;
-      double2* W1 = W + pair_col(bi, bj, jb + 16) * ldw + rbw;
-      double2* V0 = V + pair_col(bi, bj, jb) * ldv + rbv;
-      double2* V1 = V + pair_col(bi, bj, jb + 16) * ldv + rbv;
-      if (r0 < nrw) {
-        W0[r0] = w00;
-        W1[r0] = w10;
-      }
-      if (r0 + 16 < nrw) {
-        W0[r0 + 16] = w01;
-        W1[r0 + 16] = w11;
-      }
-      if (r0 < nrv) {
-        V0[r0] = v00;
-        V1[r0] = v10;
-      }
-      if (r0 + 16 < nrv) {
-        V0[r0 + 16] = v01;
-        V1[r0 + 16] = v11;
-      }
-    }
-    __syncthreads();
-  }
-}
-
 __device__ __forceinline__ long long now_ticks() { return (long long)wall_clock64(); }
 
 // Pair owning block x in round k of the circle schedule (inverse of pair_blocks).
@@ -428,114 +359,415 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
   return (y < nb / 2) ? y : nb - 1 - y;
 }
 
-// Phase A: partial Gram matrix of rows [r0, r1) of the pair's columns into dst
-// (PW x PW, row-major).  Thread (ib, jb) accumulates the 2 x 2 block of
-// entries (ib + 16x, jb + 16y): four LDS reads per row feed four complex FMAs.
-__device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
-                             int64_t r0, int64_t r1, double2* __restrict__ dst, double2* tile) {
-  static_assert(PW == 32, "the 2 x 2 register blocking assumes 256 threads and PW = 32");
-  const int tid = threadIdx.x;
-  const int ib = tid >> 4, jb = tid & 15;
-  double2 a00 = make_double2(0, 0), a01 = a00, a10 = a00, a11 = a00;
-  for (int64_t rb = r0; rb < r1; rb += RT) {
-    const int nr = (int)min((int64_t)RT, r1 - rb);
-    for (int e = tid; e < PW * RT; e += blockDim.x) {
-      const int t = e / RT, rr = e % RT;
-      tile[t * RTP + rr] =
-          (rr < nr) ? w.W[pair_col(bi, bj, t) * s.len + rb + rr] : make_double2(0, 0);
-    }
-    __syncthreads();
-    const double2* x0 = tile + ib * RTP;
-    const double2* x1 = tile + (ib + 16) * RTP;
-    const double2* y0 = tile + jb * RTP;
-    const double2* y1 = tile + (jb + 16) * RTP;
-    for (int rr = 0; rr < nr; ++rr) {
-      const double2 u0 = x0[rr], u1 = x1[rr], v0 = y0[rr], v1 = y1[rr];
-      a00 = cfmac(u0, v0, a00);
-      a01 = cfmac(u0, v1, a01);
-      a10 = cfmac(u1, v0, a10);
-      a11 = cfmac(u1, v1, a11);
-    }
-    __syncthreads();
+// ---- one block pair on one workgroup --------------------------------------
+//
+// 512 threads.  A tile of RT rows of the pair's PW columns sits in LDS
+// (column-major, padded); its Gram matrix is taken from it on the matrix cores,
+// then the inner Jacobi rotates G and the tile in registers.
+//
+// A level H of the inner Jacobi pairs index base + t with base + H + (t + k) mod H
+// in round k (base = 0, 2H, ..): H rounds of 16 disjoint rotations that visit
+// every pair across the two halves of each group of 2H indices once.  Level 16
+// visits the pairs across the two blocks; levels 16, 8, 4, 2, 1 together every
+// pair of the 32.  The first index of a pair stays where it is and the second
+// moves one place a round, so wavefronts 0-3 keep G in registers, a 2 x 2 block
+// a thread, and pass entries to the neighbouring thread: along a row of threads
+// by DPP, between rows through LDS.  Wavefronts 4-7 hold the tile, a row a lane,
+// four pairs of columns a wavefront, and pass one column a round.  One barrier
+// a round: the thread that holds pair p's own block derives its rotation from
+// what it has (the second index's diagonal entry comes with that pair's
+// rotation), everyone applies it after the barrier.
+//
+// A round takes 0.51 us, two thirds of it instruction issue (48 FP64
+// operations a thread in either role, the rotation's chain of 45); with G and
+// the tile in LDS it took 1.07 us, LDS traffic (100 KB a round).
+constexpr int JT = 512;            // threads
+constexpr int TP = RT + 1;         // padded tile column (complex)
+constexpr int NP = PW / 2;         // pairs a round
+constexpr int ROUNDS = PW - 1;     // rounds of all levels
+
+// Rotation of a pair, [x_a, x_b] <- [cs x_a - conj(s) x_b, s x_a + cs x_b], and
+// the diagonal entry that it gives index b.
+struct Rot {
+  double cs, gbb;
+  double2 s;
+};
+
+// Indices of pair p in round k of level H.
+__device__ __forceinline__ void slot_cols(int H, int p, int k, int* a, int* b) {
+  const int t = p & (H - 1), base = (p - t) * 2;
+  *a = base + t;
+  *b = base + H + ((t + k) & (H - 1));
+}
+// The pair whose second index pair p takes over in the next round.
+__device__ __forceinline__ int slot_next(int H, int p) {
+  return (p & ~(H - 1)) | ((p + 1) & (H - 1));
+}
+// x of the thread of pair slot_next(q) (q: the thread's place in its row of 16).
+template <int H>
+__device__ __forceinline__ double lane_next(double x) {
+  if (H == 16) return wave::dpp<0x12F>(x);  // row_ror:15
+  if (H == 8) {
+    const double u = wave::dpp<0x12F>(x), v = wave::dpp<0x127>(x);  // row_ror:15, :7
+    return (threadIdx.x & 7) == 7 ? v : u;
   }
-  dst[ib * PW + jb] = a00;
-  dst[ib * PW + jb + 16] = a01;
-  dst[(ib + 16) * PW + jb] = a10;
-  dst[(ib + 16) * PW + jb + 16] = a11;
+  if (H == 4) return wave::dpp<0x39>(x);  // quad_perm 1, 2, 3, 0
+  if (H == 2) return wave::dpp<0xB1>(x);  // quad_perm 1, 0, 3, 2
+  return x;
 }
 
-// Phases B + C for item (p, r): G = sum of the R partials at src, the pair's
-// off-diagonal measure (r == 0) into *off_slot, inner Jacobi, rotation of this
-// chunk's rows of W and V.  prof/pt/t0: phase timing of workgroup 0.
+struct PairLds {
+  double2 tile[PW * TP];
+  double2 G[PW * GP], G2[PW * GP];
+  double2 sh[2][2][NP * NP];  // second rows of the 2 x 2 blocks, by round parity
+  double2 xch[2][4][RT];      // the tile columns on their way
+  double off[JT / 64];
+  int flag;
+};
+
+// Rotation that annihilates c = G_ab; identity when the pair is orthogonal to
+// tol or either column negligible.  t = tan(angle), the smaller root of
+// t^2 + 2 tau t - 1 = 0, comes from the hardware's reciprocal and square root
+// estimates (relative error about 1e-7): an angle that far off leaves 1e-7 of
+// G_ab, which the next sweep removes.  cs and |s| are refined to a few ulp, so
+// the rotation is unitary whatever t is.
+__device__ __forceinline__ Rot pair_rotation(double gaa, double gbb, double2 c, double tol2,
+                                             double tiny2) {
+  Rot q;
+  q.cs = 1.0;
+  q.gbb = gbb;
+  q.s = make_double2(0.0, 0.0);
+  const double s2 = cabs2(c);
+  const bool any = s2 > 0.0 && gaa > tiny2 && gbb > tiny2 && s2 > (tol2 * gaa) * gbb;
+  const double tau = (gbb - gaa) * (0.5 * __builtin_amdgcn_rsq(s2));
+  const double at = fmin(fabs(tau), 1e150);
+  const double u = fma(at, at, 1.0);
+  const double t = copysign(__builtin_amdgcn_rcp(fma(u, __builtin_amdgcn_rsq(u), at)), tau);
+  const double cs = jac::rsqrt_nr(fma(t, t, 1.0)), r = jac::rsqrt_nr(s2);
+  const double sn = t * cs * r;
+  if (any) {
+    q.cs = cs;
+    q.gbb = fma(t, s2 * r, gbb);
+    q.s = make_double2(c.x * sn, c.y * sn);
+  }
+  return q;
+}
+
+__device__ __forceinline__ double2 rscale(double f, double2 x) {
+  return make_double2(f * x.x, f * x.y);
+}
+
+// Level H on L.G and L.tile, on every wavefront of the workgroup; rec receives
+// its H x NP rotations.  Ends with a barrier.
+template <int H>
+__device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, double tiny2) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (wv < 4) {
+    const int p = tid >> 4, q = tid & 15, pn = slot_next(H, p);
+    int a, b, c, d;
+    slot_cols(H, p, 0, &a, &b);
+    slot_cols(H, q, 0, &c, &d);
+    double2 ac = L.G[a * GP + c], ad = L.G[a * GP + d];
+    double2 bc = L.G[b * GP + c], bd = L.G[b * GP + d];
+    double gbb = bd.x;
+#pragma unroll 2
+    for (int k = 0; k < H; ++k) {
+      Rot* rot = rec + k * NP;
+      const Rot own = pair_rotation(ac.x, gbb, ad, tol2, tiny2);
+      if (p == q) rot[p] = own;
+      __syncthreads();
+      const Rot rp = rot[p], rq = rot[q];
+      gbb = rot[pn].gbb;
+      if (k > 0) {
+        bc = L.sh[k & 1][0][pn * NP + q];
+        bd = L.sh[k & 1][1][pn * NP + q];
+      }
+      // Z = J_p^H X J_q on the block (rows of pair p, columns of pair q)
+      const double2 mq = make_double2(-rq.s.x, rq.s.y), mp = make_double2(-rp.s.x, -rp.s.y);
+      const double2 cp = make_double2(rp.s.x, -rp.s.y);
+      const double2 yac = cfma(mq, ad, rscale(rq.cs, ac)), yad = cfma(rq.s, ac, rscale(rq.cs, ad));
+      const double2 ybc = cfma(mq, bd, rscale(rq.cs, bc)), ybd = cfma(rq.s, bc, rscale(rq.cs, bd));
+      ac = cfma(mp, ybc, rscale(rp.cs, yac));
+      ad = cfma(mp, ybd, rscale(rp.cs, yad));
+      bc = cfma(cp, yac, rscale(rp.cs, ybc));
+      bd = cfma(cp, yad, rscale(rp.cs, ybd));
+      if (k + 1 < H) {
+        ad = make_double2(lane_next<H>(ad.x), lane_next<H>(ad.y));
+        bd = make_double2(lane_next<H>(bd.x), lane_next<H>(bd.y));
+        L.sh[(k + 1) & 1][0][tid] = bc;
+        L.sh[(k + 1) & 1][1][tid] = bd;
+      }
+    }
+    slot_cols(H, p, H - 1, &a, &b);
+    slot_cols(H, q, H - 1, &c, &d);
+    L.G[a * GP + c] = ac;
+    L.G[a * GP + d] = ad;
+    L.G[b * GP + c] = bc;
+    L.G[b * GP + d] = bd;
+  } else {
+    const int w = wv - 4;
+    const int wn = H == 16 ? (w + 1) & 3 : H == 8 ? w ^ 1 : w;  // owner of the column to come
+    double2 xa[4], xb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int a, b;
+      slot_cols(H, 4 * w + i, 0, &a, &b);
+      xa[i] = L.tile[a * TP + lane];
+      xb[i] = L.tile[b * TP + lane];
+    }
+#pragma unroll 2
+    for (int k = 0; k < H; ++k) {
+      __syncthreads();
+      // the four rotations (16 doubles) in the lanes, broadcast from there
+      const double rd = ((const double*)(rec + k * NP + 4 * w))[lane & 15];
+      if (H >= 8 && k > 0) xb[3] = L.xch[k & 1][wn][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double cs = wave::bcast(rd, 4 * i);
+        const double2 sp = make_double2(wave::bcast(rd, 4 * i + 2), wave::bcast(rd, 4 * i + 3));
+        const double2 x = xa[i], y = xb[i];
+        xa[i] = cfma(make_double2(-sp.x, sp.y), y, rscale(cs, x));
+        xb[i] = cfma(sp, x, rscale(cs, y));
+      }
+      if (k + 1 < H) {
+        const double2 x = xb[0];
+        if (H == 2) {
+          xb[0] = xb[1];
+          xb[1] = x;
+          const double2 y = xb[2];
+          xb[2] = xb[3];
+          xb[3] = y;
+        } else {
+          if (H >= 8) L.xch[(k + 1) & 1][w][lane] = x;
+          xb[0] = xb[1];
+          xb[1] = xb[2];
+          xb[2] = xb[3];
+          if (H == 4) xb[3] = x;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int a, b;
+      slot_cols(H, 4 * w + i, H - 1, &a, &b);
+      L.tile[a * TP + lane] = xa[i];
+      L.tile[b * TP + lane] = xb[i];
+    }
+  }
+  __syncthreads();
+}
+
+// Inner sweeps: level 16 (cross) or all levels.  Returns the number of rounds.
+__device__ int inner_rounds(PairLds& L, Rot* rec, double tol, double tiny2, int sweeps,
+                            bool cross) {
+  const double tol2 = tol * tol;
+  int n = 0;
+  for (int sw = 0; sw < sweeps; ++sw) {
+    inner_level<16>(L, rec + n * NP, tol2, tiny2);
+    n += 16;
+    if (cross) continue;
+    inner_level<8>(L, rec + n * NP, tol2, tiny2);
+    inner_level<4>(L, rec + (n + 8) * NP, tol2, tiny2);
+    inner_level<2>(L, rec + (n + 12) * NP, tol2, tiny2);
+    inner_level<1>(L, rec + (n + 14) * NP, tol2, tiny2);
+    n += 15;
+  }
+  return n;
+}
+
+// Rows [rb, rb + nr) of the pair's columns of M into the tile (zeros below).
+__device__ __forceinline__ void load_tile(const double2* __restrict__ M, int64_t ld, int64_t bi,
+                                          int64_t bj, int64_t rb, int nr, double2* tile) {
+  for (int e = threadIdx.x; e < PW * RT; e += JT) {
+    const int t = e / RT, rr = e % RT;
+    tile[t * TP + rr] = rr < nr ? M[pair_col(bi, bj, t) * ld + rb + rr] : make_double2(0.0, 0.0);
+  }
+}
+__device__ __forceinline__ void store_tile(double2* __restrict__ M, int64_t ld, int64_t bi,
+                                           int64_t bj, int64_t rb, int nr, const double2* tile) {
+  for (int e = threadIdx.x; e < PW * RT; e += JT) {
+    const int t = e / RT, rr = e % RT;
+    if (rr < nr) M[pair_col(bi, bj, t) * ld + rb + rr] = tile[t * TP + rr];
+  }
+}
+
+// One of the 12 shares of the Gram matrix's upper 16 x 16 tiles: tile
+// (00, 11 or 01), real or imaginary part, first or second half of the rows.
+struct GramShare {
+  int ti, tj, im, half;
+};
+__device__ __forceinline__ GramShare gram_share(int q) {
+  const int tl = q % 3;
+  return GramShare{tl == 1 ? 1 : 0, tl == 0 ? 0 : 1, (q / 3) & 1, q / 6};
+}
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// acc += this share of the tile's Gram matrix (nr valid rows).
+__device__ __forceinline__ void gram_accumulate(const double2* tile, int nr, GramShare q, d4* acc) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int steps = (nr + 3) >> 2, mid = (steps + 1) >> 1;
+  const double2* ca = tile + (q.ti * 16 + li) * TP + lk;
+  const double2* cb = tile + (q.tj * 16 + li) * TP + lk;
+  for (int k = q.half ? mid : 0; k < (q.half ? steps : mid); ++k) {
+    const double2 x = ca[4 * k], y = cb[4 * k];
+    // conj(x) y: re = xr yr + xi yi, im = xr yi - xi yr
+    *acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, q.im ? y.y : y.x, *acc, 0, 0, 0);
+    *acc = __builtin_amdgcn_mfma_f64_16x16x4f64(q.im ? -x.y : x.y, q.im ? y.x : y.y, *acc, 0, 0, 0);
+  }
+}
+
+// The share into its half's buffer (upper tiles of the PW x PW matrix).
+__device__ __forceinline__ void gram_store(double2* dst, GramShare q, d4 acc) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  double* d = (double*)dst + q.im;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    d[2 * ((q.ti * 16 + lk + 4 * r) * GP + q.tj * 16 + li)] = acc[r];
+}
+
+// Phase A for item (p, r): the Gram matrix of rows [r0, r1) of the pair's
+// columns; the last tile of the rows stays in LDS.  R > 1: into dst
+// (PW x PW, i <= j only), to be summed over the chunks; else the two halves are
+// left in L.G and L.G2.
+__device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
+                             int64_t r0, int64_t r1, double2* __restrict__ dst, PairLds& L) {
+  const int wave = threadIdx.x >> 6;
+  const GramShare q0 = gram_share(wave), q1 = gram_share(wave + 8 < 12 ? wave + 8 : 0);
+  d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0;
+  for (int64_t rb = r0; rb == r0 || rb < r1; rb += RT) {
+    const int nr = (int)max((int64_t)0, min((int64_t)RT, r1 - rb));
+    __syncthreads();
+    load_tile(w.W, s.len, bi, bj, rb, nr, L.tile);
+    __syncthreads();
+    gram_accumulate(L.tile, nr, q0, &c0);
+    if (wave + 8 < 12) gram_accumulate(L.tile, nr, q1, &c1);
+  }
+  gram_store(q0.half ? L.G2 : L.G, q0, c0);
+  if (wave + 8 < 12) gram_store(q1.half ? L.G2 : L.G, q1, c1);
+  __syncthreads();
+  if (s.R == 1) return;
+  for (int e = threadIdx.x; e < PW * PW; e += JT) {
+    const int i = e / PW, j = e % PW;
+    if (i <= j) dst[e] = cadd(L.G[i * GP + j], L.G2[i * GP + j]);
+  }
+}
+
+// The recorded rotations of n rounds on rows [lo, hi) of the pair's columns of
+// M, a tile at a time in LDS (two pairs a wavefront).
+__device__ void replay(double2* __restrict__ M, int64_t ld, int64_t bi, int64_t bj, int64_t lo,
+                       int64_t hi, const Rot* rec, int n, bool cross, PairLds& L) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int64_t rb = lo; rb < hi; rb += RT) {
+    const int nr = (int)min((int64_t)RT, hi - rb);
+    __syncthreads();
+    load_tile(M, ld, bi, bj, rb, nr, L.tile);
+    __syncthreads();
+    int H = 16, k = 0;
+    for (int m = 0; m < n; ++m) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int t = 2 * wave + i;
+        int a, b;
+        slot_cols(H, t, k, &a, &b);
+        const Rot q = rec[m * NP + t];
+        const double2 x = L.tile[a * TP + lane], y = L.tile[b * TP + lane];
+        L.tile[a * TP + lane] = cfma(make_double2(-q.s.x, q.s.y), y, rscale(q.cs, x));
+        L.tile[b * TP + lane] = cfma(q.s, x, rscale(q.cs, y));
+      }
+      __syncthreads();
+      if (++k == H) {  // the next level; level 16 again after the last (or, cross, at once)
+        k = 0;
+        H = cross || H == 1 ? 16 : H >> 1;
+      }
+    }
+    store_tile(M, ld, bi, bj, rb, nr, L.tile);
+  }
+}
+
+// LDS of item (p, r) as partial_gram left it, in a workgroup that has held
+// other items since.
+__device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r0,
+                       int64_t r1, PairLds& L) {
+  __syncthreads();
+  if (s.R == 1) {
+    partial_gram(s, w, bi, bj, r0, r1, nullptr, L);
+  } else if (r0 < r1) {
+    const int64_t last = r0 + (r1 - r0 - 1) / RT * RT;
+    load_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile);
+  }
+}
+
+// Phases B + C for item (p, r): G = sum of the R partials at src (R > 1), the
+// pair's off-diagonal measure (r == 0) into *off_slot, inner Jacobi, rotation of
+// this chunk's rows of W and V.  prof/pt/t0: phase timing of workgroup 0.
 __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
                             int64_t r, const double2* __restrict__ src,
                             unsigned long long* off_slot, double tol, double tiny2,
-                            int inner_sweeps, bool cross, double2* G, double2* G2,
-                            double2* Q, double2* rot, int* s_active, double2* tile, double* s_off,
-                            bool prof, long long* pt, long long* t0) {
+                            int inner_sweeps, bool cross, PairLds& L, Rot* rec, bool prof,
+                            long long* pt, long long* t0) {
   const int tid = threadIdx.x;
   const int64_t rc = ceil_div(s.len, s.R);
   const int64_t rcv = ceil_div(s.ncolp, s.R);
-  // Upper triangle from the partials; the lower one mirrors it, so G is
-  // exactly Hermitian.
-  for (int e = tid; e < PW * PW; e += blockDim.x) {
+  // Upper triangle; the lower one mirrors it, so G is exactly Hermitian.
+  for (int e = tid; e < PW * PW; e += JT) {
     const int i = e / PW, j = e % PW;
-    Q[i * GP + j] = make_double2((i == j) ? 1.0 : 0.0, 0.0);
     if (i > j) continue;
-    double2 gq[RMAX];
+    double2 g;
+    if (s.R == 1) {
+      g = cadd(L.G[i * GP + j], L.G2[i * GP + j]);
+    } else {
+      double2 gq[RMAX];
 #pragma unroll
-    for (int q = 0; q < RMAX; ++q) gq[q] = (q < s.R) ? src[q * PW * PW + e] : make_double2(0.0, 0.0);
-    double2 g = gq[0];
+      for (int q = 0; q < RMAX; ++q)
+        gq[q] = (q < s.R) ? src[q * PW * PW + e] : make_double2(0.0, 0.0);
+      g = gq[0];
 #pragma unroll
-    for (int q = 1; q < RMAX; ++q) g = cadd(g, gq[q]);
+      for (int q = 1; q < RMAX; ++q) g = cadd(g, gq[q]);
+    }
     if (i == j) g.y = 0.0;
-    G[i * GP + j] = g;
-    G[j * GP + i] = make_double2(g.x, -g.y);
+    L.G[i * GP + j] = g;
+    L.G[j * GP + i] = make_double2(g.x, -g.y);
   }
   __syncthreads();
   // max normalised off-diagonal over non-negligible column pairs (every
   // workgroup of the pair derives the same value from the same G)
   double mx = 0.0;
-  for (int e = tid; e < PW * PW; e += blockDim.x) {
+  for (int e = tid; e < PW * PW; e += JT) {
     const int i = e / PW, j = e % PW;
     if (i < j) {
-      const double gi = G[i * GP + i].x, gj = G[j * GP + j].x;
-      if (gi > tiny2 && gj > tiny2) {
-        const double2 gij = G[i * GP + j];
-        mx = fmax(mx, sqrt(cabs2(gij) / gi / gj));
-      }
+      const double gi = L.G[i * GP + i].x, gj = L.G[j * GP + j].x;
+      if (gi > tiny2 && gj > tiny2) mx = fmax(mx, cabs2(L.G[i * GP + j]) / gi / gj);
     }
   }
   for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-  if ((tid & 63) == 0) s_off[tid >> 6] = mx;
+  if ((tid & 63) == 0) L.off[tid >> 6] = mx;
   __syncthreads();
   double pair_off = 0.0;
-  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) pair_off = fmax(pair_off, s_off[q]);
+  for (int q = 0; q < JT / 64; ++q) pair_off = fmax(pair_off, L.off[q]);
+  pair_off = sqrt(pair_off);
   if (r == 0 && tid == 0) atomicMax(off_slot, (unsigned long long)__double_as_longlong(pair_off));
-  if (pair_off <= tol) {
-    // already orthogonal to tolerance: no rotation is applied to this pair
-    if (prof) {
-      const long long t1 = now_ticks();
-      pt[2] += t1 - *t0;
-      *t0 = t1;
-    }
-    __syncthreads();
-    return;
-  }
   if (prof) {
     const long long t1 = now_ticks();
     pt[2] += t1 - *t0;
     *t0 = t1;
   }
-  inner_jacobi(G, G2, Q, rot, s_active, tol, tiny2, inner_sweeps, nullptr, cross);
+  // already orthogonal to tolerance: no rotation is applied to this pair
+  if (pair_off <= tol) return;
+  const int n = inner_rounds(L, rec, tol, tiny2, inner_sweeps, cross);
   if (prof) {
     const long long t1 = now_ticks();
     pt[3] += t1 - *t0;
     *t0 = t1;
   }
-  // G2 is free after the inner solve: it holds the V tile
-  rotate_rows(w.W, s.len, r * rc, min(s.len, r * rc + rc), w.V, s.ncolp, r * rcv,
-              min(s.ncolp, r * rcv + rcv), bi, bj, Q, tile, G2);
+  // the tile in LDS is the chunk's last one
+  const int64_t r0 = r * rc, r1 = min(s.len, r0 + rc);
+  if (r0 < r1) {
+    const int64_t last = r0 + (r1 - r0 - 1) / RT * RT;
+    store_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile);
+    replay(w.W, s.len, bi, bj, r0, last, rec, n, cross, L);
+  }
+  replay(w.V, s.ncolp, bi, bj, r * rcv, min(s.ncolp, r * rcv + rcv), rec, n, cross, L);
   if (prof) {
     const long long t1 = now_ticks();
     pt[4] += t1 - *t0;
@@ -623,16 +855,10 @@ __device__ inline void local_item(int64_t b, int64_t G, int64_t R, int64_t* p, i
 // counters).  One grid barrier per sweep reduces the convergence measure.
 // !LOCAL: items are strided over the grid, with two grid barriers per step.
 template <bool LOCAL>
-__global__ __launch_bounds__(256) void svd_jacobi(SvdShape s, SvdWork w, double tol,
-                                                  int max_sweeps) {
-  __shared__ double2 tile[PW * RTP];
-  __shared__ double2 G[PW * GP];
-  __shared__ double2 G2[PW * GP];
-  __shared__ double2 Q[PW * GP];
-  __shared__ double2 rot[PW];
-  __shared__ int s_flag;
-  __shared__ int s_active[2];
-  __shared__ double s_off[8];
+__global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double tol,
+                                                 int max_sweeps) {
+  __shared__ PairLds L;
+  extern __shared__ Rot rec[];  // inner_sweeps_of(s) x ROUNDS x NP
 
   const int tid = threadIdx.x;
   const bool prof = (blockIdx.x == 0 && tid == 0);
@@ -641,7 +867,7 @@ __global__ __launch_bounds__(256) void svd_jacobi(SvdShape s, SvdWork w, double 
   const int64_t items = s.P * s.R;
   const int64_t rc = ceil_div(s.len, s.R);  // rows of W per chunk
   const int64_t steps = s.nb - 1;
-  const int inner_sweeps = (s.nb == 2) ? 3 : 1;
+  const int inner_sweeps = inner_sweeps_of(s);
   const double tiny2 = w.ctrl->tiny2;
   const size_t part_stride = (size_t)s.P * RMAX * PW * PW;
   unsigned int* pair_ctr = w.sync;
@@ -670,7 +896,7 @@ __global__ __launch_bounds__(256) void svd_jacobi(SvdShape s, SvdWork w, double 
           const int64_t kp = (k == 0) ? steps - 1 : k - 1;
           const int64_t oi = block_owner(s.nb, kp, bi), oj = block_owner(s.nb, kp, bj);
           if (!wait_counters(w.ctrl, &chunk_ctr[oi * s.R + r], &chunk_ctr[oj * s.R + r],
-                             (unsigned int)g, &s_flag))
+                             (unsigned int)g, &L.flag))
             goto aborted;
         }
         if (prof) {
@@ -679,38 +905,40 @@ __global__ __launch_bounds__(256) void svd_jacobi(SvdShape s, SvdWork w, double 
           t0 = t1;
         }
         partial_gram(s, w, bi, bj, r * rc, min(s.len, r * rc + rc),
-                     part + (p * RMAX + r) * PW * PW, tile);
+                     part + (p * RMAX + r) * PW * PW, L);
         if (prof) {
           const long long t1 = now_ticks();
           pt[0] += t1 - t0;
           t0 = t1;
         }
-        signal_add(&pair_ctr[p]);
-        if (!wait_counters(w.ctrl, &pair_ctr[p], nullptr, (unsigned int)((g + 1) * s.R),
-                           &s_flag))
-          goto aborted;
+        if (s.R > 1) {
+          signal_add(&pair_ctr[p]);
+          if (!wait_counters(w.ctrl, &pair_ctr[p], nullptr, (unsigned int)((g + 1) * s.R),
+                             &L.flag))
+            goto aborted;
+        }
         if (prof) {
           const long long t1 = now_ticks();
           pt[1] += t1 - t0;
           t0 = t1;
         }
         pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                    inner_sweeps, cross, G, G2, Q, rot, s_active, tile, s_off, prof, pt, &t0);
+                    inner_sweeps, cross, L, rec, prof, pt, &t0);
         signal_set(&chunk_ctr[p * s.R + r], (unsigned int)(g + 1));
       } else {
-        for (int64_t it = blockIdx.x; it < items; it += G_) {
+        for (int64_t it = blockIdx.x; it < items && s.R > 1; it += G_) {
           const int64_t p = it / s.R, r = it % s.R;
           int64_t bi, bj;
           pair_blocks(s.nb, k, p, &bi, &bj);
           partial_gram(s, w, bi, bj, r * rc, min(s.len, r * rc + rc),
-                       part + (p * RMAX + r) * PW * PW, tile);
+                       part + (p * RMAX + r) * PW * PW, L);
         }
         if (prof) {
           const long long t1 = now_ticks();
           pt[0] += t1 - t0;
           t0 = t1;
         }
-        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &s_flag)) goto aborted;
+        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
         if (prof) {
           const long long t1 = now_ticks();
           pt[1] += t1 - t0;
@@ -720,16 +948,19 @@ __global__ __launch_bounds__(256) void svd_jacobi(SvdShape s, SvdWork w, double 
           const int64_t p = it / s.R, r = it % s.R;
           int64_t bi, bj;
           pair_blocks(s.nb, k, p, &bi, &bj);
+          // the chunk's last tile (and, R = 1, its Gram matrix) again: L has
+          // held other items since
+          reload(s, w, bi, bj, r * rc, min(s.len, r * rc + rc), L);
           pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                      inner_sweeps, cross, G, G2, Q, rot, s_active, tile, s_off, prof, pt, &t0);
+                      inner_sweeps, cross, L, rec, prof, pt, &t0);
         }
-        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &s_flag)) goto aborted;
+        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
         if (prof) pt[5] += now_ticks() - t0;
       }
     }
     if (LOCAL) {
       // all pairs' measures of this sweep are in *off_slot after the barrier
-      if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &s_flag)) goto aborted;
+      if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
     }
     {
       const unsigned long long bits =
@@ -1037,18 +1268,18 @@ __global__ void truncate_kernel(int64_t N, const double* __restrict__ s, int met
   *err_out = err;
 }
 
-int cooperative_grid(int64_t items, int* grid) {
+// Dynamic LDS of svd_jacobi: the rotations of a step's rounds.
+size_t jacobi_lds(const SvdShape& s) {
+  return (size_t)inner_sweeps_of(s) * ROUNDS * NP * sizeof(Rot);
+}
+
+int cooperative_grid(int64_t items, size_t lds, int* grid) {
   DeviceInfo di;
   int st = device_info(&di);
   if (st) return st;
-  static thread_local int occ_dev = -1, occ = 0;
-  if (occ_dev != di.device) {
-    int o = 0;
-    SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &o, (const void*)svd_jacobi<true>, 256, 0));
-    occ = o;
-    occ_dev = di.device;
-  }
+  int occ = 0;
+  SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)svd_jacobi<true>, JT,
+                                                          lds));
   int64_t lim = (int64_t)occ * di.num_cu;
   if (lim < 1) {
     set_error("svd: kernel cannot be resident on this device");
@@ -1105,7 +1336,7 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
   hipLaunchKernelGGL(svd_frob, dim3(1), dim3(1024), 0, stream, s, w);
   if ((st = check_launch("svd_frob"))) return st;
   int grid = 1;
-  if ((st = cooperative_grid(s.P * s.R, &grid))) return st;
+  if ((st = cooperative_grid(s.P * s.R, jacobi_lds(s), &grid))) return st;
   // Relative orthogonality target: a few times above the rounding floor of the
   // measured Gram entries (~sqrt(len) eps), so that rounding alone cannot keep
   // the measure above it.
@@ -1119,7 +1350,8 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
     // one work item per workgroup when they all fit: local step ordering
     const bool local = (grid == s.P * s.R);
     const void* fn = local ? (const void*)svd_jacobi<true> : (const void*)svd_jacobi<false>;
-    SEEMPS_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(256), args, 0, stream));
+    SEEMPS_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(JT), args, (unsigned)jacobi_lds(s),
+                                          stream));
   }
   hipLaunchKernelGGL(svd_sigma, dim3((unsigned)(s.ncolp < 1024 ? s.ncolp : 1024)), dim3(256), 0,
                      stream, s, w);

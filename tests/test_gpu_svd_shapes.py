@@ -42,3 +42,45 @@ def test_qr_edges(K, m, n):
     assert np.abs(VH @ VH.conj().T - np.eye(r)).max() < 1e-12
     s_ref = np.linalg.svd(A, compute_uv=False)
     assert np.abs(S - s_ref).max() < 5e-13 * s_ref[0]
+
+
+# columns: one block pair (16, 32), an odd number of blocks (33, 48), one more
+# than a tile of rows (65), padding up to 31 columns; the split's orientation
+# for wide and tall matrices
+@pytest.mark.parametrize("m,n", [(2, 40), (16, 16), (32, 32), (33, 40), (48, 33), (65, 65),
+                                 (97, 130), (130, 97), (129, 129), (250, 193)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_split_edges(K, m, n, mode):
+    rng = np.random.default_rng(m * 1000 + n)
+    r = min(m, n)
+    A = crandn(rng, m, r) * np.exp(-20.0 / r * np.arange(r)) @ crandn(rng, r, n)
+    A /= np.linalg.norm(A)
+    u, s, v = np.linalg.svd(A, full_matrices=False)
+    for cap in (r, max(1, r // 2)):
+        Ad, Bd, D, err2, sd = K.svd_split(K.as_dev(A), m, n, mode, 0 if cap == r else 2, 1e-30,
+                                          cap, want_s=True)
+        Ad, Bd = K.to_numpy(Ad), K.to_numpy(Bd)
+        assert D == cap
+        iso = Ad.conj().T @ Ad if mode == 0 else Bd @ Bd.conj().T
+        assert np.abs(iso - np.eye(D)).max() < 1e-12
+        # the kept subspace moves by rounding / (gap at the cut), gap >= s_D / r here
+        assert rel(Ad @ Bd, (u[:, :D] * s[:D]) @ v[:D]) < 1e-12
+        assert np.abs(sd.cpu().numpy() - s[:D]).max() < 5e-13 * s[0]
+        assert abs(err2 - np.sum(s[D:] ** 2)) < 1e-12
+
+
+@pytest.mark.parametrize("n", [1060, 1100])
+def test_svd_beyond_the_register_tiles(K, n):
+    """More than 1024 rows: QR panels in memory, and (35 block pairs leave seven
+    workgroups each) row chunks of three LDS tiles.  A column takes n rotations
+    a sweep for about ten sweeps, so the backward error is bounded by
+    10 n units in the last place of 2 eps each."""
+    rng = np.random.default_rng(n)
+    A = crandn(rng, n, n)
+    A /= np.linalg.norm(A)
+    U, S, VH = K.svd(K.as_dev(A))
+    U, S, VH = K.to_numpy(U), S.cpu().numpy(), K.to_numpy(VH)
+    tol = 20 * n * np.finfo(float).eps
+    assert rel((U * S) @ VH, A) < tol
+    assert np.abs(U.conj().T @ U - np.eye(n)).max() < tol
+    assert np.abs(VH @ VH.conj().T - np.eye(n)).max() < tol
