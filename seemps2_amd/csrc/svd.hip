@@ -34,65 +34,19 @@
 #include <cmath>
 #include <cstdlib>
 
-#include "jacobi_inner.h"
+#include "svd_work.h"
 #include "wave.h"
 
 namespace seemps {
 
 namespace {
 
-using jac::GP;
-using jac::PW;
-
-constexpr int BW = PW / 2;      // block width (columns); PW, GP from jacobi_inner.h
-constexpr int RT = 64;          // rows per LDS tile: a row a lane
-constexpr int RMAX = 16;        // max row chunks per pair
 // Relative off-diagonal measure from which one more sweep is known to suffice
 // (quadratic convergence: the sweep leaves ~1e-18 against a target ~1e-13).
 constexpr double QUAD_STOP = 1e-9;
 constexpr int QR_MIN_COLS = 17; // use the QR preconditioner from this many columns
 constexpr int MAX_SWEEPS = 60;
 constexpr unsigned long long SPIN_LIMIT = 4000000ull;
-
-struct Ctrl {
-  unsigned int barrier;       // grid barrier arrivals
-  unsigned int abort;         // set when a barrier wait timed out
-  unsigned long long off[3];  // per-sweep max normalised off-diagonal (as bits), slot sweep % 3
-  int info[4];                // sweeps, converged, aborted, unused
-  long long prof[8];          // wall-clock ticks of workgroup 0 per phase
-  double frob2;               // ||W||_F^2 (invariant under the rotations)
-  double tiny2;               // squared norm below which a column is negligible
-  double offhist[64];         // off-diagonal measure of each sweep (diagnostics)
-};
-
-struct SvdShape {
-  int64_t m, n;         // input shape
-  int64_t lenA, ncol;   // working matrix B: ncol columns of length lenA
-  int64_t len;          // Jacobi column length (ncol with QR, lenA without)
-  int64_t nb, ncolp;    // blocks (even), padded column count
-  int64_t P, R;         // pairs per step, row chunks
-  int transposed;       // 1 if B = A^H
-  int use_qr;
-  int cross_inner;      // inner solves after a sweep's first step: cross-block pairs only
-};
-
-struct SvdWork {
-  double2* Acm;   // ncol x lenA (QR in place)
-  double2* Vall;  // ncol x lenA (QR vectors)
-  double2* tau;   // ncol
-  double2* Y;     // ncol x lenA (Q V)
-  double2* W;     // ncolp x len
-  double2* V;     // ncolp x ncolp
-  double2* part;  // 2 x P x RMAX x PW x PW (partial Grams, by step parity)
-  unsigned int* sync;  // P pair arrival counters, then P x R chunk step counters
-  double* colnrm;  // ncol squared column norms of B (QR path)
-  int* colperm;    // ncol: B's columns by decreasing norm (QR path)
-  double* sigma;  // ncolp
-  int* perm;      // ncolp
-  Ctrl* ctrl;
-};
-
-inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 SvdShape svd_shape(int64_t m, int64_t n, int num_cu, bool precondition = true) {
   SvdShape s;
@@ -103,49 +57,22 @@ SvdShape svd_shape(int64_t m, int64_t n, int num_cu, bool precondition = true) {
   s.ncol = s.transposed ? m : n;
   s.use_qr = precondition && (s.ncol >= QR_MIN_COLS);
   s.len = s.use_qr ? s.ncol : s.lenA;
-  int64_t nb = ceil_div(s.ncol, BW);
-  if (nb < 2) nb = 2;
-  nb += (nb & 1);
-  s.nb = nb;
-  s.ncolp = nb * BW;
-  s.P = nb / 2;
-  // Row chunks per pair: a tile each, as far as one workgroup per CU allows.
-  // The chunk's rotations then hide behind the inner rounds; a longer chunk
-  // replays them tile by tile.
-  int64_t R = num_cu / s.P;
-  // tuning knob: cap on the row chunks per pair (SEEMPS_SVD_ROW_CHUNKS)
-  static const int64_t r_cap = [] {
-    const char* e = getenv("SEEMPS_SVD_ROW_CHUNKS");
-    const long v = e ? atol(e) : 0;
-    return (int64_t)(v > 0 ? v : RMAX);
-  }();
-  if (R > r_cap) R = r_cap;
-  const int64_t rmax_len = ceil_div(s.len, RT);
-  if (R > rmax_len) R = rmax_len;
-  if (R > RMAX) R = RMAX;
-  if (R < 1) R = 1;
-  s.R = R;
-  // Inner solves: every block's own pairs are visited at the first step of a
-  // sweep (each block meets one partner there); with cross_inner the later
-  // steps rotate only the pairs across the two blocks (16 rounds instead of
-  // 31).  Measured over whole chi=256 DMRG sweeps this is faster in both the
-  // QR-preconditioned and the basis-sketched splits (more sweeps at times,
-  // each about half as long); the convergence test is the same either way.
-  // SEEMPS_SVD_INNER=full restores the full inner sweep at every step, and
-  // SEEMPS_SVD_INNER=hybrid keeps it for the first sweep only (tuning: hybrid
-  // converges the sketch matrices in fewer sweeps, but lost over DMRG sweeps).
-  static const int inner_mode = [] {
-    const char* e = getenv("SEEMPS_SVD_INNER");
-    if (e && strcmp(e, "full") == 0) return 0;
-    if (e && strcmp(e, "hybrid") == 0) return 2;  // full inner sweeps in sweep 0
-    return 1;
-  }();
-  s.cross_inner = s.nb > 2 ? inner_mode : 0;
+  jacobi_shape(&s, num_cu);
   return s;
 }
 
-// Inner sweeps per step: a single pair (two blocks) has nothing to wait for.
-__host__ __device__ inline int inner_sweeps_of(const SvdShape& s) { return s.nb == 2 ? 3 : 1; }
+// Inner sweeps per step: a single pair (two blocks) has nothing to wait for, but
+// tiles that replay the rotations find only the last sweep's.
+__host__ __device__ inline int inner_sweeps_of(const SvdShape& s) {
+  return s.nb == 2 && ceil_div(s.len, s.R) <= RT && ceil_div(s.ncolp, s.R) <= RT ? 3 : 1;
+}
+// First level of a full inner sweep: of 32 indices, unless a single pair holds
+// fewer columns (the padding is zero and takes no rotation).
+__host__ __device__ inline int inner_top_of(const SvdShape& s) {
+  int top = 16;
+  while (s.nb == 2 && top > 1 && s.ncol <= top) top >>= 1;
+  return top;
+}
 
 #define SEEMPS_SVD_REGIONS(X)                                         \
   X(Acm, s.use_qr ? s.ncol * s.lenA : 0, double2)                     \
@@ -361,9 +288,10 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
 
 // ---- one block pair on one workgroup --------------------------------------
 //
-// 512 threads.  A tile of RT rows of the pair's PW columns sits in LDS
-// (column-major, padded); its Gram matrix is taken from it on the matrix cores,
-// then the inner Jacobi rotates G and the tile in registers.
+// 768 threads.  A tile of RT rows of the pair's PW columns of W sits in LDS
+// (column-major, padded), and one of V; the Gram matrix is taken from the former
+// on the matrix cores, then the inner Jacobi rotates G and both tiles in
+// registers.
 //
 // A level H of the inner Jacobi pairs index base + t with base + H + (t + k) mod H
 // in round k (base = 0, 2H, ..): H rounds of 16 disjoint rotations that visit
@@ -372,8 +300,8 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
 // pair of the 32.  The first index of a pair stays where it is and the second
 // moves one place a round, so wavefronts 0-3 keep G in registers, a 2 x 2 block
 // a thread, and pass entries to the neighbouring thread: along a row of threads
-// by DPP, between rows through LDS.  Wavefronts 4-7 hold the tile, a row a lane,
-// four pairs of columns a wavefront, and pass one column a round.  One barrier
+// by DPP, between rows through LDS.  Wavefronts 4-7 hold W's tile, a row a lane,
+// four pairs of columns a wavefront, and pass one column a round; 8-11 hold V's.  One barrier
 // a round: the thread that holds pair p's own block derives its rotation from
 // what it has (the second index's diagonal entry comes with that pair's
 // rotation), everyone applies it after the barrier.
@@ -381,7 +309,7 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
 // A round takes 0.51 us, two thirds of it instruction issue (48 FP64
 // operations a thread in either role, the rotation's chain of 45); with G and
 // the tile in LDS it took 1.07 us, LDS traffic (100 KB a round).
-constexpr int JT = 512;            // threads
+constexpr int JT = 768;            // threads
 constexpr int TP = RT + 1;         // padded tile column (complex)
 constexpr int NP = PW / 2;         // pairs a round
 constexpr int ROUNDS = PW - 1;     // rounds of all levels
@@ -417,10 +345,14 @@ __device__ __forceinline__ double lane_next(double x) {
 }
 
 struct PairLds {
-  double2 tile[PW * TP];
-  double2 G[PW * GP], G2[PW * GP];
-  double2 sh[2][2][NP * NP];  // second rows of the 2 x 2 blocks, by round parity
-  double2 xch[2][4][RT];      // the tile columns on their way
+  double2 tile[2][PW * TP];   // of W, of V
+  double2 G[PW * GP];
+  union {
+    double2 G2[PW * GP];          // second half's Gram matrix
+    double2 sh[2][2][NP * NP];    // second rows of the 2 x 2 blocks, by round parity
+  };
+  double2 xch[2][2][4][RT];   // the tiles' columns on their way, by round parity
+  Rot rec[ROUNDS * NP];       // rotations of a sweep's rounds
   double off[JT / 64];
   int flag;
 };
@@ -457,8 +389,8 @@ __device__ __forceinline__ double2 rscale(double f, double2 x) {
   return make_double2(f * x.x, f * x.y);
 }
 
-// Level H on L.G and L.tile, on every wavefront of the workgroup; rec receives
-// its H x NP rotations.  Ends with a barrier.
+// Level H on L.G and the tiles, on every wavefront of the workgroup; rec
+// receives its H x NP rotations.  Ends with a barrier.
 template <int H>
 __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, double tiny2) {
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -505,22 +437,23 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
     L.G[b * GP + c] = bc;
     L.G[b * GP + d] = bd;
   } else {
-    const int w = wv - 4;
+    const int w = wv & 3, which = wv >= 8;
+    double2* tile = L.tile[which];
     const int wn = H == 16 ? (w + 1) & 3 : H == 8 ? w ^ 1 : w;  // owner of the column to come
     double2 xa[4], xb[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       int a, b;
       slot_cols(H, 4 * w + i, 0, &a, &b);
-      xa[i] = L.tile[a * TP + lane];
-      xb[i] = L.tile[b * TP + lane];
+      xa[i] = tile[a * TP + lane];
+      xb[i] = tile[b * TP + lane];
     }
 #pragma unroll 2
     for (int k = 0; k < H; ++k) {
       __syncthreads();
       // the four rotations (16 doubles) in the lanes, broadcast from there
       const double rd = ((const double*)(rec + k * NP + 4 * w))[lane & 15];
-      if (H >= 8 && k > 0) xb[3] = L.xch[k & 1][wn][lane];
+      if (H >= 8 && k > 0) xb[3] = L.xch[k & 1][which][wn][lane];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const double cs = wave::bcast(rd, 4 * i);
@@ -538,7 +471,7 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
           xb[2] = xb[3];
           xb[3] = y;
         } else {
-          if (H >= 8) L.xch[(k + 1) & 1][w][lane] = x;
+          if (H >= 8) L.xch[(k + 1) & 1][which][w][lane] = x;
           xb[0] = xb[1];
           xb[1] = xb[2];
           xb[2] = xb[3];
@@ -550,27 +483,40 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
     for (int i = 0; i < 4; ++i) {
       int a, b;
       slot_cols(H, 4 * w + i, H - 1, &a, &b);
-      L.tile[a * TP + lane] = xa[i];
-      L.tile[b * TP + lane] = xb[i];
+      tile[a * TP + lane] = xa[i];
+      tile[b * TP + lane] = xb[i];
     }
   }
   __syncthreads();
 }
 
-// Inner sweeps: level 16 (cross) or all levels.  Returns the number of rounds.
-__device__ int inner_rounds(PairLds& L, Rot* rec, double tol, double tiny2, int sweeps,
-                            bool cross) {
+// Inner sweeps: level 16 (cross) or the levels from top down to 1.  Returns the
+// number of rounds of the last one, whose rotations L.rec holds.
+__device__ int inner_rounds(PairLds& L, double tol, double tiny2, int sweeps, bool cross, int top) {
   const double tol2 = tol * tol;
+  Rot* rec = L.rec;
   int n = 0;
   for (int sw = 0; sw < sweeps; ++sw) {
-    inner_level<16>(L, rec + n * NP, tol2, tiny2);
-    n += 16;
-    if (cross) continue;
-    inner_level<8>(L, rec + n * NP, tol2, tiny2);
-    inner_level<4>(L, rec + (n + 8) * NP, tol2, tiny2);
-    inner_level<2>(L, rec + (n + 12) * NP, tol2, tiny2);
-    inner_level<1>(L, rec + (n + 14) * NP, tol2, tiny2);
-    n += 15;
+    n = 0;
+    if (top == 16) {
+      inner_level<16>(L, rec + n * NP, tol2, tiny2);
+      n += 16;
+      if (cross) continue;
+    }
+    if (top >= 8) {
+      inner_level<8>(L, rec + n * NP, tol2, tiny2);
+      n += 8;
+    }
+    if (top >= 4) {
+      inner_level<4>(L, rec + n * NP, tol2, tiny2);
+      n += 4;
+    }
+    if (top >= 2) {
+      inner_level<2>(L, rec + n * NP, tol2, tiny2);
+      n += 2;
+    }
+    inner_level<1>(L, rec + n * NP, tol2, tiny2);
+    n += 1;
   }
   return n;
 }
@@ -591,7 +537,7 @@ __device__ __forceinline__ void store_tile(double2* __restrict__ M, int64_t ld, 
   }
 }
 
-// One of the 12 shares of the Gram matrix's upper 16 x 16 tiles: tile
+// A wavefront's share of the Gram matrix's upper 16 x 16 tiles: tile
 // (00, 11 or 01), real or imaginary part, first or second half of the rows.
 struct GramShare {
   int ti, tj, im, half;
@@ -632,19 +578,16 @@ __device__ __forceinline__ void gram_store(double2* dst, GramShare q, d4 acc) {
 // left in L.G and L.G2.
 __device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
                              int64_t r0, int64_t r1, double2* __restrict__ dst, PairLds& L) {
-  const int wave = threadIdx.x >> 6;
-  const GramShare q0 = gram_share(wave), q1 = gram_share(wave + 8 < 12 ? wave + 8 : 0);
-  d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0;
+  const GramShare q = gram_share(threadIdx.x >> 6);
+  d4 c = {0.0, 0.0, 0.0, 0.0};
   for (int64_t rb = r0; rb == r0 || rb < r1; rb += RT) {
     const int nr = (int)max((int64_t)0, min((int64_t)RT, r1 - rb));
     __syncthreads();
-    load_tile(w.W, s.len, bi, bj, rb, nr, L.tile);
+    load_tile(w.W, s.len, bi, bj, rb, nr, L.tile[0]);
     __syncthreads();
-    gram_accumulate(L.tile, nr, q0, &c0);
-    if (wave + 8 < 12) gram_accumulate(L.tile, nr, q1, &c1);
+    gram_accumulate(L.tile[0], nr, q, &c);
   }
-  gram_store(q0.half ? L.G2 : L.G, q0, c0);
-  if (wave + 8 < 12) gram_store(q1.half ? L.G2 : L.G, q1, c1);
+  gram_store(q.half ? L.G2 : L.G, q, c);
   __syncthreads();
   if (s.R == 1) return;
   for (int e = threadIdx.x; e < PW * PW; e += JT) {
@@ -654,34 +597,33 @@ __device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, in
 }
 
 // The recorded rotations of n rounds on rows [lo, hi) of the pair's columns of
-// M, a tile at a time in LDS (two pairs a wavefront).
+// M, a tile at a time in LDS.
 __device__ void replay(double2* __restrict__ M, int64_t ld, int64_t bi, int64_t bj, int64_t lo,
-                       int64_t hi, const Rot* rec, int n, bool cross, PairLds& L) {
+                       int64_t hi, int n, bool cross, int top, PairLds& L) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int64_t rb = lo; rb < hi; rb += RT) {
     const int nr = (int)min((int64_t)RT, hi - rb);
     __syncthreads();
-    load_tile(M, ld, bi, bj, rb, nr, L.tile);
+    double2* tile = L.tile[0];
+    load_tile(M, ld, bi, bj, rb, nr, tile);
     __syncthreads();
-    int H = 16, k = 0;
+    int H = top, k = 0;
     for (int m = 0; m < n; ++m) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int t = 2 * wave + i;
+      for (int t = wave; t < NP; t += JT / 64) {
         int a, b;
         slot_cols(H, t, k, &a, &b);
-        const Rot q = rec[m * NP + t];
-        const double2 x = L.tile[a * TP + lane], y = L.tile[b * TP + lane];
-        L.tile[a * TP + lane] = cfma(make_double2(-q.s.x, q.s.y), y, rscale(q.cs, x));
-        L.tile[b * TP + lane] = cfma(q.s, x, rscale(q.cs, y));
+        const Rot q = L.rec[m * NP + t];
+        const double2 x = tile[a * TP + lane], y = tile[b * TP + lane];
+        tile[a * TP + lane] = cfma(make_double2(-q.s.x, q.s.y), y, rscale(q.cs, x));
+        tile[b * TP + lane] = cfma(q.s, x, rscale(q.cs, y));
       }
       __syncthreads();
-      if (++k == H) {  // the next level; level 16 again after the last (or, cross, at once)
+      if (++k == H) {  // the next level; the first again after the last (or, cross, at once)
         k = 0;
-        H = cross || H == 1 ? 16 : H >> 1;
+        H = cross || H == 1 ? top : H >> 1;
       }
     }
-    store_tile(M, ld, bi, bj, rb, nr, L.tile);
+    store_tile(M, ld, bi, bj, rb, nr, tile);
   }
 }
 
@@ -694,7 +636,7 @@ __device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t 
     partial_gram(s, w, bi, bj, r0, r1, nullptr, L);
   } else if (r0 < r1) {
     const int64_t last = r0 + (r1 - r0 - 1) / RT * RT;
-    load_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile);
+    load_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile[0]);
   }
 }
 
@@ -704,8 +646,8 @@ __device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t 
 __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
                             int64_t r, const double2* __restrict__ src,
                             unsigned long long* off_slot, double tol, double tiny2,
-                            int inner_sweeps, bool cross, PairLds& L, Rot* rec, bool prof,
-                            long long* pt, long long* t0) {
+                            int inner_sweeps, bool cross, PairLds& L, bool prof, long long* pt,
+                            long long* t0) {
   const int tid = threadIdx.x;
   const int64_t rc = ceil_div(s.len, s.R);
   const int64_t rcv = ceil_div(s.ncolp, s.R);
@@ -717,13 +659,15 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
     if (s.R == 1) {
       g = cadd(L.G[i * GP + j], L.G2[i * GP + j]);
     } else {
-      double2 gq[RMAX];
+      g = make_double2(0.0, 0.0);
+      for (int q0 = 0; q0 < s.R; q0 += 4) {
+        double2 gq[4];
 #pragma unroll
-      for (int q = 0; q < RMAX; ++q)
-        gq[q] = (q < s.R) ? src[q * PW * PW + e] : make_double2(0.0, 0.0);
-      g = gq[0];
+        for (int q = 0; q < 4; ++q)
+          gq[q] = (q0 + q < s.R) ? src[(q0 + q) * PW * PW + e] : make_double2(0.0, 0.0);
 #pragma unroll
-      for (int q = 1; q < RMAX; ++q) g = cadd(g, gq[q]);
+        for (int q = 0; q < 4; ++q) g = cadd(g, gq[q]);
+      }
     }
     if (i == j) g.y = 0.0;
     L.G[i * GP + j] = g;
@@ -754,7 +698,13 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
   }
   // already orthogonal to tolerance: no rotation is applied to this pair
   if (pair_off <= tol) return;
-  const int n = inner_rounds(L, rec, tol, tiny2, inner_sweeps, cross);
+  const int64_t v0 = r * rcv, v1 = min(s.ncolp, v0 + rcv);
+  const bool v_live = w.V && rcv <= RT && v0 < v1;  // V's rows of this chunk are one tile
+  if (v_live) {
+    load_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
+    __syncthreads();
+  }
+  const int n = inner_rounds(L, tol, tiny2, inner_sweeps, cross, inner_top_of(s));
   if (prof) {
     const long long t1 = now_ticks();
     pt[3] += t1 - *t0;
@@ -764,10 +714,13 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
   const int64_t r0 = r * rc, r1 = min(s.len, r0 + rc);
   if (r0 < r1) {
     const int64_t last = r0 + (r1 - r0 - 1) / RT * RT;
-    store_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile);
-    replay(w.W, s.len, bi, bj, r0, last, rec, n, cross, L);
+    store_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile[0]);
+    replay(w.W, s.len, bi, bj, r0, last, n, cross, inner_top_of(s), L);
   }
-  replay(w.V, s.ncolp, bi, bj, r * rcv, min(s.ncolp, r * rcv + rcv), rec, n, cross, L);
+  if (v_live)
+    store_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
+  else if (w.V)
+    replay(w.V, s.ncolp, bi, bj, v0, v1, n, cross, inner_top_of(s), L);
   if (prof) {
     const long long t1 = now_ticks();
     pt[4] += t1 - *t0;
@@ -858,7 +811,6 @@ template <bool LOCAL>
 __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double tol,
                                                  int max_sweeps) {
   __shared__ PairLds L;
-  extern __shared__ Rot rec[];  // inner_sweeps_of(s) x ROUNDS x NP
 
   const int tid = threadIdx.x;
   const bool prof = (blockIdx.x == 0 && tid == 0);
@@ -923,7 +875,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           t0 = t1;
         }
         pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                    inner_sweeps, cross, L, rec, prof, pt, &t0);
+                    inner_sweeps, cross, L, prof, pt, &t0);
         signal_set(&chunk_ctr[p * s.R + r], (unsigned int)(g + 1));
       } else {
         for (int64_t it = blockIdx.x; it < items && s.R > 1; it += G_) {
@@ -952,7 +904,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           // held other items since
           reload(s, w, bi, bj, r * rc, min(s.len, r * rc + rc), L);
           pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                      inner_sweeps, cross, L, rec, prof, pt, &t0);
+                      inner_sweeps, cross, L, prof, pt, &t0);
         }
         if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
         if (prof) pt[5] += now_ticks() - t0;
@@ -1082,23 +1034,18 @@ __global__ void svd_output(SvdShape s, SvdWork w, double2* __restrict__ U, doubl
 // 1 - leverage >= 1 - k/len > 0, so the completion cannot fail.  Projection is
 // classical Gram-Schmidt applied twice, one wavefront per dot product.  Only
 // slots k < *kmax are completed when kmax is given (the caller keeps no more).
-// One workgroup of 1024 threads; coef holds at least ncol complex values.
-__global__ __launch_bounds__(1024) void svd_complete(SvdShape s, SvdWork w, double2* __restrict__ U,
-                                                     double2* __restrict__ VH,
-                                                     const int64_t* __restrict__ kmax) {
-  const int64_t r = s.ncol, len = s.len;
-  const int wside_u = (s.use_qr == s.transposed);
-  // element x of W-side vector k, as a plain (unconjugated) vector component
+// One workgroup of 1024 threads; w.part holds at least r complex values.
+__global__ __launch_bounds__(1024) void svd_complete(SvdWork w, double2* __restrict__ base,
+                                                     int64_t sk, int64_t sx, int conj, int64_t r,
+                                                     int64_t len, const int64_t* __restrict__ kmax) {
+  const double cy = conj ? -1.0 : 1.0;
+  // component x of vector k, as a plain (unconjugated) one
   auto load = [&](int64_t k, int64_t x) -> double2 {
-    if (wside_u) return U[x * r + k];
-    const double2 v = VH[k * s.n + x];
-    return make_double2(v.x, -v.y);
+    const double2 v = base[k * sk + x * sx];
+    return make_double2(v.x, cy * v.y);
   };
   auto store = [&](int64_t k, int64_t x, double2 v) {
-    if (wside_u)
-      U[x * r + k] = v;
-    else
-      VH[k * s.n + x] = make_double2(v.x, -v.y);
+    base[k * sk + x * sx] = make_double2(v.x, cy * v.y);
   };
   __shared__ double s_val[16];
   __shared__ int64_t s_idx[16];
@@ -1204,15 +1151,12 @@ __global__ __launch_bounds__(1024) void svd_complete(SvdShape s, SvdWork w, doub
   }
 }
 
-// Truncation rule: one lane runs the reference's sequential loops (summation
-// order identical to truncation.pxi:251-327, products and sums rounded
-// separately as in the reference's compiled loops) over an LDS copy of s
+// Truncation rule: one lane runs it over an LDS copy of s
 // (STAGED, spectra of up to TRUNC_STAGE values) or over s itself.
 constexpr int64_t TRUNC_STAGE = 4096;
 template <bool STAGED>
 __global__ void truncate_kernel(int64_t N, const double* __restrict__ s, int method, double tol,
                                 int64_t max_bond, int64_t* D_out, double* err_out) {
-#pragma clang fp contract(off)
   extern __shared__ double stage[];
   if (STAGED) {
     for (int64_t i = threadIdx.x; i < N; i += blockDim.x) stage[i] = s[i];
@@ -1220,66 +1164,21 @@ __global__ void truncate_kernel(int64_t N, const double* __restrict__ s, int met
   }
   const double* ss = STAGED ? stage : s;
   if (threadIdx.x != 0) return;
-  int64_t D = N;
-  double err = 0.0;
-  if (method == SEEMPS_TRUNC_NONE) {
-    D = N;
-    err = 0.0;
-  } else if (method == SEEMPS_TRUNC_REL_NORM2) {
-    // errors[i] = sum of the i smallest s^2, accumulated from the smallest.
-    double total = 0.0;
-    for (int64_t i = 0; i < N; ++i) {
-      const double x = ss[N - 1 - i];
-      total += x * x;
-    }
-    const double max_error = total * tol;
-    double acc = 0.0;
-    int64_t i_stop = N - 1;
-    for (int64_t i = 0; i < N; ++i) {
-      if (acc > max_error) {
-        i_stop = i - 1;
-        break;
-      }
-      const double x = ss[N - 1 - i];
-      acc += x * x;
-    }
-    D = N - i_stop;
-    if (D > max_bond) D = max_bond;
-    double e = 0.0;  // errors[N - D]
-    for (int64_t i = 0; i < N - D; ++i) {
-      const double x = ss[N - 1 - i];
-      e += x * x;
-    }
-    err = e;
-  } else {
-    const double thr = (method == SEEMPS_TRUNC_REL_SV) ? tol * ss[0] : tol;
-    D = (N < max_bond) ? N : max_bond;
-    for (int64_t i = 1; i < D; ++i) {
-      if (ss[i] <= thr) {
-        D = i;
-        break;
-      }
-    }
-    double e = 0.0;
-    for (int64_t i = D; i < N; ++i) e += ss[i] * ss[i];
-    err = e;
-  }
-  *D_out = D;
-  *err_out = err;
+  truncation_rule(N, ss, method, tol, max_bond, D_out, err_out);
 }
 
-// Dynamic LDS of svd_jacobi: the rotations of a step's rounds.
-size_t jacobi_lds(const SvdShape& s) {
-  return (size_t)inner_sweeps_of(s) * ROUNDS * NP * sizeof(Rot);
-}
-
-int cooperative_grid(int64_t items, size_t lds, int* grid) {
+int cooperative_grid(int64_t items, int* grid) {
   DeviceInfo di;
   int st = device_info(&di);
   if (st) return st;
-  int occ = 0;
-  SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)svd_jacobi<true>, JT,
-                                                          lds));
+  static thread_local int occ_dev = -1, occ = 0;
+  if (occ_dev != di.device) {
+    int o = 0;
+    SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &o, (const void*)svd_jacobi<true>, JT, 0));
+    occ = o;
+    occ_dev = di.device;
+  }
   int64_t lim = (int64_t)occ * di.num_cu;
   if (lim < 1) {
     set_error("svd: kernel cannot be resident on this device");
@@ -1298,6 +1197,87 @@ unsigned blocks_for(int64_t n) {
   return (unsigned)b;
 }
 
+}  // namespace
+
+void jacobi_shape(SvdShape* s, int num_cu) {
+  int64_t nb = ceil_div(s->ncol, BW);
+  if (nb < 2) nb = 2;
+  nb += (nb & 1);
+  s->nb = nb;
+  s->ncolp = nb * BW;
+  s->P = nb / 2;
+  // Row chunks per pair: a tile each, as far as one workgroup per CU allows.
+  // The chunk's rotations then hide behind the inner rounds; a longer chunk
+  // replays them tile by tile.
+  int64_t R = num_cu / s->P;
+  // tuning knob: cap on the row chunks per pair (SEEMPS_SVD_ROW_CHUNKS)
+  static const int64_t r_cap = [] {
+    const char* e = getenv("SEEMPS_SVD_ROW_CHUNKS");
+    const long v = e ? atol(e) : 0;
+    return (int64_t)(v > 0 ? v : RMAX);
+  }();
+  if (R > r_cap) R = r_cap;
+  const int64_t rmax_len = ceil_div(s->len, RT);
+  if (R > rmax_len) R = rmax_len;
+  if (R > RMAX) R = RMAX;
+  if (R < 1) R = 1;
+  s->R = R;
+  // Inner solves: every block's own pairs are visited at the first step of a
+  // sweep (each block meets one partner there); with cross_inner the later
+  // steps rotate only the pairs across the two blocks (16 rounds instead of
+  // 31).  Measured over whole chi=256 DMRG sweeps this is faster in both the
+  // QR-preconditioned and the basis-sketched splits (more sweeps at times,
+  // each about half as long); the convergence test is the same either way.
+  // SEEMPS_SVD_INNER=full restores the full inner sweep at every step, and
+  // SEEMPS_SVD_INNER=hybrid keeps it for the first sweep only (tuning: hybrid
+  // converges the sketch matrices in fewer sweeps, but lost over DMRG sweeps).
+  static const int inner_mode = [] {
+    const char* e = getenv("SEEMPS_SVD_INNER");
+    if (e && strcmp(e, "full") == 0) return 0;
+    if (e && strcmp(e, "hybrid") == 0) return 2;  // full inner sweeps in sweep 0
+    return 1;
+  }();
+  s->cross_inner = s->nb > 2 ? inner_mode : 0;
+}
+
+int jacobi_enqueue(const SvdShape& s, const SvdWork& w, hipStream_t stream) {
+  int st, grid = 1;
+  if ((st = cooperative_grid(s.P * s.R, &grid))) return st;
+  // Relative orthogonality target: a few times above the rounding floor of the
+  // measured Gram entries (~sqrt(len) eps), so that rounding alone cannot keep
+  // the measure above it.
+  double tol = 32.0 * sqrt((double)s.len) * 2.220446049250313e-16;
+  int max_sweeps = MAX_SWEEPS;
+  void* args[] = {(void*)&s, (void*)&w, (void*)&tol, (void*)&max_sweeps};
+  // nominal SVD flops (complex): 4 * (6 M N^2 + 16 N^3), M >= N
+  const double M_ = (double)s.lenA, N_ = (double)s.ncol;
+  TimedLaunch timed("svd_jacobi", stream, 4.0 * (6.0 * M_ * N_ * N_ + 16.0 * N_ * N_ * N_));
+  // one work item per workgroup when they all fit: local step ordering
+  const void* fn = grid == s.P * s.R ? (const void*)svd_jacobi<true> : (const void*)svd_jacobi<false>;
+  if (grid == 1) {  // nothing to be resident with
+    SEEMPS_HIP(hipLaunchKernel(fn, dim3(1), dim3(JT), args, 0, stream));
+    return SEEMPS_OK;
+  }
+  SEEMPS_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(JT), args, 0, stream));
+  return SEEMPS_OK;
+}
+
+int complete_enqueue(const SvdWork& w, double2* base, int64_t sk, int64_t sx, int conj, int64_t r,
+                     int64_t len, const int64_t* kmax, hipStream_t stream) {
+  TimedLaunch timed("svd_complete", stream, 0.0);
+  hipLaunchKernelGGL(svd_complete, dim3(1), dim3(1024), 0, stream, w, base, sk, sx, conj, r, len,
+                     kmax);
+  return check_launch("svd_complete");
+}
+
+namespace {
+// The W side's vectors among the outputs: columns of U, or conjugated rows of VH.
+int complete_sides(const SvdShape& s, const SvdWork& w, double2* U, double2* VH,
+                   const int64_t* kmax, hipStream_t stream) {
+  if (s.use_qr == s.transposed)
+    return complete_enqueue(w, U, 1, s.ncol, 0, s.ncol, s.len, kmax, stream);
+  return complete_enqueue(w, VH, s.n, 1, 1, s.ncol, s.len, kmax, stream);
+}
 }  // namespace
 
 // Enqueue the SVD.  With kmax_dev == nullptr every slot is completed; otherwise
@@ -1335,24 +1315,7 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
   if ((st = check_launch("init_v_ctrl"))) return st;
   hipLaunchKernelGGL(svd_frob, dim3(1), dim3(1024), 0, stream, s, w);
   if ((st = check_launch("svd_frob"))) return st;
-  int grid = 1;
-  if ((st = cooperative_grid(s.P * s.R, jacobi_lds(s), &grid))) return st;
-  // Relative orthogonality target: a few times above the rounding floor of the
-  // measured Gram entries (~sqrt(len) eps), so that rounding alone cannot keep
-  // the measure above it.
-  const double tol = 32.0 * sqrt((double)s.len) * 2.220446049250313e-16;
-  int max_sweeps = MAX_SWEEPS;
-  void* args[] = {(void*)&s, (void*)&w, (void*)&tol, (void*)&max_sweeps};
-  {
-    // nominal SVD flops (complex): 4 * (6 M N^2 + 16 N^3), M >= N
-    const double M_ = (double)s.lenA, N_ = (double)s.ncol;
-    TimedLaunch timed("svd_jacobi", stream, 4.0 * (6.0 * M_ * N_ * N_ + 16.0 * N_ * N_ * N_));
-    // one work item per workgroup when they all fit: local step ordering
-    const bool local = (grid == s.P * s.R);
-    const void* fn = local ? (const void*)svd_jacobi<true> : (const void*)svd_jacobi<false>;
-    SEEMPS_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(JT), args, (unsigned)jacobi_lds(s),
-                                          stream));
-  }
+  if ((st = jacobi_enqueue(s, w, stream))) return st;
   hipLaunchKernelGGL(svd_sigma, dim3((unsigned)(s.ncolp < 1024 ? s.ncolp : 1024)), dim3(256), 0,
                      stream, s, w);
   if ((st = check_launch("svd_sigma"))) return st;
@@ -1371,12 +1334,7 @@ int svd_enqueue(int64_t m, int64_t n, const double2* A, int64_t lda, double2* U,
   const int64_t big = s.ncol * (s.len > s.lenA ? s.len : s.lenA);
   hipLaunchKernelGGL(svd_output, dim3(blocks_for(big)), dim3(256), 0, stream, s, w, U, S, VH);
   if ((st = check_launch("svd_output"))) return st;
-  if (complete) {
-    TimedLaunch timed("svd_complete", stream, 0.0);
-    hipLaunchKernelGGL(svd_complete, dim3(1), dim3(1024), 0, stream, s, w, U, VH,
-                       (const int64_t*)nullptr);
-    if ((st = check_launch("svd_complete"))) return st;
-  }
+  if (complete && (st = complete_sides(s, w, U, VH, nullptr, stream))) return st;
   if (info_dev_off) *info_dev_off = (int)((char*)w.ctrl - (char*)work);
   return SEEMPS_OK;
 }
@@ -1389,9 +1347,7 @@ int svd_complete_enqueue(int64_t m, int64_t n, double2* U, double2* VH, void* wo
   if (st) return st;
   const SvdShape s = svd_shape(m, n, di.num_cu, precondition);
   SvdWork w = svd_carve(s, work);
-  TimedLaunch timed("svd_complete", stream, 0.0);
-  hipLaunchKernelGGL(svd_complete, dim3(1), dim3(1024), 0, stream, s, w, U, VH, kmax_dev);
-  return check_launch("svd_complete");
+  return complete_sides(s, w, U, VH, kmax_dev, stream);
 }
 
 int64_t svd_workspace_bytes(int64_t m, int64_t n, bool precondition) {
@@ -1424,6 +1380,10 @@ int svd_read_ctrl(void* work, int off, int32_t* info, hipStream_t stream) {
   SEEMPS_HIP(hipStreamSynchronize(stream));
   Ctrl h;
   memcpy(&h, hp, sizeof(h));
+  return ctrl_status(h, info);
+}
+
+int ctrl_status(const Ctrl& h, int32_t* info) {
   if (info) {
     info[0] = h.info[0];
     info[1] = h.info[1];
@@ -1480,74 +1440,4 @@ extern "C" int seemps_truncate(int64_t N, const double* s, int method, double to
                                int64_t max_bond, int64_t* D_out, double* err_out, void* stream) {
   return seemps::truncate_enqueue(N, s, method, tolerance, max_bond, D_out, err_out,
                                   (hipStream_t)stream);
-}
-
-namespace seemps {
-
-int64_t svd_split_bytes(int64_t m, int64_t n) {
-  const int64_t r = m < n ? m : n;
-  auto al = [](int64_t x) { return (x + 255) & ~int64_t(255); };
-  return al(m * r * 16) + al(r * 8) + al(r * n * 16) + al(64) + svd_workspace_bytes(m, n);
-}
-
-int svd_split_impl(int64_t m, int64_t n, const double2* A, int mode, int method, double tolerance,
-                   int64_t max_bond, double2* outA, double2* outB, double* s_out,
-                   int64_t* D_host, double* err_host, void* work, int64_t work_bytes,
-                   int32_t* info, hipStream_t st_) {
-  SEEMPS_CHECK_ARG(m >= 1 && n >= 1, "svd_split: empty matrix");
-  SEEMPS_CHECK_ARG(mode == 0 || mode == 1, "svd_split: invalid mode");
-  SEEMPS_CHECK_ARG(work_bytes >= svd_split_bytes(m, n), "svd_split: workspace too small");
-  const int64_t r = m < n ? m : n;
-  auto al = [](int64_t x) { return (x + 255) & ~int64_t(255); };
-  char* p = (char*)work;
-  double2* U = (double2*)p;
-  p += al(m * r * 16);
-  double* S = (double*)p;
-  p += al(r * 8);
-  double2* VH = (double2*)p;
-  p += al(r * n * 16);
-  int64_t* Ddev = (int64_t*)p;
-  double* edev = (double*)(p + 8);
-  p += al(64);
-  int off = 0;
-  int st = svd_enqueue(m, n, A, n, U, S, VH, p, work_bytes - (p - (char*)work), st_, &off, false);
-  if (st) return st;
-  if ((st = truncate_enqueue(r, S, method, tolerance, max_bond, Ddev, edev, st_))) return st;
-  if ((st = svd_complete_enqueue(m, n, U, VH, p, Ddev, st_))) return st;
-  char* hp = (char*)pinned_stage(PINNED_BYTES);
-  SEEMPS_CHECK_ARG(hp != nullptr, "pinned host staging could not be allocated");
-  SEEMPS_HIP(hipMemcpyAsync(hp, Ddev, 8, hipMemcpyDeviceToHost, st_));
-  SEEMPS_HIP(hipMemcpyAsync(hp + 8, edev, 8, hipMemcpyDeviceToHost, st_));
-  if ((st = svd_read_ctrl(p, off, info, st_))) return st;  // synchronises
-  int64_t hD = 0;
-  double herr = 0.0;
-  memcpy(&hD, hp, 8);
-  memcpy(&herr, hp + 8, 8);
-  const int64_t D = hD;
-  if (mode == 0) {
-    if ((st = zscale2d_impl(m, D, nullptr, nullptr, U, r, outA, D, st_))) return st;
-    if ((st = zscale2d_impl(D, n, S, nullptr, VH, n, outB, n, st_))) return st;
-  } else {
-    if ((st = zscale2d_impl(m, D, nullptr, S, U, r, outA, D, st_))) return st;
-    if ((st = zscale2d_impl(D, n, nullptr, nullptr, VH, n, outB, n, st_))) return st;
-  }
-  if (s_out) SEEMPS_HIP(hipMemcpyAsync(s_out, S, r * 8, hipMemcpyDeviceToDevice, st_));
-  *D_host = D;
-  *err_host = herr;
-  return SEEMPS_OK;
-}
-
-}  // namespace seemps
-
-extern "C" int64_t seemps_svd_split_workspace(int64_t m, int64_t n) {
-  return seemps::svd_split_bytes(m, n);
-}
-
-extern "C" int seemps_svd_split(int64_t m, int64_t n, const void* A, int mode, int method,
-                                double tolerance, int64_t max_bond, void* outA, void* outB,
-                                double* s_out, int64_t* D_host, double* err_host, void* work,
-                                int64_t work_bytes, int32_t* info, void* stream) {
-  return seemps::svd_split_impl(m, n, (const double2*)A, mode, method, tolerance, max_bond,
-                                (double2*)outA, (double2*)outB, s_out, D_host, err_host, work,
-                                work_bytes, info, (hipStream_t)stream);
 }
