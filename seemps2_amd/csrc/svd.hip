@@ -230,16 +230,49 @@ __global__ void load_y(SvdShape s, SvdWork w) {
   }
 }
 
-// Bounded grid barrier.  Returns false if the barrier was aborted.
-__device__ bool grid_barrier(Ctrl* ctrl, unsigned int target, int* s_flag) {
+// ---- data that workgroups hand to one another --------------------------------
+//
+// W, V and the partial Gram matrices are read and written past the caches that
+// are not coherent between the XCDs (sc1: agent scope), so a reader needs no
+// cache invalidation, which would also drop what the other workgroups of its
+// XCD hold.  A writer waits for its stores in every wavefront (vmcnt), then
+// releases and sets the counter.  128 workgroups handing 64 KB (8 KB) to one
+// another: 6.7 (3.3) us, against 11.1 (6.7) with plain accesses and an acquire.
+constexpr int SC1 = 16;  // cache policy bit of the raw buffer operations
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t shared_rsrc(const double2* base, int elems) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, elems * 16, 0x00027000);
+}
+// Element e of the resource (zero past its end).
+__device__ __forceinline__ double2 shared_load(__amdgpu_buffer_rsrc_t r, int e) {
+  const auto w = __builtin_amdgcn_raw_buffer_load_b128(r, e * 16, 0, SC1);
+  return make_double2(__hiloint2double((int)w[1], (int)w[0]), __hiloint2double((int)w[3], (int)w[2]));
+}
+// (dropped past its end)
+__device__ __forceinline__ void shared_store(__amdgpu_buffer_rsrc_t r, int e, double2 v) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  const u4 w = {(unsigned)__double2loint(v.x), (unsigned)__double2hiint(v.x),
+                (unsigned)__double2loint(v.y), (unsigned)__double2hiint(v.y)};
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, e * 16, 0, SC1);
+}
+// This workgroup's stores are done and released: called by every thread, then
+// thread 0 may set a counter.
+__device__ __forceinline__ void publish() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+}
+
+// Bounded wait (thread 0 polls, the block follows) until every counter has
+// reached target.  Returns false if the wait was aborted.
+__device__ bool wait_counters(Ctrl* ctrl, const unsigned int* c0, const unsigned int* c1,
+                              unsigned int target, int* s_flag) {
   __syncthreads();
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // publish, then arrive
-    atomicAdd(&ctrl->barrier, 1u);
     unsigned long long spins = 0;
     int ok = 1;
-    while (__hip_atomic_load(&ctrl->barrier, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-           target) {
+    while (__hip_atomic_load(c0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target ||
+           (c1 && __hip_atomic_load(c1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)) {
       if (__hip_atomic_load(&ctrl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
         ok = 0;
         break;
@@ -251,11 +284,28 @@ __device__ bool grid_barrier(Ctrl* ctrl, unsigned int target, int* s_flag) {
       }
       __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // see every arrival's stores
     *s_flag = ok;
   }
+  // the loads that follow must stay behind the counter's
+  asm volatile("" ::: "memory");
   __syncthreads();
   return *s_flag != 0;
+}
+
+// Bounded grid barrier.  Returns false if the barrier was aborted.
+__device__ bool grid_barrier(Ctrl* ctrl, unsigned int target, int* s_flag) {
+  publish();
+  if (threadIdx.x == 0) atomicAdd(&ctrl->barrier, 1u);
+  return wait_counters(ctrl, &ctrl->barrier, nullptr, target, s_flag);
+}
+
+__device__ void signal_add(unsigned int* c) {
+  publish();
+  if (threadIdx.x == 0) atomicAdd(c, 1u);
+}
+__device__ void signal_set(unsigned int* c, unsigned int v) {
+  publish();
+  if (threadIdx.x == 0) __hip_atomic_store(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Block indices of pair p in round k of the circle schedule over nb blocks.
@@ -389,6 +439,16 @@ __device__ __forceinline__ double2 rscale(double f, double2 x) {
   return make_double2(f * x.x, f * x.y);
 }
 
+// One row of a pair's columns, rotated by the Rot at doubles N .. N + 3 of rd.
+template <int N>
+__device__ __forceinline__ void rotate_columns(double2& x, double2& y, double rd) {
+  const double cs = wave::row_bcast<N>(rd);
+  const double2 sp = make_double2(wave::row_bcast<N + 2>(rd), wave::row_bcast<N + 3>(rd));
+  const double2 x0 = x;
+  x = cfma(make_double2(-sp.x, sp.y), y, rscale(cs, x0));
+  y = cfma(sp, x0, rscale(cs, y));
+}
+
 // Level H on L.G and the tiles, on every wavefront of the workgroup; rec
 // receives its H x NP rotations.  Ends with a barrier.
 template <int H>
@@ -402,7 +462,7 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
     double2 ac = L.G[a * GP + c], ad = L.G[a * GP + d];
     double2 bc = L.G[b * GP + c], bd = L.G[b * GP + d];
     double gbb = bd.x;
-#pragma unroll 2
+#pragma unroll 4
     for (int k = 0; k < H; ++k) {
       Rot* rot = rec + k * NP;
       const Rot own = pair_rotation(ac.x, gbb, ad, tol2, tiny2);
@@ -448,20 +508,16 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
       xa[i] = tile[a * TP + lane];
       xb[i] = tile[b * TP + lane];
     }
-#pragma unroll 2
+#pragma unroll 4
     for (int k = 0; k < H; ++k) {
       __syncthreads();
-      // the four rotations (16 doubles) in the lanes, broadcast from there
+      // the four rotations (16 doubles) in the lanes of each row, broadcast from there
       const double rd = ((const double*)(rec + k * NP + 4 * w))[lane & 15];
       if (H >= 8 && k > 0) xb[3] = L.xch[k & 1][which][wn][lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double cs = wave::bcast(rd, 4 * i);
-        const double2 sp = make_double2(wave::bcast(rd, 4 * i + 2), wave::bcast(rd, 4 * i + 3));
-        const double2 x = xa[i], y = xb[i];
-        xa[i] = cfma(make_double2(-sp.x, sp.y), y, rscale(cs, x));
-        xb[i] = cfma(sp, x, rscale(cs, y));
-      }
+      rotate_columns<0>(xa[0], xb[0], rd);
+      rotate_columns<4>(xa[1], xb[1], rd);
+      rotate_columns<8>(xa[2], xb[2], rd);
+      rotate_columns<12>(xa[3], xb[3], rd);
       if (k + 1 < H) {
         const double2 x = xb[0];
         if (H == 2) {
@@ -521,20 +577,21 @@ __device__ int inner_rounds(PairLds& L, double tol, double tiny2, int sweeps, bo
   return n;
 }
 
-// Rows [rb, rb + nr) of the pair's columns of M into the tile (zeros below).
+// Rows [rb, rb + nr) of the pair's columns of M into the tile (zeros below), a
+// column a wavefront.
 __device__ __forceinline__ void load_tile(const double2* __restrict__ M, int64_t ld, int64_t bi,
                                           int64_t bj, int64_t rb, int nr, double2* tile) {
-  for (int e = threadIdx.x; e < PW * RT; e += JT) {
-    const int t = e / RT, rr = e % RT;
-    tile[t * TP + rr] = rr < nr ? M[pair_col(bi, bj, t) * ld + rb + rr] : make_double2(0.0, 0.0);
-  }
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int t = wv; t < PW; t += JT / 64)
+    tile[t * TP + lane] = shared_load(shared_rsrc(M + pair_col(bi, bj, t) * ld + rb, nr), lane);
 }
 __device__ __forceinline__ void store_tile(double2* __restrict__ M, int64_t ld, int64_t bi,
                                            int64_t bj, int64_t rb, int nr, const double2* tile) {
-  for (int e = threadIdx.x; e < PW * RT; e += JT) {
-    const int t = e / RT, rr = e % RT;
-    if (rr < nr) M[pair_col(bi, bj, t) * ld + rb + rr] = tile[t * TP + rr];
-  }
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int t = wv; t < PW; t += JT / 64)
+    shared_store(shared_rsrc(M + pair_col(bi, bj, t) * ld + rb, nr), lane, tile[t * TP + lane]);
 }
 
 // A wavefront's share of the Gram matrix's upper 16 x 16 tiles: tile
@@ -572,27 +629,56 @@ __device__ __forceinline__ void gram_store(double2* dst, GramShare q, d4 acc) {
     d[2 * ((q.ti * 16 + lk + 4 * r) * GP + q.tj * 16 + li)] = acc[r];
 }
 
+// Rows of V that chunk r rotates; one tile of them rotates along with W's.
+__device__ __forceinline__ bool v_rows(const SvdShape& s, const SvdWork& w, int64_t r, int64_t* v0,
+                                       int64_t* v1) {
+  const int64_t rcv = ceil_div(s.ncolp, s.R);
+  *v0 = r * rcv;
+  *v1 = min(s.ncolp, *v0 + rcv);
+  return w.V && rcv <= RT && *v0 < *v1;
+}
+
 // Phase A for item (p, r): the Gram matrix of rows [r0, r1) of the pair's
-// columns; the last tile of the rows stays in LDS.  R > 1: into dst
+// columns; the last tile of the rows stays in LDS, with V's.  R > 1: into dst
 // (PW x PW, i <= j only), to be summed over the chunks; else the two halves are
 // left in L.G and L.G2.
-__device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
+__device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r,
                              int64_t r0, int64_t r1, double2* __restrict__ dst, PairLds& L) {
-  const GramShare q = gram_share(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const GramShare q = gram_share(wv);
   d4 c = {0.0, 0.0, 0.0, 0.0};
+  int64_t v0, v1;
+  const bool v_live = v_rows(s, w, r, &v0, &v1);
+  constexpr int PER = (PW + JT / 64 - 1) / (JT / 64);  // columns of a tile per wavefront
+  double2 vt[PER];
   for (int64_t rb = r0; rb == r0 || rb < r1; rb += RT) {
     const int nr = (int)max((int64_t)0, min((int64_t)RT, r1 - rb));
     __syncthreads();
     load_tile(w.W, s.len, bi, bj, rb, nr, L.tile[0]);
+    if (rb == r0 && v_live) {
+      // V's tile is on its way while the Gram matrix is formed
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int t = min(wv + i * (JT / 64), PW - 1);
+        vt[i] = shared_load(
+            shared_rsrc(w.V + pair_col(bi, bj, t) * s.ncolp + v0, (int)(v1 - v0)), lane);
+      }
+    }
     __syncthreads();
     gram_accumulate(L.tile[0], nr, q, &c);
+  }
+  if (v_live) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (wv + i * (JT / 64) < PW) L.tile[1][(wv + i * (JT / 64)) * TP + lane] = vt[i];
   }
   gram_store(q.half ? L.G2 : L.G, q, c);
   __syncthreads();
   if (s.R == 1) return;
+  const auto out = shared_rsrc(dst, PW * PW);
   for (int e = threadIdx.x; e < PW * PW; e += JT) {
     const int i = e / PW, j = e % PW;
-    if (i <= j) dst[e] = cadd(L.G[i * GP + j], L.G2[i * GP + j]);
+    if (i <= j) shared_store(out, e, cadd(L.G[i * GP + j], L.G2[i * GP + j]));
   }
 }
 
@@ -629,15 +715,19 @@ __device__ void replay(double2* __restrict__ M, int64_t ld, int64_t bi, int64_t 
 
 // LDS of item (p, r) as partial_gram left it, in a workgroup that has held
 // other items since.
-__device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r0,
-                       int64_t r1, PairLds& L) {
-  __syncthreads();
+__device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r,
+                       int64_t r0, int64_t r1, PairLds& L) {
   if (s.R == 1) {
-    partial_gram(s, w, bi, bj, r0, r1, nullptr, L);
-  } else if (r0 < r1) {
+    partial_gram(s, w, bi, bj, r, r0, r1, nullptr, L);
+    return;
+  }
+  __syncthreads();
+  if (r0 < r1) {
     const int64_t last = r0 + (r1 - r0 - 1) / RT * RT;
     load_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile[0]);
   }
+  int64_t v0, v1;
+  if (v_rows(s, w, r, &v0, &v1)) load_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
 }
 
 // Phases B + C for item (p, r): G = sum of the R partials at src (R > 1), the
@@ -650,7 +740,7 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
                             long long* t0) {
   const int tid = threadIdx.x;
   const int64_t rc = ceil_div(s.len, s.R);
-  const int64_t rcv = ceil_div(s.ncolp, s.R);
+  const auto parts = shared_rsrc(src, RMAX * PW * PW);
   // Upper triangle; the lower one mirrors it, so G is exactly Hermitian.
   for (int e = tid; e < PW * PW; e += JT) {
     const int i = e / PW, j = e % PW;
@@ -664,7 +754,8 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
         double2 gq[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          gq[q] = (q0 + q < s.R) ? src[(q0 + q) * PW * PW + e] : make_double2(0.0, 0.0);
+          gq[q] = (q0 + q < s.R) ? shared_load(parts, (q0 + q) * PW * PW + e)
+                                 : make_double2(0.0, 0.0);
 #pragma unroll
         for (int q = 0; q < 4; ++q) g = cadd(g, gq[q]);
       }
@@ -698,12 +789,8 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
   }
   // already orthogonal to tolerance: no rotation is applied to this pair
   if (pair_off <= tol) return;
-  const int64_t v0 = r * rcv, v1 = min(s.ncolp, v0 + rcv);
-  const bool v_live = w.V && rcv <= RT && v0 < v1;  // V's rows of this chunk are one tile
-  if (v_live) {
-    load_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
-    __syncthreads();
-  }
+  int64_t v0, v1;
+  const bool v_live = v_rows(s, w, r, &v0, &v1);
   const int n = inner_rounds(L, tol, tiny2, inner_sweeps, cross, inner_top_of(s));
   if (prof) {
     const long long t1 = now_ticks();
@@ -725,53 +812,6 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
     const long long t1 = now_ticks();
     pt[4] += t1 - *t0;
     *t0 = t1;
-  }
-}
-
-// Bounded wait (thread 0 polls, the block follows) until every counter in
-// ctr[0..n) has reached target.  Returns false if the wait was aborted.
-__device__ bool wait_counters(Ctrl* ctrl, const unsigned int* c0, const unsigned int* c1,
-                              unsigned int target, int* s_flag) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long spins = 0;
-    int ok = 1;
-    while (__hip_atomic_load(c0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target ||
-           (c1 && __hip_atomic_load(c1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)) {
-      if (__hip_atomic_load(&ctrl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        ok = 0;
-        break;
-      }
-      if (++spins > SPIN_LIMIT) {
-        atomicExch(&ctrl->abort, 1u);
-        ok = 0;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // see the signallers' stores
-    *s_flag = ok;
-  }
-  __syncthreads();
-  return *s_flag != 0;
-}
-
-// Publish this block's writes, then add 1 to / set a counter.
-// Signals publish this workgroup's stores: the barrier gathers them in thread
-// 0, whose release fence precedes the counter update; a wait that observes the
-// counter acquires them (and its barrier passes them on to its workgroup).
-__device__ void signal_add(unsigned int* c) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    atomicAdd(c, 1u);
-  }
-}
-__device__ void signal_set(unsigned int* c, unsigned int v) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __hip_atomic_store(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -832,7 +872,9 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
   for (; sweep < max_sweeps; ++sweep) {
     // Slot (sweep + 1) % 3 was last read after the grid barrier ending sweep
     // sweep - 2; every workgroup has passed the barrier ending sweep - 1 since.
-    if (blockIdx.x == 0 && tid == 0) w.ctrl->off[(sweep + 1) % 3] = 0ull;
+    if (blockIdx.x == 0 && tid == 0)
+      __hip_atomic_store(&w.ctrl->off[(sweep + 1) % 3], 0ull, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
     unsigned long long* off_slot = &w.ctrl->off[sweep % 3];
     for (int64_t k = 0; k < steps; ++k) {
       const int64_t g = (int64_t)sweep * steps + k;
@@ -856,7 +898,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           pt[5] += t1 - t0;
           t0 = t1;
         }
-        partial_gram(s, w, bi, bj, r * rc, min(s.len, r * rc + rc),
+        partial_gram(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
                      part + (p * RMAX + r) * PW * PW, L);
         if (prof) {
           const long long t1 = now_ticks();
@@ -882,7 +924,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           const int64_t p = it / s.R, r = it % s.R;
           int64_t bi, bj;
           pair_blocks(s.nb, k, p, &bi, &bj);
-          partial_gram(s, w, bi, bj, r * rc, min(s.len, r * rc + rc),
+          partial_gram(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
                        part + (p * RMAX + r) * PW * PW, L);
         }
         if (prof) {
@@ -902,7 +944,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           pair_blocks(s.nb, k, p, &bi, &bj);
           // the chunk's last tile (and, R = 1, its Gram matrix) again: L has
           // held other items since
-          reload(s, w, bi, bj, r * rc, min(s.len, r * rc + rc), L);
+          reload(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc), L);
           pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
                       inner_sweeps, cross, L, prof, pt, &t0);
         }

@@ -51,6 +51,14 @@ __device__ __forceinline__ double bcast(double x, int l) {
                           __builtin_amdgcn_readlane(__double2loint(x), l));
 }
 
+// The value of lane N of each 16-lane row, in every lane of the row (one
+// instruction, where readlane takes two into scalar registers).
+template <int N>
+__device__ __forceinline__ double row_bcast(double x) {
+  return __longlong_as_double(
+      __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(x), 0x150 + N, 0xf, 0xf, true));
+}
+
 // Sum over the wavefront, in every lane.
 __device__ __forceinline__ double sum(double x) {
   x = fold32(x, x);
