@@ -7,16 +7,17 @@
 // quarter fewer MFMAs for the same output; its rounding error is bounded, like
 // 4M's, by a small multiple of u * sum |a||b| (normwise), though the imaginary
 // part alone is not resolved to relative precision when it is much smaller
-// than the real part.  The FP64 32 x 32 tile uses 3M unless
+// than the real part.  The FP64 32 x 32 tile and the direct kernel use 3M unless
 // SEEMPS_GEMM_SCHEME=4m; the 64 x 64 tile (no registers to spare for a third
 // accumulator) and FP32 use 4M.
 //
-// Operand tiles are staged in LDS split into real and imaginary planes,
-// K-major, so each MFMA fragment read is a contiguous run of 16 doubles; the
-// op(.) transposition / conjugation is folded into the global->LDS load (no
-// transposed copies are materialised).
+// Most FP64 products without a batch take zgemm_direct (operands straight into
+// registers, choose_direct); the rest is staged.  Staged operand tiles are kept
+// in LDS split into real and imaginary planes, K-major, so each MFMA fragment
+// read is a contiguous run of 16 doubles; the op(.) transposition / conjugation
+// is folded into the global->LDS load (no transposed copies are materialised).
 //
-// Tiles: 64 x 64 or 32 x 32 outputs per 256-thread workgroup (4 waves of a
+// Staged tiles: 64 x 64 or 32 x 32 outputs per 256-thread workgroup (4 waves of a
 // quarter each), chosen per call to spread the tiles evenly over the CUs;
 // K step 16, next K-tile prefetched into registers while the current one is used.
 //
@@ -313,6 +314,151 @@ __global__ __launch_bounds__(256, tile_occupancy(TM, TN, G3)) void zgemm_kernel(
       }
 }
 
+// One 16 F x 16 F output tile per workgroup, its KS wavefronts each taking a run
+// of the K steps with the operands loaded straight into the MFMA layout (no LDS
+// staging, no barrier in the loop), and summing their partial tiles in LDS in
+// the order of the runs.  FP64 MFMA asks little of the memory path (a 32 x 32
+// step of four k is 768 cycles of the matrix core for 4 KB), so what limits
+// products of few tiles is the chain of staging and barriers that this leaves
+// out: 64^3 5.6 -> 3.1 us (a launch is 2.2), 256 x 400 x 200 15.2 -> 7.0.  Of
+// large ones the loads are the limit of 16 x 16 tiles, the matrix cores that of
+// 32 x 32 (2048 x 2048 x 512 at 75 of a large product's 72 TFLOP/s).
+template <int OPA, int OPB, int F, int KS>
+__global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, int64_t K,
+                                                        double2 alpha,
+                                                        const double2* __restrict__ A, int64_t lda,
+                                                        const double2* __restrict__ B, int64_t ldb,
+                                                        double2 beta, double2* __restrict__ C,
+                                                        int64_t ldc) {
+  constexpr int U = 4, NBUF = 2;  // blocks of U K steps (of 4), one loaded ahead
+  constexpr bool AT = OPA == SEEMPS_OP_T || OPA == SEEMPS_OP_H;
+  constexpr bool BT = OPB == SEEMPS_OP_T || OPB == SEEMPS_OP_H;
+  constexpr double SGA = (OPA == SEEMPS_OP_C || OPA == SEEMPS_OP_H) ? -1.0 : 1.0;
+  constexpr double SGB = (OPB == SEEMPS_OP_C || OPB == SEEMPS_OP_H) ? -1.0 : 1.0;
+  extern __shared__ double2 part[];  // KS x (4 F F items) x 64 lanes
+  const int64_t tiles_n = ceil_div(N, 16 * F);
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t m0 = (tile / tiles_n) * (16 * F), n0 = (tile % tiles_n) * (16 * F);
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // rows and columns past the edge are read from the last one and not stored
+  const double2 *pa[F], *pb[F];
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    const int64_t m = min(m0 + 16 * f + li, M - 1), n = min(n0 + 16 * f + li, N - 1);
+    pa[f] = AT ? A + m : A + m * lda;
+    pb[f] = BT ? B + n * ldb : B + n;
+  }
+  const int64_t stepA = AT ? lda : 1, stepB = BT ? 1 : ldb;
+  d4 t1[F][F], t2[F][F], t3[F][F];
+#pragma unroll
+  for (int a = 0; a < F; ++a)
+#pragma unroll
+    for (int b = 0; b < F; ++b) t1[a][b] = t2[a][b] = t3[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+  auto load = [&](int64_t k, double2 (&x)[F], double2 (&y)[F]) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      x[f] = pa[f][k * stepA];
+      y[f] = pb[f][k * stepB];
+    }
+  };
+  auto mac = [&](const double2 (&x)[F], const double2 (&y)[F]) {
+#pragma unroll
+    for (int a = 0; a < F; ++a)
+#pragma unroll
+      for (int b = 0; b < F; ++b) {
+        t1[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].x, y[b].x, t1[a][b], 0, 0, 0);
+        t2[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].y, y[b].y, t2[a][b], 0, 0, 0);
+        t3[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].x + SGA * x[a].y,
+                                                        y[b].x + SGB * y[b].y, t3[a][b], 0, 0, 0);
+      }
+  };
+  const int64_t steps = ceil_div(K, (int64_t)4), per = ceil_div(steps, (int64_t)KS);
+  const int64_t s0 = min(wv * per, steps), s1 = min(s0 + per, steps);
+  const int64_t full = min(s1, K / 4);  // steps [s0, full) need no bounds test
+  const int64_t nb = full > s0 ? (full - s0) / U : 0;
+  double2 x[NBUF][U][F], y[NBUF][U][F];
+  auto load_block = [&](int64_t b, double2 (&xx)[U][F], double2 (&yy)[U][F]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load((s0 + b * U + u) * 4 + lk, xx[u], yy[u]);
+  };
+  if (nb > 0) {
+#pragma unroll
+    for (int i = 0; i < NBUF - 1; ++i)
+      if (i < nb) load_block(i, x[i], y[i]);
+  }
+  for (int64_t b = 0; b < nb; b += NBUF) {
+#pragma unroll
+    for (int i = 0; i < NBUF; ++i) {
+      if (b + i < nb) {
+        constexpr int AHEAD = NBUF - 1;
+        if (F > 1)
+          load_block(min(b + i + AHEAD, nb - 1), x[(i + AHEAD) % NBUF], y[(i + AHEAD) % NBUF]);
+        else if (b + i + AHEAD < nb)
+          load_block(b + i + AHEAD, x[(i + AHEAD) % NBUF], y[(i + AHEAD) % NBUF]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mac(x[i][u], y[i][u]);
+      }
+    }
+  }
+  // the last steps together: past the run or past K they are read in bounds
+  // and count as zero
+  if (s0 + nb * U < s1) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t s = s0 + nb * U + u;
+      load(min(s * 4 + lk, K - 1), x[0][u], y[0][u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t s = s0 + nb * U + u;
+      if (s >= s1) break;
+      if (s * 4 + lk >= K) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) x[0][u][f] = y[0][u][f] = make_double2(0.0, 0.0);
+      }
+      mac(x[0][u], y[0][u]);
+    }
+  }
+  const bool use_beta = (beta.x != 0.0 || beta.y != 0.0);
+  auto put = [&](int a, int b, int r, double2 acc) {
+    const int64_t m = m0 + 16 * a + lk + 4 * r, n = n0 + 16 * b + li;
+    if (m < M && n < N) {
+      double2 out = cmul(alpha, acc);
+      if (use_beta) out = cfma(beta, C[m * ldc + n], out);
+      C[m * ldc + n] = out;
+    }
+  };
+#pragma unroll
+  for (int a = 0; a < F; ++a)
+#pragma unroll
+    for (int b = 0; b < F; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double u = t1[a][b][r], v = SGA * SGB * t2[a][b][r];
+        const double2 acc = make_double2(u - v, (t3[a][b][r] - u) - v);
+        if (KS == 1)
+          put(a, b, r, acc);
+        else
+          part[(wv * (4 * F * F) + (a * F + b) * 4 + r) * 64 + lane] = acc;
+      }
+  if (KS == 1) return;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < F; ++a)
+#pragma unroll
+    for (int b = 0; b < F; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int item = (a * F + b) * 4 + r;
+        if (item % KS != wv && !(KS > 4 * F * F && wv == item)) continue;
+        double2 acc = part[item * 64 + lane];
+#pragma unroll
+        for (int q = 1; q < KS; ++q) acc = cadd(acc, part[(q * (4 * F * F) + item) * 64 + lane]);
+        put(a, b, r, acc);
+      }
+}
+
 // Tile shape for an M x N output in `batch` slices on `num_cu` CUs.  The
 // 64 x 64 tile (three workgroups per CU) is the faster one per output element
 // once every CU holds four or more of them; below that the 32 x 32 tile (five
@@ -344,6 +490,66 @@ bool gemm_scheme_3m() {
     return !(e && !strcmp(e, "4m"));
   }();
   return g3;
+}
+
+// How an FP64 product without a batch runs: the direct kernel with (F, KS), or
+// staged through LDS (F = 0).  t counts 32 x 32 tiles; a tile of four waves fills
+// one CU, so t / 256 CUs says how evenly the work divides.  Times in us, staged
+// (with split-K where it applied) against 1,4 / 2,4 / 2,1:
+//   M N K (t)                staged    1,4    2,4    2,1
+//   64 64 64 (4)                5.6    3.1    5.4    9.4
+//   256 400 200 (104)          15.2    7.0   11.2   23.4
+//   640 512 512 (320)          32.7   26.6   34.5   56.6
+//   1280 512 256 (640)         36.9   30.0   28.4   36.1
+//   512 512 512 (256)          27.8   22.3   22.2   54.7
+//   1024 1024 1024 (1024)     142.8  176.0  121.4  123.0
+//   2048 2048 512 (4096)      280.1  330.6  233.6  228.3
+//   1500 1100 300 (1645)       74.8   78.9   71.0   69.9
+//   1024 1024 64 (1024)        13.4   16.4   14.8   14.8
+//   1280 1024 256 (1280)       49.3   58.7   51.1   58.7
+// Few tiles: 16 x 16 ones for four times the waves.  From a tile for each CU:
+// 32 x 32 ones, which ask half the loads, where whole rounds of the CUs come out
+// at least four fifths full, and one wave a tile once every SIMD has its own.
+// Many tiles that leave a round part empty, and short K, stay staged.  So do few
+// tiles with both operands contiguous along a long K: a load of theirs touches
+// sixteen rows, and splitting K over more CUs wins (64 x 64 x 1024 NT 12.4 against
+// 16.7, 64 x 2048 x 2048 NT 46.9 / 59.1; 1024 x 256 x 1280 NT alone 54.7 / 53.2
+// but 2.5 us slower within a matvec; shorter K win, 512 x 128 x 640 NT 15.5 /
+// 11.7, as NN and HN at any K, 64 x 64 x 4096 HN 33.8 / 32.7).
+struct Direct {
+  int F, KS;
+};
+
+// op(A)'s rows and op(B)'s columns both contiguous along K
+bool rows_in_k(int opA, int opB) {
+  return (opA == SEEMPS_OP_N || opA == SEEMPS_OP_C) && (opB == SEEMPS_OP_T || opB == SEEMPS_OP_H);
+}
+
+Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_cu) {
+  static const bool off = getenv("SEEMPS_GEMM_TILE") != nullptr;  // the knob names staged tiles
+  if (off || !gemm_scheme_3m()) return {0, 0};
+  const int64_t cu = num_cu > 0 ? num_cu : 256, simd = 4 * cu;
+  const int64_t t = ceil_div(M, 32) * ceil_div(N, 32);
+  auto full = [&](int64_t units) { return 5 * t >= 4 * units * ceil_div(t, units); };
+  if (t >= simd) return full(simd) && t * K >= 128 * simd ? Direct{2, 1} : Direct{0, 0};
+  if (rows_in_k(opA, opB) && K >= 1024) return {0, 0};
+  return t >= cu && full(cu) ? Direct{2, 4} : Direct{1, 4};
+}
+
+template <int OPA, int OPB>
+void launch_direct(Direct d, hipStream_t s, int64_t M, int64_t N, int64_t K, double2 alpha,
+                   const double2* A, int64_t lda, const double2* B, int64_t ldb, double2 beta,
+                   double2* C, int64_t ldc) {
+#define SEEMPS_DIRECT_CASE(F_, KS_)                                                             \
+  if (d.F == F_ && d.KS == KS_)                                                                 \
+    hipLaunchKernelGGL((zgemm_direct<OPA, OPB, F_, KS_>),                                       \
+                       dim3((unsigned)(ceil_div(M, 16 * F_) * ceil_div(N, 16 * F_))),           \
+                       dim3(64 * KS_), KS_ == 1 ? 0 : KS_ * 4 * F_ * F_ * 64 * 16, s, M, N, K,  \
+                       alpha, A, lda, B, ldb, beta, C, ldc);
+  SEEMPS_DIRECT_CASE(1, 4)
+  SEEMPS_DIRECT_CASE(2, 4)
+  SEEMPS_DIRECT_CASE(2, 1)
+#undef SEEMPS_DIRECT_CASE
 }
 
 template <int OPA, int OPB>
@@ -393,6 +599,9 @@ int dispatch(int prec, int opA, int opB, int64_t batch, hipStream_t stream, int6
   const int ist = device_info(&info);
   if (ist) return ist;
   const int tile = choose_tile(M, N, batch, info.num_cu);
+  const Direct direct = batch == 1 && prec == SEEMPS_PREC_FP64
+                            ? choose_direct(opA, opB, M, N, K, info.num_cu)
+                            : Direct{0, 0};
   // the tile index runs along grid.x (at most 2^31 - 1 workgroups)
   SEEMPS_CHECK_ARG(ceil_div(M, 32) * ceil_div(N, 32) < (int64_t)INT32_MAX,
                    "zgemm: output too large");
@@ -400,6 +609,10 @@ int dispatch(int prec, int opA, int opB, int64_t batch, hipStream_t stream, int6
                     flops);
 #define SEEMPS_GEMM_CASE(x, y)                                                              \
   if (opA == x && opB == y) {                                                               \
+    if (direct.F) {                                                                         \
+      launch_direct<x, y>(direct, stream, M, N, K, alpha, a, lda, b, ldb, beta, c, ldc);    \
+      return check_launch("zgemm");                                                         \
+    }                                                                                       \
     launch<x, y>(prec, tile, batch, stream, M, N, K, Klast, alpha, a, lda, sA, b, ldb, sB,   \
                  beta, c, ldc, sC);                                                         \
     return check_launch("zgemm");                                                           \
@@ -442,7 +655,11 @@ int64_t splitk_workspace(int64_t M, int64_t N, int64_t K) {
 int zgemm_ws(int opA, int opB, int64_t M, int64_t N, int64_t K, double2 alpha, const void* A,
              int64_t lda, const void* B, int64_t ldb, double2 beta, void* C, int64_t ldc,
              double2* ws, int64_t ws_elems, hipStream_t stream, int prec) {
-  const int64_t z = splitk_slices(M, N, K);
+  DeviceInfo info;
+  const int ist = device_info(&info);
+  if (ist) return ist;
+  const bool direct = prec == SEEMPS_PREC_FP64 && choose_direct(opA, opB, M, N, K, info.num_cu).F;
+  const int64_t z = direct ? 1 : splitk_slices(M, N, K);
   if (z <= 1 || ws == nullptr || ws_elems < z * M * N)
     return zgemm(opA, opB, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 1, stream,
                  prec);

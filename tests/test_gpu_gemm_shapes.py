@@ -1,0 +1,50 @@
+"""Edges of the direct GEMM kernel: tiles of 16 and 32, K remainders of every
+wavefront's run, leading dimensions beyond the rows, all sixteen operand forms.
+
+Gaussian integers: every partial sum is an exact integer in any order, so the
+result equals the exact one bit for bit.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+OPS = {0: lambda x: x, 1: lambda x: x.T, 2: lambda x: x.conj().T, 3: lambda x: x.conj()}
+
+
+# one tile and its edges; four waves' runs with none, one or part of a step; a
+# tile for each CU (512 x 512), for each SIMD (1024 x 1023), and neither (320 tiles)
+@pytest.mark.parametrize("M,N,K_", [(1, 1, 1), (16, 16, 3), (17, 33, 5), (31, 15, 67), (2, 40, 64),
+                                    (49, 16, 129), (512, 511, 71), (630, 509, 18),
+                                    (1024, 1023, 129)])
+def test_direct_gemm_edges(M, N, K_):
+    from seemps2_amd import kernels as K
+    from seemps2_amd._lib import check, lib
+
+    rng = np.random.default_rng(M * 7 + N)
+
+    def ints(r, c):
+        return rng.integers(-3, 4, (r, c)) + 1j * rng.integers(-3, 4, (r, c))
+
+    def padded(x, extra):  # rows followed by NaN that nothing may read into a result
+        p = np.full((x.shape[0], x.shape[1] + extra), np.nan + 1j * np.nan)
+        p[:, :x.shape[1]] = x
+        return K.as_dev(p)
+
+    alpha, beta = 1 + 2j, 2 - 1j
+    for opA in range(4):
+        for opB in range(4):
+            A = ints(*((K_, M) if opA in (1, 2) else (M, K_)))
+            B = ints(*((N, K_) if opB in (1, 2) else (K_, N)))
+            C = ints(M, N)
+            ref = alpha * (OPS[opA](A) @ OPS[opB](B)) + beta * C
+            a, b, c = padded(A, 3), padded(B, 1), padded(C, 2)
+            check(lib.seemps_zgemm(opA, opB, M, N, K_, alpha.real, alpha.imag, a.data_ptr(),
+                                   a.shape[1], 0, b.data_ptr(), b.shape[1], 0, beta.real,
+                                   beta.imag, c.data_ptr(), c.shape[1], 0, 1,
+                                   torch.cuda.current_stream().cuda_stream))
+            out = K.to_numpy(c)
+            assert np.array_equal(out[:, :N], ref), (opA, opB)
+            assert np.isnan(out[:, N:]).all()
