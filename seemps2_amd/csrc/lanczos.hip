@@ -6,10 +6,10 @@
 // 187-237) and the scipy eigsh / ARPACK call of _diagonalize_two_site
 // (src/seemps/optimization/dmrg.py:15-23).
 #include <cmath>
-#include <cstddef>
-#include <vector>
 
 #include "common.h"
+#include "jacobi_inner.h"
+#include "wave.h"
 
 namespace seemps {
 namespace {
@@ -54,449 +54,443 @@ __global__ void permute_kernel(int64_t total, PermDesc p, const double2* __restr
 }
 
 
-// x[i] = sum_{j<k} V[j*ldv + i] * y[j]  (y real)
-__global__ void combine_kernel(int64_t n, int k, const double2* __restrict__ V, int64_t ldv,
-                               const double* __restrict__ y, double2* __restrict__ x) {
-  __shared__ double ys[64];
-  if (threadIdx.x < k) ys[threadIdx.x] = y[threadIdx.x];
-  __syncthreads();
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int j = 0; j < k; ++j) {
-      const double2 v = V[j * ldv + i];
-      acc.x += v.x * ys[j];
-      acc.y += v.y * ys[j];
-    }
-    x[i] = acc;
-  }
-}
-
 // Scalars of one Lanczos cycle kept on the device.
 struct LzScalars {
   double alpha[64];
   double beta[64];
   double y[64];
-  double2 h[64];
-  double2 h2[64];
-  double2 nrm;      // <w, w>
-  double theta;
-  double resid;
-  double scale;     // running max |alpha| + |beta| (breakdown reference)
+  double2 h;        // first-pass coefficient of the last basis vector
   int kd;           // effective Krylov dimension of the cycle
   int broken;       // breakdown seen in this cycle
-  double scl[64];   // scale after step j
+  double scl[64];   // running max |alpha| + |beta| after step j (breakdown reference)
   int brk[64];      // breakdown seen up to step j
 };
 
-constexpr int LZ_NV = 64;  // stride of the per-block partial dot products
-
-// Block-wide sum of one complex value per thread (256 threads), result valid
-// in every thread.
-__device__ double2 lz_block_sum(double2 v, double2* red) {
-  for (int off = 32; off > 0; off >>= 1) {
-    v.x += __shfl_down(v.x, off, 64);
-    v.y += __shfl_down(v.y, off, 64);
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  double2 t = make_double2(0.0, 0.0);
-  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t = cadd(t, red[q]);
-  return t;
-}
-
-// Classical Gram-Schmidt of w against V[0..k) with the DGKS second pass
-// (applied only when the first pass removed more than half of |w|^2), in three
-// launches over lz_blocks(n) chunks.  Each block keeps the k entries V[j][i] of
-// its elements in registers (k <= LZ_KREG), so every launch reads V once.
-// Partial sums are reduced redundantly by every block in a fixed order, which
-// keeps the result deterministic without an extra launch.
+// Bound of the basis size (register arrays of one entry per basis vector).
 constexpr int LZ_KREG = 24;
+constexpr int LZ_THREADS = 256;
 
-// Number of chunks of the orthogonalisation launches.
+// Blocks of the orthogonalisation launches: an element per thread up to one
+// block per CU, so that a short vector is spread over as many CUs as it can use.
 inline int lz_blocks(int64_t n) {
-  int64_t b = ceil_div(n, 1024);
+  int64_t b = ceil_div(n, (int64_t)LZ_THREADS);
   if (b > 256) b = 256;
   if (b < 1) b = 1;
   return (int)b;
 }
 
-// Sum over blocks of per-thread partials (k complex values and one real per
-// thread) into part[blockIdx.x * LZ_NV + j] and pn[blockIdx.x].
-__device__ void lz_store_partials(const double2* acc, int k, double nrm, double2* red,
-                                  double* redn, double2* __restrict__ part,
-                                  double* __restrict__ pn) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// sum_b pn[b], b < nb <= 256, in every lane of a wavefront (fixed order).
+__device__ __forceinline__ double lz_wave_sum(int nb, const double* __restrict__ pn) {
+  const int lane = threadIdx.x & 63;
+  double t[4];
 #pragma unroll
-  for (int j = 0; j < LZ_KREG; ++j) {
-    if (j < k) {
-      double2 v = acc[j];
-      for (int off = 32; off > 0; off >>= 1) {
-        v.x += __shfl_down(v.x, off, 64);
-        v.y += __shfl_down(v.y, off, 64);
-      }
-      if (lane == 0) red[wave * LZ_KREG + j] = v;
-    }
+  for (int q = 0; q < 4; ++q) t[q] = pn[min(lane + 64 * q, nb - 1)];
+  double r = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r += lane + 64 * q < nb ? t[q] : 0.0;
+  return wave::sum(r);
+}
+
+// Per-thread partials (k of the KR complex values, one real) to
+// part[j * nb + block] and pn[block].
+template <int KR>
+__device__ __forceinline__ void lz_store_partials(const double2 (&acc)[KR], int k, double nrm,
+                                                  double2* __restrict__ part,
+                                                  double* __restrict__ pn) {
+  __shared__ double red[LZ_THREADS / 64][2 * KR + 1];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < KR; j += 2) {
+    const double s = wave::row_sum(wave::fold16(wave::fold32(acc[j].x, acc[j].y),
+                                                wave::fold32(acc[j + 1].x, acc[j + 1].y)));
+    // rows 0, 2: value j; rows 1, 3: value j + 1
+    if ((lane & 15) == 0) red[wv][2 * (j + (row & 1)) + (row >> 1)] = s;
   }
-  for (int off = 32; off > 0; off >>= 1) nrm += __shfl_down(nrm, off, 64);
-  if (lane == 0) redn[wave] = nrm;
+  nrm = wave::sum(nrm);
+  if (lane == 0) red[wv][2 * KR] = nrm;
   __syncthreads();
-  const int nw = (int)(blockDim.x >> 6);
-  if ((int)threadIdx.x < k) {
-    double2 t = make_double2(0.0, 0.0);
-    for (int q = 0; q < nw; ++q) t = cadd(t, red[q * LZ_KREG + threadIdx.x]);
-    part[blockIdx.x * LZ_NV + threadIdx.x] = t;
-  }
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int q = 0; q < nw; ++q) t += redn[q];
-    pn[blockIdx.x] = t;
+  const int t = threadIdx.x;
+  if (t < 2 * k || t == 2 * KR) {
+    double v = red[0][t];
+#pragma unroll
+    for (int q = 1; q < LZ_THREADS / 64; ++q) v += red[q][t];
+    if (t < 2 * k)
+      ((double*)part)[2 * ((t >> 1) * (int64_t)gridDim.x + blockIdx.x) + (t & 1)] = v;
+    else
+      pn[blockIdx.x] = v;
   }
 }
 
-// h[j] = sum_b part[b * LZ_NV + j] into LDS, j < k (8 k <= blockDim.x): eight
-// lanes per j each add every eighth partial, then a three-step shuffle tree.
-// The order is fixed, so every block derives the same h.  Called by every
-// thread of the block.
-__device__ void lz_load_coeffs(int k, int nb, const double2* __restrict__ part, double2* hs) {
+// hs[j] = sum_b part[j * nb + b], j < k: eight lanes per j each add every
+// eighth partial, eight loads in flight, then a tree.  Fixed order: every block
+// derives the same hs.  Called by every thread; the caller synchronises.
+__device__ __forceinline__ void lz_load_coeffs(int k, int nb, const double2* __restrict__ part,
+                                               double2* hs) {
   const int j = (int)threadIdx.x >> 3, sub = (int)threadIdx.x & 7;
+  const double2* p = part + (int64_t)min(j, k - 1) * nb;
   double2 acc = make_double2(0.0, 0.0);
-  if (j < k)
-    for (int b = sub; b < nb; b += 8) acc = cadd(acc, part[b * LZ_NV + j]);
-  for (int off = 1; off < 8; off <<= 1) {
-    acc.x += __shfl_xor(acc.x, off, 64);
-    acc.y += __shfl_xor(acc.y, off, 64);
+  for (int b0 = sub; b0 - sub < nb; b0 += 64) {
+    double2 v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = p[min(b0 + 8 * q, nb - 1)];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (b0 + 8 * q < nb) acc = cadd(acc, v[q]);
   }
+#define SEEMPS_LZ_STEP(ctrl)            \
+  acc.x += wave::dpp<ctrl>(acc.x);      \
+  acc.y += wave::dpp<ctrl>(acc.y);
+  SEEMPS_LZ_STEP(0xB1)   // quad_perm 1 0 3 2
+  SEEMPS_LZ_STEP(0x4E)   // quad_perm 2 3 0 1
+  SEEMPS_LZ_STEP(0x141)  // row_half_mirror
+#undef SEEMPS_LZ_STEP
   if (j < k && sub == 0) hs[j] = acc;
 }
 
-// sum_b pn[b], b < nb, by one whole wavefront: lane l adds pn[l], pn[l + 64],
-// ..., then a butterfly, which leaves the same total (same order) in every lane.
-__device__ double lz_wave_sum(int nb, const double* __restrict__ pn) {
-  double t = 0.0;
-  for (int b = (int)threadIdx.x & 63; b < nb; b += 64) t += pn[b];
-  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-  return t;
+// The k entries V[j][i]; those past k repeat the last.
+template <int KR>
+__device__ __forceinline__ void lz_column(int64_t n, int k, int64_t i,
+                                          const double2* __restrict__ V, double2 (&v)[KR]) {
+#pragma unroll
+  for (int j = 0; j < KR; ++j) v[j] = V[min(j, k - 1) * n + i];
 }
 
-// Pass 1: part = chunk sums of conj(V_j) w; pn0 = chunk sums of |w|^2.
-__global__ __launch_bounds__(256) void lz_orth1(int64_t n, int k, const double2* __restrict__ V,
-                                                const double2* __restrict__ w,
-                                                double2* __restrict__ part,
-                                                double* __restrict__ pn0) {
-  __shared__ double2 red[4 * LZ_KREG];
-  __shared__ double redn[4];
-  const int64_t chunk = ceil_div(n, (int64_t)gridDim.x);
-  const int64_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
-  double2 acc[LZ_KREG];
+// Classical Gram-Schmidt of w = H v_{k-1} against V[0..k) with the DGKS second
+// pass (applied only when the first removed more than half of |w|^2), the norm
+// and the scalars, in three launches.  Each is bound by its launch and by one
+// round of loads: with n = 36864 the basis is 0.6 MB a vector and lies in the
+// last-level cache.  So a thread takes one element and asks for all its basis
+// entries at once (KR >= k of them, a multiple of four, in registers; testing
+// j < k load by load serialises them), sums go through DPP, and partials lie so
+// that blocks read them back coalesced.  n = 36864, k <= 20: 38 us a step in
+// four launches of four elements a thread -> LZ_TIME.
+//
+// Pass 1: part = block sums of conj(V_j) w; pn0 = block sums of |w|^2.
+template <int KR>
+__global__ __launch_bounds__(LZ_THREADS) void lz_orth1(int64_t n, int k,
+                                                       const double2* __restrict__ V,
+                                                       const double2* __restrict__ w,
+                                                       double2* __restrict__ part,
+                                                       double* __restrict__ pn0) {
+  double2 acc[KR];
 #pragma unroll
-  for (int j = 0; j < LZ_KREG; ++j) acc[j] = make_double2(0.0, 0.0);
+  for (int j = 0; j < KR; ++j) acc[j] = make_double2(0.0, 0.0);
   double nrm = 0.0;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+  for (int64_t i = blockIdx.x * (int64_t)LZ_THREADS + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * LZ_THREADS) {
+    double2 v[KR];
+    lz_column<KR>(n, k, i, V, v);
     const double2 x = w[i];
     nrm += cabs2(x);
 #pragma unroll
-    for (int j = 0; j < LZ_KREG; ++j)
-      if (j < k) acc[j] = cfmac(V[j * n + i], x, acc[j]);
+    for (int j = 0; j < KR; ++j) acc[j] = cfmac(v[j], x, acc[j]);
   }
-  lz_store_partials(acc, k, nrm, red, redn, part, pn0);
+  lz_store_partials<KR>(acc, k, nrm, part, pn0);
 }
 
-// Pass 2: h = sum of pass-1 partials (block 0 stores it); w -= V h; then the
-// chunk sums of conj(V_j) w (part_out) and |w|^2 (pn1) of the updated w.
-__global__ __launch_bounds__(256) void lz_orth2(int64_t n, int k, const double2* __restrict__ V,
-                                                double2* __restrict__ w,
-                                                const double2* __restrict__ part_in,
-                                                double2* __restrict__ part_out,
-                                                double* __restrict__ pn1,
-                                                double2* __restrict__ h_out) {
+// Pass 2: h = sum of pass-1 partials (h_{k-1} is kept); w -= V h; then the
+// block sums of conj(V_j) w (part_out) and |w|^2 (pn1) of the updated w.
+template <int KR>
+__global__ __launch_bounds__(LZ_THREADS) void lz_orth2(int64_t n, int k,
+                                                       const double2* __restrict__ V,
+                                                       double2* __restrict__ w,
+                                                       const double2* __restrict__ part_in,
+                                                       double2* __restrict__ part_out,
+                                                       double* __restrict__ pn1,
+                                                       LzScalars* __restrict__ s) {
   __shared__ double2 hs[LZ_KREG];
-  __shared__ double2 red[4 * LZ_KREG];
-  __shared__ double redn[4];
+  const int64_t step = (int64_t)gridDim.x * LZ_THREADS;
+  int64_t i = blockIdx.x * (int64_t)LZ_THREADS + threadIdx.x;
+  double2 v[KR], x = w[min(i, n - 1)];
+  lz_column<KR>(n, k, min(i, n - 1), V, v);
+  if (threadIdx.x < LZ_KREG) hs[threadIdx.x] = make_double2(0.0, 0.0);
+  __syncthreads();
   lz_load_coeffs(k, gridDim.x, part_in, hs);
   __syncthreads();
-  if (blockIdx.x == 0 && (int)threadIdx.x < k) h_out[threadIdx.x] = hs[threadIdx.x];
-  const int64_t chunk = ceil_div(n, (int64_t)gridDim.x);
-  const int64_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
-  double2 acc[LZ_KREG];
+  if (blockIdx.x == 0 && threadIdx.x == 0) s->h = hs[k - 1];
+  double2 acc[KR];
 #pragma unroll
-  for (int j = 0; j < LZ_KREG; ++j) acc[j] = make_double2(0.0, 0.0);
+  for (int j = 0; j < KR; ++j) acc[j] = make_double2(0.0, 0.0);
   double nrm = 0.0;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    double2 vr[LZ_KREG];
-    double2 x = w[i];
+  for (; i < n;) {
 #pragma unroll
-    for (int j = 0; j < LZ_KREG; ++j) {
-      if (j < k) {
-        vr[j] = V[j * n + i];
-        const double2 t = cmul(vr[j], hs[j]);
-        x.x -= t.x;
-        x.y -= t.y;
-      }
+    for (int j = 0; j < KR; ++j) {
+      const double2 t = cmul(v[j], hs[j]);
+      x.x -= t.x;
+      x.y -= t.y;
     }
     w[i] = x;
     nrm += cabs2(x);
 #pragma unroll
-    for (int j = 0; j < LZ_KREG; ++j)
-      if (j < k) acc[j] = cfmac(vr[j], x, acc[j]);
+    for (int j = 0; j < KR; ++j) acc[j] = cfmac(v[j], x, acc[j]);
+    i += step;
+    if (i < n) {
+      x = w[i];
+      lz_column<KR>(n, k, i, V, v);
+    }
   }
-  lz_store_partials(acc, k, nrm, red, redn, part_out, pn1);
+  lz_store_partials<KR>(acc, k, nrm, part_out, pn1);
 }
 
-// Pass 3 (DGKS): if |w|^2 after pass 1 is at least half of |w|^2 before it,
-// the first pass was accurate and w is kept (h2 = 0); otherwise w -= V h2 with
-// h2 = the pass-2 coefficients.  pn2 receives the final chunk norms.
-__global__ __launch_bounds__(256) void lz_orth3(int64_t n, int k, const double2* __restrict__ V,
-                                                double2* __restrict__ w,
-                                                const double2* __restrict__ part_in,
-                                                const double* __restrict__ pn0,
-                                                const double* __restrict__ pn1,
-                                                double* __restrict__ pn2,
-                                                double2* __restrict__ h2_out) {
+// Lowest eigenpair of the symmetric tridiagonal tridiag(beta, alpha, beta) of
+// dimension kd < LZ_KREG, by one wavefront; a[] and b[] in LDS (b[kd - 1] may hold
+// anything).  64-way multisection on whether T - x has a negative pivot for
+// theta: ten rounds narrow the Gershgorin interval by 65^10 (about 1e-18 of its
+// width), below the spacing of doubles.  Then inverse iteration for y in every
+// lane alike.
+//
+// Both are chains of kd dependent steps, so what counts is the length of a step.
+// The pivots d_i = a_i - x - b_{i-1}^2 / d_{i-1} are taken as ratios of the
+// leading minors p_i = (a_i - x) p_{i-1} - b_{i-1}^2 p_{i-2} (one dependent FMA, no
+// division; T is scaled by a power of two and the minors rescaled on the way, so
+// they stay in range).  The shift of the inverse iteration lies just below the
+// interval, where T - x is positive definite: its L D L^T needs no pivoting and
+// the iterates no intermediate norm.  All loops run to the constant bound over
+// rows that continue T as decoupled ones of a large diagonal.  At kd = 20 29 us as
+// a kernel of its own, about 5 at the end of the step's last launch.
+__device__ void lz_tridiag(const double* a, const double* b, int kd, double* theta_out,
+                           double (&y)[LZ_KREG]) {
+  const int lane = threadIdx.x & 63;
+  const double al = lane < kd ? a[lane] : 0.0;
+  const double bl = lane < kd - 1 ? fabs(b[lane]) : 0.0;
+  const double bp = lane > 0 && lane < kd ? fabs(b[lane - 1]) : 0.0;
+  double lo = lane < kd ? al - bl - bp : HUGE_VAL, hi = lane < kd ? al + bl + bp : -HUGE_VAL;
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, off, 64));
+    hi = fmax(hi, __shfl_xor(hi, off, 64));
+  }
+  const double top = fmax(fabs(lo), fabs(hi));
+  const double pad = 1e-12 * top + 1e-300;
+  lo -= pad;
+  hi += pad;
+  const int ex = top > 0.0 && top < HUGE_VAL ? ilogb(top) + 1 : 0;  // |T| <= 1 scaled
+  lo = ldexp(lo, -ex);
+  hi = ldexp(hi, -ex);
+  double A[LZ_KREG], B2[LZ_KREG];
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i) {
+    A[i] = i < kd ? ldexp(a[i], -ex) : 4.0;
+    const double t = i < kd - 1 ? ldexp(b[i], -ex) : 0.0;
+    B2[i] = t * t;
+  }
+  for (int round = 0; round < 10; ++round) {
+    const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
+    double p = A[0] - x, q = 1.0;
+    bool neg = p < 0.0;
+#pragma unroll
+    for (int i = 1; i < LZ_KREG; ++i) {
+      const double r = fma(A[i] - x, p, -B2[i - 1] * q);
+      q = p;
+      p = r;
+      neg = neg || p < 0.0;
+      if (i % 4 == 0) {
+        const int e = p != 0.0 ? __builtin_amdgcn_frexp_exp(p) : 0;
+        p = ldexp(p, -e);
+        q = ldexp(q, -e);
+      }
+    }
+    // smallest lane whose point has at least one eigenvalue below it
+    const unsigned long long mask = __ballot(neg);
+    const int l = mask ? __ffsll((long long)mask) - 1 : 64;
+    const double nlo = l == 0 ? lo : lo + (hi - lo) * (double)l / 65.0;
+    hi = l == 64 ? hi : lo + (hi - lo) * (double)(l + 1) / 65.0;
+    lo = nlo;
+  }
+  *theta_out = ldexp(0.5 * (lo + hi), ex);
+  // T - x = L D L^T, x below every eigenvalue by a rounding or two
+  const double x = lo - 4.440892098500626e-16;
+  double rd[LZ_KREG], l[LZ_KREG];
+  double d = A[0] - x;
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i) {
+    rd[i] = jac::rcp_nr(fmax(d, 2.220446049250313e-16));
+    const double t = i < kd - 1 ? ldexp(b[i], -ex) : 0.0;
+    l[i] = t * rd[i];
+    if (i + 1 < LZ_KREG) d = fma(-t, l[i], A[i + 1] - x);
+  }
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i) y[i] = i < kd ? 1.0 : 0.0;
+  for (int it = 0; it < 4; ++it) {
+#pragma unroll
+    for (int i = 1; i < LZ_KREG; ++i) y[i] = fma(-l[i - 1], y[i - 1], y[i]);
+#pragma unroll
+    for (int i = 0; i < LZ_KREG; ++i) y[i] *= rd[i];
+#pragma unroll
+    for (int i = LZ_KREG - 2; i >= 0; --i) y[i] = fma(-l[i], y[i + 1], y[i]);
+  }
+  // unit norm, largest component positive
+  double big = 0.0;
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i)
+    if (fabs(y[i]) > fabs(big)) big = y[i];
+  const double inv = 1.0 / big;
+  double nn = 0.0;
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i) {
+    y[i] *= inv;
+    nn = fma(y[i], y[i], nn);
+  }
+  const double sc = 1.0 / sqrt(nn);
+#pragma unroll
+  for (int i = 0; i < LZ_KREG; ++i) y[i] *= sc;
+}
+
+// Pass 3 and the end of step j = k - 1.  DGKS: if |w|^2 after pass 1 is at least
+// half of |w|^2 before it, the first pass was accurate and w is kept (h2 = 0);
+// otherwise w -= V h2 with h2 = the pass-2 coefficients, and |w|^2 falls by
+// |h2|^2 (V is orthonormal and h2 the projections on it; where that cancels, w is
+// the rounding of H v and far below the breakdown bound either way).  Then
+// beta_j = |w|, alpha_j = Re(h_j + h2_j), the breakdown test and
+// v_{j+1} = w / beta_j (0 after a breakdown).  Block 0 records the scalars and,
+// with `ritz`, the lowest Ritz pair of the k vectors: y for the combination,
+// theta and the residual beta_j |y_j| to the host's `out`.
+template <int KR>
+__global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
+                                                       const double2* __restrict__ V,
+                                                       double2* __restrict__ w,
+                                                       const double2* __restrict__ part_in,
+                                                       const double* __restrict__ pn0,
+                                                       const double* __restrict__ pn1,
+                                                       LzScalars* __restrict__ s, int ritz,
+                                                       double* __restrict__ out) {
   __shared__ double2 hs[LZ_KREG];
-  __shared__ double s_nrm[2];
-  __shared__ double2 red[4];
-  const int nb = gridDim.x;
-  if (threadIdx.x < 64) {
-    const double t = lz_wave_sum(nb, pn0);
-    if (threadIdx.x == 0) s_nrm[0] = t;
-  } else if (threadIdx.x < 128) {
-    const double t = lz_wave_sum(nb, pn1);
-    if (threadIdx.x == 64) s_nrm[1] = t;
-  }
-  lz_load_coeffs(k, nb, part_in, hs);
+  __shared__ double as[LZ_KREG], bs[LZ_KREG];
+  const int nb = gridDim.x, j = k - 1;
+  const int64_t step = (int64_t)gridDim.x * LZ_THREADS;
+  int64_t i = blockIdx.x * (int64_t)LZ_THREADS + threadIdx.x;
+  double2 v[KR], x = w[min(i, n - 1)];
+  lz_column<KR>(n, k, min(i, n - 1), V, v);
+  const double h = s->h.x;
+  const double prev = j > 0 ? s->beta[j - 1] : 0.0, scale_prev = j > 0 ? s->scl[j - 1] : 0.0;
+  const int brk_prev = j > 0 ? s->brk[j - 1] : 0;
+  const int kd_prev = s->kd;
+  const double n0 = lz_wave_sum(nb, pn0), n1 = lz_wave_sum(nb, pn1);
+  if (threadIdx.x < LZ_KREG) hs[threadIdx.x] = make_double2(0.0, 0.0);
   __syncthreads();
-  const bool second = !(s_nrm[1] >= 0.5 * s_nrm[0]);
-  if (blockIdx.x == 0 && (int)threadIdx.x < k)
-    h2_out[threadIdx.x] = second ? hs[threadIdx.x] : make_double2(0.0, 0.0);
-  if (!second) {
-    if (threadIdx.x == 0) pn2[blockIdx.x] = pn1[blockIdx.x];
-    return;
-  }
-  const int64_t chunk = ceil_div(n, (int64_t)gridDim.x);
-  const int64_t lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
-  double nrm = 0.0;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    double2 x = w[i];
+  const bool second = !(n1 >= 0.5 * n0);
+  if (second) lz_load_coeffs(k, nb, part_in, hs);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const double h2 = wave::sum(lane < k ? cabs2(hs[lane]) : 0.0);
+  const double a = h + hs[j].x;
+  const double beta = sqrt(fmax(n1 - h2, 0.0));
+  const double ref = fmax(scale_prev, fabs(a) + prev);
+  const int brk = brk_prev || (beta <= 1e-12 * ref);
+  const double inv = brk ? 0.0 : 1.0 / beta;
+  for (; i < n;) {
+    if (second) {
 #pragma unroll
-    for (int j = 0; j < LZ_KREG; ++j) {
-      if (j < k) {
-        const double2 t = cmul(V[j * n + i], hs[j]);
+      for (int q = 0; q < KR; ++q) {
+        const double2 t = cmul(v[q], hs[q]);
         x.x -= t.x;
         x.y -= t.y;
       }
     }
-    w[i] = x;
-    nrm += cabs2(x);
-  }
-  const double2 t = lz_block_sum(make_double2(nrm, 0.0), red);
-  if (threadIdx.x == 0) pn2[blockIdx.x] = t.x;
-}
-
-// Step j done: beta_j = ||w|| (from the partial norms, in every block),
-// alpha_j = Re(h_j + h2_j), breakdown test, v_{j+1} = w / beta_j (0 after a
-// breakdown).  Block 0 records the scalars.
-__global__ __launch_bounds__(256) void lz_finish(int64_t n, int nparts, int j,
-                                                 const double* __restrict__ pnorm,
-                                                 LzScalars* __restrict__ s, double2* __restrict__ w) {
-  __shared__ double s_b;
-  __shared__ int s_brk;
-  const double nrm2 = (threadIdx.x < 64) ? lz_wave_sum(nparts, pnorm) : 0.0;
-  if (threadIdx.x == 0) {
-    const double a = s->h[j].x + s->h2[j].x;
-    const double b = sqrt(fmax(nrm2, 0.0));
-    const double prev = (j > 0) ? s->beta[j - 1] : 0.0;
-    const double scale_prev = (j > 0) ? s->scl[j - 1] : 0.0;
-    const int brk_prev = (j > 0) ? s->brk[j - 1] : 0;
-    const double ref = fmax(scale_prev, fabs(a) + prev);
-    const int brk = brk_prev || (b <= 1e-12 * ref);
-    s_b = b;
-    s_brk = brk;
-    if (blockIdx.x == 0) {
-      s->alpha[j] = a;
-      s->beta[j] = brk ? 0.0 : b;
-      s->scl[j] = ref;
-      s->brk[j] = brk;
-      s->broken = brk;
-      if (brk && !brk_prev) s->kd = j + 1;
+    w[i] = make_double2(x.x * inv, x.y * inv);
+    i += step;
+    if (i < n) {
+      x = w[i];
+      if (second) lz_column<KR>(n, k, i, V, v);
     }
   }
+  if (blockIdx.x != 0 || threadIdx.x >= 64) return;
+  const int kd_new = brk && !brk_prev ? k : kd_prev;
+  if (lane == 0) {
+    s->alpha[j] = a;
+    s->beta[j] = brk ? 0.0 : beta;
+    s->scl[j] = ref;
+    s->brk[j] = brk;
+    s->broken = brk;
+    s->kd = kd_new;
+  }
+  if (!ritz) return;
+  if (lane < k) {
+    as[lane] = lane == j ? a : s->alpha[lane];
+    bs[lane] = lane == j ? (brk ? 0.0 : beta) : s->beta[lane];
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int kd = brk ? kd_new : k;
+  double theta, y[LZ_KREG];
+  lz_tridiag(as, bs, kd, &theta, y);
+  if (lane == 0) {
+    double last = 0.0;
+#pragma unroll
+    for (int q = 0; q < LZ_KREG; ++q) {
+      s->y[q] = y[q];
+      if (q == kd - 1) last = y[q];
+    }
+    out[0] = theta;
+    out[1] = brk ? 0.0 : fabs(beta * last);
+  }
+}
+
+// x = sum_{j<k} y_j V_j over V_0 (k > 0), or x unchanged (k == 0), with the
+// block sums of |x|^2 in pn.
+__global__ __launch_bounds__(LZ_THREADS) void lz_combine(int64_t n, int k, double2* __restrict__ x,
+                                                         const double* __restrict__ y,
+                                                         double* __restrict__ pn) {
+  __shared__ double red[LZ_THREADS / 64];
+  double nrm = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)LZ_THREADS + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * LZ_THREADS) {
+    double2 acc;
+    if (k == 0) {
+      acc = x[i];
+    } else {
+      acc = make_double2(0.0, 0.0);
+      for (int j0 = 0; j0 < k; j0 += 8) {
+        double2 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = x[min(j0 + q, k - 1) * n + i];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const double t = j0 + q < k ? y[j0 + q] : 0.0;
+          acc.x = fma(v[q].x, t, acc.x);
+          acc.y = fma(v[q].y, t, acc.y);
+        }
+      }
+      x[i] = acc;
+    }
+    nrm += cabs2(acc);
+  }
+  nrm = wave::sum(nrm);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = nrm;
   __syncthreads();
-  const double inv = s_brk ? 0.0 : 1.0 / s_b;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double2 x = w[i];
-    w[i] = make_double2(x.x * inv, x.y * inv);
-  }
+  if (threadIdx.x == 0) pn[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// Scale v in place by 1/sqrt(<v,v>) read from s->nrm.
-__global__ void lz_unit(int64_t n, const LzScalars* __restrict__ s, double2* __restrict__ v) {
-  const double nn = sqrt(fmax(s->nrm.x, 0.0));
+// v = x / |x| from the block sums pn of |x|^2 (0 if x is), to `copy` as well if
+// given; the scalars are reset for the cycle that starts from v.
+__global__ __launch_bounds__(LZ_THREADS) void lz_unit(int64_t n, int nb,
+                                                      const double* __restrict__ pn,
+                                                      const double2* x, double2* v, double2* copy,
+                                                      LzScalars* __restrict__ s) {
+  const double nn = sqrt(fmax(lz_wave_sum(nb, pn), 0.0));
   const double inv = (nn > 0.0) ? 1.0 / nn : 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double2 x = v[i];
-    v[i] = make_double2(x.x * inv, x.y * inv);
-  }
-}
-
-__global__ void lz_reset(LzScalars* s) {
-  if (threadIdx.x == 0) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     s->broken = 0;
     s->kd = 0;
-    s->scale = 0.0;
   }
-}
-
-// Sturm count: number of eigenvalues of the leading kd x kd block below x.
-__device__ int sturm(const double* a, const double* b, int kd, double x) {
-  int cnt = 0;
-  double d = a[0] - x;
-  if (d < 0.0) ++cnt;
-  for (int i = 1; i < kd; ++i) {
-    const double dd = (d == 0.0) ? 1e-300 : d;
-    d = a[i] - x - b[i - 1] * b[i - 1] / dd;
-    if (d < 0.0) ++cnt;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const double2 t = x[i], u = make_double2(t.x * inv, t.y * inv);
+    v[i] = u;
+    if (copy) copy[i] = u;
   }
-  return cnt;
-}
-
-// Lowest eigenpair of the symmetric tridiagonal T = tridiag(beta, alpha, beta)
-// of dimension kd (= m, or the breakdown size): 64-way multisection on Sturm
-// counts for theta, then inverse iteration (tridiagonal LU with partial
-// pivoting, LAPACK dgttrf/dgttrs steps) for y.  One wavefront; alpha and beta
-// are staged in LDS first, so the serial Sturm recurrences and the inverse
-// iteration wait on no global loads.  Ten rounds narrow the Gershgorin
-// interval by 65^10 (about 1e-18 of its width), below the spacing of doubles.
-__global__ __launch_bounds__(64) void lz_tridiag(LzScalars* s, int m) {
-  __shared__ double lo_s, hi_s;
-  __shared__ double a[64], b[64];
-  const int lane = threadIdx.x;
-  const int kd = s->broken ? s->kd : m;
-  a[lane] = (lane < m) ? s->alpha[lane] : 0.0;
-  b[lane] = (lane < m) ? s->beta[lane] : 0.0;
-  __syncthreads();
-  if (lane == 0) {
-    double lo = 1e300, hi = -1e300;
-    for (int i = 0; i < kd; ++i) {
-      const double r = (i > 0 ? fabs(b[i - 1]) : 0.0) + (i < kd - 1 ? fabs(b[i]) : 0.0);
-      lo = fmin(lo, a[i] - r);
-      hi = fmax(hi, a[i] + r);
-    }
-    const double pad = 1e-12 * fmax(fabs(lo), fabs(hi)) + 1e-300;
-    lo_s = lo - pad;
-    hi_s = hi + pad;
-  }
-  __syncthreads();
-  for (int round = 0; round < 10; ++round) {
-    const double lo = lo_s, hi = hi_s;
-    const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
-    const int c = sturm(a, b, kd, x);
-    // smallest lane whose point has at least one eigenvalue below it
-    const unsigned long long mask = __ballot(c >= 1);
-    __syncthreads();
-    if (lane == 0) {
-      if (mask) {
-        const int l = __ffsll((long long)mask) - 1;
-        const double nhi = lo + (hi - lo) * (double)(l + 1) / 65.0;
-        const double nlo = (l == 0) ? lo : lo + (hi - lo) * (double)l / 65.0;
-        lo_s = nlo;
-        hi_s = nhi;
-      } else {
-        lo_s = lo + (hi - lo) * 64.0 / 65.0;
-      }
-    }
-    __syncthreads();
-  }
-  if (lane != 0) return;
-  const double theta = 0.5 * (lo_s + hi_s);
-  // Inverse iteration on (T - theta I), one lane; the factors live in LDS
-  // (dynamically indexed private arrays would spill to scratch memory).
-  __shared__ double d[64], dl[64], du[64], du2[64], y[64];
-  __shared__ int piv[64];
-  double tnorm = 0.0;
-  for (int i = 0; i < kd; ++i) tnorm = fmax(tnorm, fabs(a[i]) + (i < kd - 1 ? fabs(b[i]) : 0.0));
-  const double tiny = 2.220446049250313e-16 * fmax(tnorm, 1e-300);
-  for (int i = 0; i < kd; ++i) {
-    d[i] = a[i] - theta;
-    du[i] = (i < kd - 1) ? b[i] : 0.0;
-    dl[i] = (i < kd - 1) ? b[i] : 0.0;
-    du2[i] = 0.0;
-    piv[i] = i;
-  }
-  for (int i = 0; i < kd - 1; ++i) {
-    if (fabs(d[i]) >= fabs(dl[i])) {
-      if (d[i] == 0.0) d[i] = tiny;
-      const double fact = dl[i] / d[i];
-      dl[i] = fact;
-      d[i + 1] -= fact * du[i];
-      piv[i] = i;
-    } else {
-      const double fact = d[i] / dl[i];
-      d[i] = dl[i];
-      dl[i] = fact;
-      const double temp = du[i];
-      du[i] = d[i + 1];
-      d[i + 1] = temp - fact * d[i + 1];
-      if (i < kd - 2) {
-        du2[i] = du[i + 1];
-        du[i + 1] = -fact * du[i + 1];
-      }
-      piv[i] = i + 1;
-    }
-  }
-  for (int i = 0; i < kd; ++i)
-    if (d[i] == 0.0) d[i] = tiny;
-  for (int i = 0; i < kd; ++i) y[i] = 1.0;
-  for (int it = 0; it < 4; ++it) {
-    for (int i = 0; i < kd - 1; ++i) {
-      if (piv[i] == i) {
-        y[i + 1] -= dl[i] * y[i];
-      } else {
-        const double temp = y[i];
-        y[i] = y[i + 1];
-        y[i + 1] = temp - dl[i] * y[i];
-      }
-    }
-    y[kd - 1] /= d[kd - 1];
-    if (kd > 1) y[kd - 2] = (y[kd - 2] - du[kd - 2] * y[kd - 1]) / d[kd - 2];
-    for (int i = kd - 3; i >= 0; --i) y[i] = (y[i] - du[i] * y[i + 1] - du2[i] * y[i + 2]) / d[i];
-    double nn = 0.0;
-    for (int i = 0; i < kd; ++i) nn += y[i] * y[i];
-    nn = sqrt(nn);
-    for (int i = 0; i < kd; ++i) y[i] /= nn;
-  }
-  // Fix the sign: largest component positive.
-  int imax = 0;
-  for (int i = 1; i < kd; ++i)
-    if (fabs(y[i]) > fabs(y[imax])) imax = i;
-  const double sg = (y[imax] < 0.0) ? -1.0 : 1.0;
-  for (int i = 0; i < 64; ++i) s->y[i] = (i < kd) ? sg * y[i] : 0.0;
-  s->theta = theta;
-  s->resid = (kd == m && !s->broken) ? fabs(b[m - 1] * y[kd - 1]) : 0.0;
 }
 
 struct EigWork {
   double2* V;      // (m + 1) x n
   double2* x1;     // a*c*d1*d2*f
   double2* x2;     // a*d1*d2*w2*f
-  double2* part;   // reduction partials (64 x nblk)
-  double2* part2;  // second-pass partials (64 x nblk)
-  double* pnorm;   // partial squared norms (3 x nblk: before pass 1, after it, final)
+  double2* part;   // reduction partials (LZ_KREG x blocks)
+  double2* part2;  // second-pass partials (LZ_KREG x blocks)
+  double* pnorm;   // partial squared norms (2 x blocks: before pass 1, after it)
   double2* ks;     // split-K partials of the matvec GEMMs
   LzScalars* sc;
 };
 
 inline int64_t al256(int64_t x) { return (x + 255) & ~int64_t(255); }
-
-// Partial-sum slots needed by both the Lanczos passes and zmdotc_impl.
-inline int64_t part_blocks(int64_t n) {
-  const int64_t a = lz_blocks(n), b = reduce_blocks(n);
-  return a > b ? a : b;
-}
 
 // Split-K scratch (elements) of the two matvec GEMMs.
 int64_t matvec_ks_elems(int64_t a, int64_t c, int64_t b, int64_t d1, int64_t d2, int64_t w2,
@@ -513,9 +507,9 @@ int64_t eig_bytes_full(int64_t chiL, int64_t c, int64_t d1, int64_t d2, int64_t 
   b += al256((m + 1) * n * 16);
   b += al256(chiL * c * d1 * d2 * chiR * 16);
   b += al256(chiL * d1 * d2 * w2 * chiR * 16);
-  b += al256(64 * part_blocks(n) * 16);
-  b += al256(64 * part_blocks(n) * 16);
-  b += al256(3 * part_blocks(n) * 8);
+  b += al256(LZ_KREG * lz_blocks(n) * 16);
+  b += al256(LZ_KREG * lz_blocks(n) * 16);
+  b += al256(2 * lz_blocks(n) * 8);
   b += al256(matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR) * 16);
   b += al256(sizeof(LzScalars));
   return b;
@@ -533,11 +527,11 @@ EigWork eig_carve(void* work, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   w.x2 = (double2*)p;
   p += al256(chiL * d1 * d2 * w2 * chiR * 16);
   w.part = (double2*)p;
-  p += al256(64 * part_blocks(n) * 16);
+  p += al256(LZ_KREG * lz_blocks(n) * 16);
   w.part2 = (double2*)p;
-  p += al256(64 * part_blocks(n) * 16);
+  p += al256(LZ_KREG * lz_blocks(n) * 16);
   w.pnorm = (double*)p;
-  p += al256(3 * part_blocks(n) * 8);
+  p += al256(2 * lz_blocks(n) * 8);
   w.ks = (double2*)p;
   p += al256(matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR) * 16);
   w.sc = (LzScalars*)p;
@@ -643,6 +637,38 @@ extern "C" int64_t seemps_eigensolve_workspace(int64_t chiL, int64_t c, int64_t 
 
 namespace {
 
+// Orthogonalisation of wv = H V[k-1] against V[0..k), its norm and scalars.
+template <int KR>
+void lz_step_kr(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
+                bool ritz, double* out, hipStream_t s) {
+  const double orth = 8.0 * n * k;
+  {
+    TimedLaunch timed("lz_orth1", s, orth);
+    hipLaunchKernelGGL(lz_orth1<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part,
+                       pn0);
+  }
+  {
+    TimedLaunch timed("lz_orth2", s, 2.0 * orth);
+    hipLaunchKernelGGL(lz_orth2<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part,
+                       w.part2, pn1, w.sc);
+  }
+  TimedLaunch timed("lz_orth3", s, orth);
+  hipLaunchKernelGGL(lz_orth3<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part2, pn0,
+                     pn1, w.sc, ritz ? 1 : 0, out);
+}
+
+void lz_step(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
+             bool ritz, double* out, hipStream_t s) {
+  switch ((k + 3) / 4) {
+    case 1: return lz_step_kr<4>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 2: return lz_step_kr<8>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 3: return lz_step_kr<12>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 4: return lz_step_kr<16>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 5: return lz_step_kr<20>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    default: return lz_step_kr<24>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+  }
+}
+
 int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, int64_t w2,
                     int64_t chiR, const void* L, const void* Hm, const void* R, const void* v0,
                     void* evec, int64_t ncv, double tol, int64_t maxiter, double* stats,
@@ -665,19 +691,19 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   const double2* L_ = (const double2*)L;
   const double2* H_ = (const double2*)Hm;
   const double2* R_ = (const double2*)R;
-  const unsigned gb = grid_for(n);
   const int nbk = lz_blocks(n);
   int st;
+  double* pn0 = w.pnorm;
+  double* pn1 = w.pnorm + nbk;
   // V[0] = v0 / ||v0||
-  SEEMPS_HIP(hipMemcpyAsync(w.V, v0, n * 16, hipMemcpyDeviceToDevice, st_));
-  if ((st = zmdotc_impl(n, 1, w.V, n, w.V, &w.sc->nrm, w.part, st_))) return st;
-  hipLaunchKernelGGL(lz_unit, dim3(gb), dim3(256), 0, st_, n, w.sc, w.V);
+  hipLaunchKernelGGL(lz_combine, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, 0, (double2*)v0,
+                     w.sc->y, pn0);
+  hipLaunchKernelGGL(lz_unit, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, nbk, pn0,
+                     (const double2*)v0, w.V, (double2*)nullptr, w.sc);
   if ((st = check_launch("lz_unit"))) return st;
   double theta = 0.0, resid = 0.0;
   double* hp = (double*)pinned_stage(PINNED_BYTES);  // host reads of the scalars
   SEEMPS_CHECK_ARG(hp != nullptr, "pinned host staging could not be allocated");
-  static_assert(offsetof(LzScalars, resid) == offsetof(LzScalars, theta) + 8,
-                "theta and resid are read together");
   int64_t matvecs = 0, matvecs32 = 0, cycle = 0;
   bool converged = false;
   // FP32 phase: the operator is applied with FP32 products, whose rounding
@@ -696,7 +722,6 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   const bool early = n >= 8192;
   const int64_t first_check = 4, check_every = 2;
   for (cycle = 0; cycle < maxiter; ++cycle) {
-    hipLaunchKernelGGL(lz_reset, dim3(1), dim3(64), 0, st_, w.sc);
     int64_t kd_eff = m;
     for (int64_t j = 0; j < m; ++j) {
       double2* vj = w.V + j * n;
@@ -708,78 +733,36 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
         return st;
       ++matvecs;
       if (mv_prec == SEEMPS_PREC_FP32) ++matvecs32;
-      // Gram-Schmidt against V[0..j] with the DGKS correction, then the norm:
-      // four launches (dots | subtract + dots | conditional subtract | normalise).
-      const int kk = (int)(j + 1);
-      const double orth = 8.0 * n * kk;
-      double* pn0 = w.pnorm;
-      double* pn1 = w.pnorm + nbk;
-      double* pn2 = w.pnorm + 2 * nbk;
-      {
-        TimedLaunch timed("lz_orth1", st_, orth);
-        hipLaunchKernelGGL(lz_orth1, dim3(nbk), dim3(256), 0, st_, n, kk, w.V, wv, w.part, pn0);
-      }
-      {
-        TimedLaunch timed("lz_orth2", st_, 2.0 * orth);
-        hipLaunchKernelGGL(lz_orth2, dim3(nbk), dim3(256), 0, st_, n, kk, w.V, wv, w.part,
-                           w.part2, pn1, w.sc->h);
-      }
-      {
-        TimedLaunch timed("lz_orth3", st_, orth);
-        hipLaunchKernelGGL(lz_orth3, dim3(nbk), dim3(256), 0, st_, n, kk, w.V, wv, w.part2, pn0,
-                           pn1, pn2, w.sc->h2);
-      }
-      {
-        TimedLaunch timed("lz_finish", st_, 0.0);
-        hipLaunchKernelGGL(lz_finish, dim3(gb), dim3(256), 0, st_, n, nbk, (int)j, pn2, w.sc,
-                           wv);
-      }
+      // the Ritz pair after the last step and after each one that is checked
+      const int64_t kd = j + 1;
+      const bool check = early && mv_prec == SEEMPS_PREC_FP64 && kd < m && kd >= first_check &&
+                         (kd - first_check) % check_every == 0;
+      lz_step(n, (int)kd, nbk, w, wv, pn0, pn1, check || kd == m, hp, st_);
       if ((st = check_launch("lanczos step"))) return st;
       if (prec == SEEMPS_PREC_MIXED && cycle == 0 && j == 0) {
-        double* ab = hp;
+        double* ab = hp + 2;
         SEEMPS_HIP(hipMemcpyAsync(&ab[0], &w.sc->alpha[0], 8, hipMemcpyDeviceToHost, st_));
         SEEMPS_HIP(hipMemcpyAsync(&ab[1], &w.sc->beta[0], 8, hipMemcpyDeviceToHost, st_));
         SEEMPS_HIP(hipStreamSynchronize(st_));
         if (ab[1] > fp32_start * fmax(eps23, fabs(ab[0]))) mv_prec = SEEMPS_PREC_FP32;
       }
-      const int64_t kd = j + 1;
-      if (early && mv_prec == SEEMPS_PREC_FP64 && kd < m && kd >= first_check &&
-          (kd - first_check) % check_every == 0) {
-        {
-          TimedLaunch timed("lz_tridiag", st_, 0.0);
-          hipLaunchKernelGGL(lz_tridiag, dim3(1), dim3(64), 0, st_, w.sc, (int)kd);
-        }
-        if ((st = check_launch("lz_tridiag"))) return st;
-        double* h = hp;  // theta and resid are adjacent in LzScalars
-        SEEMPS_HIP(hipMemcpyAsync(h, &w.sc->theta, 16, hipMemcpyDeviceToHost, st_));
+      if (check) {
         SEEMPS_HIP(hipStreamSynchronize(st_));
-        if (h[1] <= tol * fmax(eps23, fabs(h[0]))) {
+        if (hp[1] <= tol * fmax(eps23, fabs(hp[0]))) {
           kd_eff = kd;
           break;
         }
       }
     }
-    if (kd_eff == m) {
-      {
-        TimedLaunch timed("lz_tridiag", st_, 0.0);
-        hipLaunchKernelGGL(lz_tridiag, dim3(1), dim3(64), 0, st_, w.sc, (int)m);
-      }
-      if ((st = check_launch("lz_tridiag"))) return st;
-    }
-    // Ritz vector into V[m] (free: at most V[kd_eff] holds a Lanczos vector),
-    // normalise, restart from it.
-    double2* x = w.V + m * n;
-    hipLaunchKernelGGL(combine_kernel, dim3(gb), dim3(256), 0, st_, n, (int)kd_eff, w.V, n,
-                       w.sc->y, x);
-    if ((st = check_launch("combine"))) return st;
-    if ((st = zmdotc_impl(n, 1, x, n, x, &w.sc->nrm, w.part, st_))) return st;
-    hipLaunchKernelGGL(lz_unit, dim3(gb), dim3(256), 0, st_, n, w.sc, x);
-    SEEMPS_HIP(hipMemcpyAsync(w.V, x, n * 16, hipMemcpyDeviceToDevice, st_));
-    double* h = hp;
-    SEEMPS_HIP(hipMemcpyAsync(h, &w.sc->theta, 16, hipMemcpyDeviceToHost, st_));
+    // Ritz vector over V[0], normalised: the result, or the next cycle's start
+    hipLaunchKernelGGL(lz_combine, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, (int)kd_eff, w.V,
+                       w.sc->y, pn0);
+    hipLaunchKernelGGL(lz_unit, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, nbk, pn0, w.V, w.V,
+                       (double2*)evec, w.sc);
+    if ((st = check_launch("lz_unit"))) return st;
     SEEMPS_HIP(hipStreamSynchronize(st_));
-    theta = h[0];
-    resid = h[1];
+    theta = hp[0];
+    resid = hp[1];
     const double scale = fmax(eps23, fabs(theta));
     if (mv_prec == SEEMPS_PREC_FP32 && prec == SEEMPS_PREC_MIXED) {
       // An FP32 residual meets the test only for tolerances FP32 can resolve.
@@ -798,7 +781,6 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
       break;
     }
   }
-  SEEMPS_HIP(hipMemcpyAsync(evec, w.V, n * 16, hipMemcpyDeviceToDevice, st_));
   if (stats) {
     stats[0] = theta;
     stats[1] = resid;
