@@ -80,6 +80,17 @@ __device__ __forceinline__ double cabs2(double2 a) { return a.x * a.x + a.y * a.
 
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Workgroups are handed to the 8 XCDs in turn (workgroup b to XCD b mod 8).
+// Renumber them so that each XCD takes one contiguous run of tiles:
+// the run shares its inputs inside one L2.
+// A bijection on [0, n) for any n.
+__device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t n) {
+  constexpr int X = 8;
+  const int64_t q = n / X, r = n % X;
+  const int64_t x = b % X, i = b / X;
+  return x * q + (x < r ? x : r) + i;
+}
+
 // Pinned host buffer of at least `bytes` for small device-to-host reads (one
 // per host thread; nullptr if it cannot be allocated).  The caller copies into
 // it on its stream and synchronises before reading.

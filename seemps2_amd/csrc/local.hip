@@ -6,49 +6,72 @@
 namespace seemps {
 namespace {
 
-constexpr int LQ = 64;  // q-values per workgroup of zlocal
+constexpr int LIC = 64;  // rows of the operator staged in LDS at a time
 
-// out[p, j1, q, j2] (+)= sum_{i0 <= i < i0 + IC} in[p, i, q] Mop[i, j1, j2] for the
-// output columns j = j1 * J2 + j2 in [j0, j0 + JC), j0 = blockIdx.y * JC.
-// One workgroup handles (p, 64 consecutive q, one j tile); the IC x 64 input
-// slab and the IC x JC operator tile are staged in LDS, 4 threads per q split
-// the tile's outputs.  The host runs the i tiles one after another, the later
-// ones accumulating, so a contracted index of any size fits in LDS.
-__global__ __launch_bounds__(256) void zlocal_kernel(int64_t P, int I, int64_t Q, int J1, int J2,
-                                                     int64_t nqb, int i0, int IC, int JC,
-                                                     const double2* __restrict__ in,
+// out[p, j1, q, j2] (+)= sum_i in[p, i, q] Mop[i, j1, j2]; outputs j = j1 J2 + j2.
+// A thread takes one (p, q), numbered through so that no width of q leaves lanes
+// idle, and JT consecutive outputs in registers.  It reads its inputs straight from
+// memory, eight ahead of the eight in use, and the operator's entries, the same
+// for all lanes, from LDS: one LDS read for four FMAs and one load for 4 JT.  What
+// bounds a short call is its launch and the loads of i in turn, a long one the
+// memory.  The J / JT groups of one (p, q) run lie next to each other on one XCD
+// and share the inputs in its L2.  P = Q = 96, I = J = 20: staging inputs in LDS
+// with a thread per five outputs, two LDS reads for four FMAs, took 9.6 us, this 5.6;
+// P = Q = 256 16.1 -> 13.9.
+template <int JT>
+__global__ __launch_bounds__(256) void zlocal_kernel(int64_t PQ, int I, int64_t Q, int J1, int J2,
+                                                     int groups, const double2* __restrict__ in,
                                                      const double2* __restrict__ Mop,
                                                      double2* __restrict__ out, int accumulate) {
-  extern __shared__ double2 smem[];
+  constexpr int U = 8;
+  __shared__ double2 ms[LIC * JT];
   const int J = J1 * J2;
-  const int j0 = blockIdx.y * JC;
-  const int jn = min(JC, J - j0);
-  double2* xs = smem;            // [IC][LQ]
-  double2* ms = smem + IC * LQ;  // [IC][JC]
-  const int64_t p = blockIdx.x / nqb;
-  const int64_t q0 = (blockIdx.x % nqb) * LQ;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < IC * LQ; e += blockDim.x) {
-    const int i = e / LQ, ql = e % LQ;
-    const int64_t q = q0 + ql;
-    xs[e] = (q < Q) ? in[(p * I + i0 + i) * Q + q] : make_double2(0.0, 0.0);
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j0 = (int)(tile % groups) * JT;
+  const int64_t e = tile / groups * 256 + threadIdx.x;
+  const int64_t ec = min(e, PQ - 1);  // lanes past the end read the last, store nothing
+  const int64_t p = PQ <= 0x7fffffff ? (int64_t)((uint32_t)ec / (uint32_t)Q) : ec / Q;
+  const int64_t q = ec - p * Q;
+  const double2* x = in + p * I * Q + q;
+  double2 acc[JT];
+#pragma unroll
+  for (int j = 0; j < JT; ++j) acc[j] = make_double2(0.0, 0.0);
+  double2 v[2][U];
+  auto load = [&](int i, double2 (&r)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = x[min(i + u, I - 1) * Q];
+  };
+  load(0, v[0]);
+  if (I > U) load(U, v[1]);
+  for (int i0 = 0; i0 < I; i0 += LIC) {
+    const int n = min(LIC, I - i0);
+    if (i0) __syncthreads();
+    for (int t = threadIdx.x; t < n * JT; t += 256)
+      ms[t] = Mop[(int64_t)(i0 + t / JT) * J + min(j0 + t % JT, J - 1)];
+    __syncthreads();
+    for (int b = 0; b < n; b += 2 * U) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int i = b + h * U;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (i + u < n) {
+#pragma unroll
+            for (int j = 0; j < JT; ++j) acc[j] = cfma(v[h][u], ms[(i + u) * JT + j], acc[j]);
+          }
+        }
+        if (i0 + i + 2 * U < I) load(i0 + i + 2 * U, v[h]);
+      }
+    }
   }
-  for (int e = tid; e < IC * jn; e += blockDim.x) {
-    const int i = e / jn, jl = e % jn;
-    ms[i * JC + jl] = Mop[(int64_t)(i0 + i) * J + j0 + jl];
-  }
-  __syncthreads();
-  const int ql = tid % LQ;
-  const int64_t q = q0 + ql;
-  if (q >= Q) return;
-  for (int jl = tid / LQ; jl < jn; jl += blockDim.x / LQ) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int i = 0; i < IC; ++i) acc = cfma(xs[i * LQ + ql], ms[i * JC + jl], acc);
-    const int j = j0 + jl;
-    const int j1 = j / J2, j2 = j % J2;
+  if (e >= PQ) return;
+#pragma unroll
+  for (int j = 0; j < JT; ++j) {
+    if (j0 + j >= J) break;
+    const int j1 = (j0 + j) / J2, j2 = (j0 + j) % J2;
     const int64_t o = ((p * J1 + j1) * Q + q) * J2 + j2;
-    if (accumulate) acc = cadd(acc, out[o]);
-    out[o] = acc;
+    if (accumulate) acc[j] = cadd(acc[j], out[o]);
+    out[o] = acc[j];
   }
 }
 
@@ -164,32 +187,18 @@ int zlocal_impl(int64_t P, int64_t I, int64_t Q, int64_t J1, int64_t J2, const d
   SEEMPS_CHECK_ARG(P >= 0 && I >= 1 && Q >= 0 && J1 >= 1 && J2 >= 1, "zlocal: bad dimensions");
   SEEMPS_CHECK_ARG(I <= 0x7fffffff && J1 * J2 <= 0x7fffffff, "zlocal: dimensions too large");
   if (P == 0 || Q == 0) return SEEMPS_OK;
-  const int64_t J = J1 * J2;
-  // LDS tiles: IC x 64 inputs and IC x JC operator entries, at most 3072
-  // complex values (48 KiB).  When the whole operator fits (the MPO and
-  // physical indices of d = 2 chains) one launch does everything; otherwise
-  // the contracted index runs in tiles of 32 and the outputs in tiles of 32.
-  int64_t IC = I, JC = J;
-  if (I * LQ + I * J > 3072) {
-    IC = I < 32 ? I : 32;
-    JC = (3072 - IC * LQ) / IC;
-    if (JC > J) JC = J;
-  }
-  const int64_t nqb = ceil_div(Q, LQ);
-  const int64_t nblocks = P * nqb;
-  const int64_t njb = ceil_div(J, JC);
-  SEEMPS_CHECK_ARG(nblocks <= 0x7fffffff && njb <= 65535, "zlocal: grid too large");
-  const size_t shmem = (size_t)(IC * LQ + IC * JC) * sizeof(double2);
+  const int64_t J = J1 * J2, PQ = P * Q;
+  // Ten outputs a thread where that still leaves eight wavefronts a CU or more,
+  // four for more wavefronts otherwise.
+  const int64_t runs = ceil_div(PQ, 256);
+  const bool wide = runs * ceil_div(J, 10) >= 512 && J > 4;
+  const int64_t groups = ceil_div(J, wide ? 10 : 4);
+  SEEMPS_CHECK_ARG(runs * groups <= 0x7fffffff, "zlocal: grid too large");
   TimedLaunch timed("zlocal_kernel", stream, 8.0 * P * I * Q * J);
-  for (int64_t i0 = 0; i0 < I; i0 += IC) {
-    const int64_t ic = (I - i0) < IC ? (I - i0) : IC;
-    hipLaunchKernelGGL(zlocal_kernel, dim3((unsigned)nblocks, (unsigned)njb), dim3(256), shmem,
-                       stream, P, (int)I, Q, (int)J1, (int)J2, nqb, (int)i0, (int)ic, (int)JC,
-                       in, Mop, out, (i0 > 0) ? 1 : accumulate);
-    const int st = check_launch("zlocal");
-    if (st) return st;
-  }
-  return SEEMPS_OK;
+  hipLaunchKernelGGL(wide ? zlocal_kernel<10> : zlocal_kernel<4>, dim3((unsigned)(runs * groups)),
+                     dim3(256), 0, stream, PQ, (int)I, Q, (int)J1, (int)J2, (int)groups, in, Mop,
+                     out, accumulate);
+  return check_launch("zlocal");
 }
 
 int zaxpby_impl(int64_t n, double2 a, const double2* x, int conj_x, double2 b, double2* y,

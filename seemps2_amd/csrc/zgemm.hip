@@ -161,17 +161,6 @@ __device__ __forceinline__ void store_b(T* __restrict__ s_re, T* __restrict__ s_
   }
 }
 
-// Workgroups are handed to the 8 XCDs in turn (workgroup b to XCD b mod 8).
-// Renumber them so that each XCD takes one contiguous run of output tiles
-// (row-major over the tile grid): the runs share A row panels inside one L2.
-// A bijection on [0, n) for any n.
-__device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t n) {
-  constexpr int X = 8;
-  const int64_t q = n / X, r = n % X;
-  const int64_t x = b % X, i = b / X;
-  return x * q + (x < r ? x : r) + i;
-}
-
 // Workgroups per CU each tile shape is compiled for (bounds the registers).
 // The 3M 32 x 32 kernel holds a third accumulator and the operand sums: five
 // workgroups per CU keep it free of spills.

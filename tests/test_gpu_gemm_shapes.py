@@ -1,4 +1,4 @@
-"""Edges of the direct GEMM kernel: tiles of 16 and 32, K remainders of every
+"""Edges of the direct GEMM and the local-operator kernels: tiles of 16 and 32, K remainders of every
 wavefront's run, leading dimensions beyond the rows, all sixteen operand forms.
 
 Gaussian integers: every partial sum is an exact integer in any order, so the
@@ -48,3 +48,27 @@ def test_direct_gemm_edges(M, N, K_):
             out = K.to_numpy(c)
             assert np.array_equal(out[:, :N], ref), (opA, opB)
             assert np.isnan(out[:, N:]).all()
+
+
+# remainders of the eight loads ahead, one and two stages of operator rows (64), outputs
+# short of a group of four, runs that end inside a workgroup and inside a q range, J2 > 1,
+# ten outputs a thread (the last three)
+@pytest.mark.parametrize("P,I,Q,J1,J2", [(1, 1, 1, 1, 1), (3, 8, 5, 2, 1), (7, 9, 37, 3, 2),
+                                         (5, 16, 51, 5, 1), (2, 17, 129, 1, 7), (3, 64, 85, 9, 1),
+                                         (4, 65, 63, 2, 3), (1, 150, 300, 13, 1),
+                                         (511, 20, 129, 20, 1), (300, 3, 437, 7, 3),
+                                         (257, 81, 512, 1, 11)])
+def test_local_edges(P, I, Q, J1, J2):
+    from seemps2_amd import kernels as K
+
+    rng = np.random.default_rng(P + 10 * I)
+
+    def ints(*shape):
+        return rng.integers(-3, 4, shape) + 1j * rng.integers(-3, 4, shape)
+
+    x, op = ints(P, I, Q), ints(I, J1, J2)
+    ref = np.tensordot(x, op, axes=(1, 0)).transpose(0, 2, 1, 3)
+    out = K.local(K.as_dev(x), K.as_dev(op), P, I, Q, J1, J2)
+    assert np.array_equal(K.to_numpy(out).reshape(ref.shape), ref)
+    out = K.local(K.as_dev(x), K.as_dev(op), P, I, Q, J1, J2, out=out, accumulate=True)
+    assert np.array_equal(K.to_numpy(out).reshape(ref.shape), 2 * ref)
