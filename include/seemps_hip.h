@@ -122,7 +122,7 @@ int seemps_zsite_product(int64_t a, int64_t d, int64_t b, int64_t c, int64_t e,
  * lists the problem of every output tile, each problem's tiles contiguous
  * from desc[p].tile0 in row-major tile order with desc[p].tiles_n tiles per
  * tile row (seemps_grouped_tiles gives a problem's tile count).  tile_cfg:
- * SEEMPS_TILE_64x64 (256 threads) or SEEMPS_TILE_32x32 (64 threads).  Op
+ * SEEMPS_TILE_64x64 or SEEMPS_TILE_32x32.  Op
  * pairs: (N,N), (H,N), (N,T), (T,N), (C,N), (N,H).  Allocates nothing and
  * does not synchronise, so it can be captured in a HIP graph. */
 #define SEEMPS_TILE_64x64 0

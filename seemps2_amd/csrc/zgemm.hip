@@ -24,6 +24,7 @@
 // MFMA f64 16x16x4 lane layout (checked on the device): A[i][k] from lane
 // i + 16k, B[k][j] from lane j + 16k, result item r of lane l is D[l/16 + 4r][l%16].
 #include "common.h"
+#include "gemm_direct.h"
 
 namespace seemps {
 namespace {
@@ -303,15 +304,11 @@ __global__ __launch_bounds__(256, tile_occupancy(TM, TN, G3)) void zgemm_kernel(
       }
 }
 
-// One 16 F x 16 F output tile per workgroup, its KS wavefronts each taking a run
-// of the K steps with the operands loaded straight into the MFMA layout (no LDS
-// staging, no barrier in the loop), and summing their partial tiles in LDS in
-// the order of the runs.  FP64 MFMA asks little of the memory path (a 32 x 32
-// step of four k is 768 cycles of the matrix core for 4 KB), so what limits
-// products of few tiles is the chain of staging and barriers that this leaves
-// out: 64^3 5.6 -> 3.1 us (a launch is 2.2), 256 x 400 x 200 15.2 -> 7.0.  Of
-// large ones the loads are the limit of 16 x 16 tiles, the matrix cores that of
-// 32 x 32 (2048 x 2048 x 512 at 75 of a large product's 72 TFLOP/s).
+// One 16 F x 16 F output tile per workgroup of KS wavefronts (gemm_direct.h).  What
+// limits products of few tiles is the chain of staging and barriers that this leaves
+// out: 64^3 5.6 -> 3.1 us (a launch is 2.2), 256 x 400 x 200 15.2 -> 7.0.  Of large
+// ones the loads are the limit of 16 x 16 tiles, the matrix cores that of 32 x 32
+// (2048 x 2048 x 512 at 75 TFLOP/s, a large library product at 72).
 template <int OPA, int OPB, int F, int KS>
 __global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, int64_t K,
                                                         double2 alpha,
@@ -319,133 +316,18 @@ __global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, in
                                                         const double2* __restrict__ B, int64_t ldb,
                                                         double2 beta, double2* __restrict__ C,
                                                         int64_t ldc) {
-  constexpr int U = 4, NBUF = 2;  // blocks of U K steps (of 4), one loaded ahead
-  constexpr bool AT = OPA == SEEMPS_OP_T || OPA == SEEMPS_OP_H;
-  constexpr bool BT = OPB == SEEMPS_OP_T || OPB == SEEMPS_OP_H;
-  constexpr double SGA = (OPA == SEEMPS_OP_C || OPA == SEEMPS_OP_H) ? -1.0 : 1.0;
-  constexpr double SGB = (OPB == SEEMPS_OP_C || OPB == SEEMPS_OP_H) ? -1.0 : 1.0;
-  extern __shared__ double2 part[];  // KS x (4 F F items) x 64 lanes
+  extern __shared__ double2 part[];
   const int64_t tiles_n = ceil_div(N, 16 * F);
   const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int64_t m0 = (tile / tiles_n) * (16 * F), n0 = (tile % tiles_n) * (16 * F);
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // rows and columns past the edge are read from the last one and not stored
-  const double2 *pa[F], *pb[F];
-#pragma unroll
-  for (int f = 0; f < F; ++f) {
-    const int64_t m = min(m0 + 16 * f + li, M - 1), n = min(n0 + 16 * f + li, N - 1);
-    pa[f] = AT ? A + m : A + m * lda;
-    pb[f] = BT ? B + n * ldb : B + n;
-  }
-  const int64_t stepA = AT ? lda : 1, stepB = BT ? 1 : ldb;
-  d4 t1[F][F], t2[F][F], t3[F][F];
-#pragma unroll
-  for (int a = 0; a < F; ++a)
-#pragma unroll
-    for (int b = 0; b < F; ++b) t1[a][b] = t2[a][b] = t3[a][b] = d4{0.0, 0.0, 0.0, 0.0};
-  auto load = [&](int64_t k, double2 (&x)[F], double2 (&y)[F]) {
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-      x[f] = pa[f][k * stepA];
-      y[f] = pb[f][k * stepB];
-    }
-  };
-  auto mac = [&](const double2 (&x)[F], const double2 (&y)[F]) {
-#pragma unroll
-    for (int a = 0; a < F; ++a)
-#pragma unroll
-      for (int b = 0; b < F; ++b) {
-        t1[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].x, y[b].x, t1[a][b], 0, 0, 0);
-        t2[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].y, y[b].y, t2[a][b], 0, 0, 0);
-        t3[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a].x + SGA * x[a].y,
-                                                        y[b].x + SGB * y[b].y, t3[a][b], 0, 0, 0);
-      }
-  };
-  const int64_t steps = ceil_div(K, (int64_t)4), per = ceil_div(steps, (int64_t)KS);
-  const int64_t s0 = min(wv * per, steps), s1 = min(s0 + per, steps);
-  const int64_t full = min(s1, K / 4);  // steps [s0, full) need no bounds test
-  const int64_t nb = full > s0 ? (full - s0) / U : 0;
-  double2 x[NBUF][U][F], y[NBUF][U][F];
-  auto load_block = [&](int64_t b, double2 (&xx)[U][F], double2 (&yy)[U][F]) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) load((s0 + b * U + u) * 4 + lk, xx[u], yy[u]);
-  };
-  if (nb > 0) {
-#pragma unroll
-    for (int i = 0; i < NBUF - 1; ++i)
-      if (i < nb) load_block(i, x[i], y[i]);
-  }
-  for (int64_t b = 0; b < nb; b += NBUF) {
-#pragma unroll
-    for (int i = 0; i < NBUF; ++i) {
-      if (b + i < nb) {
-        constexpr int AHEAD = NBUF - 1;
-        if (F > 1)
-          load_block(min(b + i + AHEAD, nb - 1), x[(i + AHEAD) % NBUF], y[(i + AHEAD) % NBUF]);
-        else if (b + i + AHEAD < nb)
-          load_block(b + i + AHEAD, x[(i + AHEAD) % NBUF], y[(i + AHEAD) % NBUF]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) mac(x[i][u], y[i][u]);
-      }
-    }
-  }
-  // the last steps together: past the run or past K they are read in bounds
-  // and count as zero
-  if (s0 + nb * U < s1) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t s = s0 + nb * U + u;
-      load(min(s * 4 + lk, K - 1), x[0][u], y[0][u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t s = s0 + nb * U + u;
-      if (s >= s1) break;
-      if (s * 4 + lk >= K) {
-#pragma unroll
-        for (int f = 0; f < F; ++f) x[0][u][f] = y[0][u][f] = make_double2(0.0, 0.0);
-      }
-      mac(x[0][u], y[0][u]);
-    }
-  }
   const bool use_beta = (beta.x != 0.0 || beta.y != 0.0);
-  auto put = [&](int a, int b, int r, double2 acc) {
-    const int64_t m = m0 + 16 * a + lk + 4 * r, n = n0 + 16 * b + li;
-    if (m < M && n < N) {
-      double2 out = cmul(alpha, acc);
-      if (use_beta) out = cfma(beta, C[m * ldc + n], out);
-      C[m * ldc + n] = out;
-    }
-  };
-#pragma unroll
-  for (int a = 0; a < F; ++a)
-#pragma unroll
-    for (int b = 0; b < F; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const double u = t1[a][b][r], v = SGA * SGB * t2[a][b][r];
-        const double2 acc = make_double2(u - v, (t3[a][b][r] - u) - v);
-        if (KS == 1)
-          put(a, b, r, acc);
-        else
-          part[(wv * (4 * F * F) + (a * F + b) * 4 + r) * 64 + lane] = acc;
-      }
-  if (KS == 1) return;
-  __syncthreads();
-#pragma unroll
-  for (int a = 0; a < F; ++a)
-#pragma unroll
-    for (int b = 0; b < F; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int item = (a * F + b) * 4 + r;
-        if (item % KS != wv && !(KS > 4 * F * F && wv == item)) continue;
-        double2 acc = part[item * 64 + lane];
-#pragma unroll
-        for (int q = 1; q < KS; ++q) acc = cadd(acc, part[(q * (4 * F * F) + item) * 64 + lane]);
-        put(a, b, r, acc);
-      }
+  direct::tile<OPA, OPB, F, KS, true>(
+      M, N, K, A, lda, B, ldb, (tile / tiles_n) * (16 * F), (tile % tiles_n) * (16 * F), wv, part,
+      [&](int64_t m, int64_t n, double2 acc) {
+        double2 out = cmul(alpha, acc);
+        if (use_beta) out = cfma(beta, C[m * ldc + n], out);
+        C[m * ldc + n] = out;
+      });
 }
 
 // Tile shape for an M x N output in `batch` slices on `num_cu` CUs.  The

@@ -72,3 +72,31 @@ def test_local_edges(P, I, Q, J1, J2):
     assert np.array_equal(K.to_numpy(out).reshape(ref.shape), ref)
     out = K.local(K.as_dev(x), K.as_dev(op), P, I, Q, J1, J2, out=out, accumulate=True)
     assert np.array_equal(K.to_numpy(out).reshape(ref.shape), 2 * ref)
+
+
+# two 32 x 32 tiles a CU or more (whole tiles), fewer (quarters), and 64 x 64 tiles
+@pytest.mark.parametrize("tile,count", [(1, 130), (1, 6), (0, 6)])
+@pytest.mark.parametrize("opA,opB", [(0, 0), (2, 0), (0, 1), (1, 0), (3, 0), (0, 2)])
+def test_grouped_gemm_edges(tile, count, opA, opB):
+    from seemps2_amd import batch, kernels as K
+
+    rng = np.random.default_rng(count)
+    edges = [1, 15, 16, 17, 33, 64, 65, 80, 97]
+    probs, refs, outs, keep = [], [], [], []
+    for p in range(count):
+        M, N, Kd = edges[p % 9], edges[(p // 2) % 9], int(rng.integers(1, 90))
+        A = rng.integers(-3, 4, (Kd, M) if opA in (1, 2) else (M, Kd)) + 1j * 0
+        A = A + 1j * rng.integers(-3, 4, A.shape)
+        B = rng.integers(-3, 4, (N, Kd) if opB in (1, 2) else (Kd, N)) + 1j * 0
+        B = B + 1j * rng.integers(-3, 4, B.shape)
+        Ad, Bd, Cd = K.as_dev(A), K.as_dev(B), K.empty(M, N)
+        keep += [Ad, Bd]
+        probs.append((M, N, Kd, Ad, A.shape[1], Bd, B.shape[1], Cd, N))
+        refs.append(OPS[opA](A) @ OPS[opB](B))
+        outs.append(Cd)
+    gg = batch.GroupedGemm(opA, opB, probs, tile)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert (gg.ntiles >= 2 * cus) == (count == 130)
+    gg.launch()
+    for Cd, ref in zip(outs, refs):
+        assert np.array_equal(K.to_numpy(Cd), ref)
