@@ -95,10 +95,24 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t n) {
 // per host thread; nullptr if it cannot be allocated).  The caller copies into
 // it on its stream and synchronises before reading.
 void* pinned_stage(size_t bytes);
-// Layout of the staging buffer: scalars at [0, PINNED_CTRL_OFF), the SVD
-// control block at [PINNED_CTRL_OFF, PINNED_BYTES).
+// Layout of the staging buffer: scalars at [0, PINNED_CTRL_OFF), with the
+// flag of host_publish at PINNED_FLAG_OFF, the SVD control block at [PINNED_CTRL_OFF, PINNED_BYTES).
 constexpr size_t PINNED_CTRL_OFF = 1024;
 constexpr size_t PINNED_BYTES = 4096;
+
+// A kernel's word to the host that its results lie in pinned memory, ahead of its
+// end and of the end-of-kernel signal: the thread that stored the results calls
+// host_publish, the host waits for the same number at host_flag(stage).
+constexpr size_t PINNED_FLAG_OFF = 512;
+__host__ __device__ inline uint64_t* host_flag(void* stage) {
+  return (uint64_t*)((char*)stage + PINNED_FLAG_OFF);
+}
+uint64_t next_ticket();  // numbers of one host thread, never zero
+int wait_host_flag(uint64_t* flag, uint64_t ticket, hipStream_t stream);
+__device__ __forceinline__ void host_publish(uint64_t* flag, uint64_t ticket) {
+  __threadfence_system();
+  __hip_atomic_store(flag, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Device properties cached per device (CU count, cooperative limits).
 struct DeviceInfo {

@@ -343,7 +343,8 @@ __device__ void lz_tridiag(const double* a, const double* b, int kd, double* the
 // beta_j = |w|, alpha_j = Re(h_j + h2_j), the breakdown test and
 // v_{j+1} = w / beta_j (0 after a breakdown).  Block 0 records the scalars and,
 // with `ritz`, the lowest Ritz pair of the k vectors: y for the combination,
-// theta and the residual beta_j |y_j| to the host's `out`.
+// theta and the residual beta_j |y_j| to the host's `out`,
+// published as ticket `ritz`.
 template <int KR>
 __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
                                                        const double2* __restrict__ V,
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
                                                        const double2* __restrict__ part_in,
                                                        const double* __restrict__ pn0,
                                                        const double* __restrict__ pn1,
-                                                       LzScalars* __restrict__ s, int ritz,
+                                                       LzScalars* __restrict__ s, uint64_t ritz,
                                                        double* __restrict__ out) {
   __shared__ double2 hs[LZ_KREG];
   __shared__ double as[LZ_KREG], bs[LZ_KREG];
@@ -421,6 +422,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
     }
     out[0] = theta;
     out[1] = brk ? 0.0 : fabs(beta * last);
+    host_publish(host_flag(out), ritz);
   }
 }
 
@@ -640,7 +642,7 @@ namespace {
 // Orthogonalisation of wv = H V[k-1] against V[0..k), its norm and scalars.
 template <int KR>
 void lz_step_kr(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
-                bool ritz, double* out, hipStream_t s) {
+                uint64_t ritz, double* out, hipStream_t s) {
   const double orth = 8.0 * n * k;
   {
     TimedLaunch timed("lz_orth1", s, orth);
@@ -654,11 +656,11 @@ void lz_step_kr(int64_t n, int k, int nb, const EigWork& w, double2* wv, double*
   }
   TimedLaunch timed("lz_orth3", s, orth);
   hipLaunchKernelGGL(lz_orth3<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part2, pn0,
-                     pn1, w.sc, ritz ? 1 : 0, out);
+                     pn1, w.sc, ritz, out);
 }
 
 void lz_step(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
-             bool ritz, double* out, hipStream_t s) {
+             uint64_t ritz, double* out, hipStream_t s) {
   switch ((k + 3) / 4) {
     case 1: return lz_step_kr<4>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
     case 2: return lz_step_kr<8>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
@@ -704,6 +706,11 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   double theta = 0.0, resid = 0.0;
   double* hp = (double*)pinned_stage(PINNED_BYTES);  // host reads of the scalars
   SEEMPS_CHECK_ARG(hp != nullptr, "pinned host staging could not be allocated");
+  void* dev = nullptr;
+  SEEMPS_HIP(hipHostGetDevicePointer(&dev, hp, 0));
+  double* hp_dev = (double*)dev;
+  uint64_t ticket = 0;
+  *host_flag(hp) = 0;
   int64_t matvecs = 0, matvecs32 = 0, cycle = 0;
   bool converged = false;
   // FP32 phase: the operator is applied with FP32 products, whose rounding
@@ -737,7 +744,8 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
       const int64_t kd = j + 1;
       const bool check = early && mv_prec == SEEMPS_PREC_FP64 && kd < m && kd >= first_check &&
                          (kd - first_check) % check_every == 0;
-      lz_step(n, (int)kd, nbk, w, wv, pn0, pn1, check || kd == m, hp, st_);
+      if (check || kd == m) ticket = next_ticket();
+      lz_step(n, (int)kd, nbk, w, wv, pn0, pn1, check || kd == m ? ticket : 0, hp_dev, st_);
       if ((st = check_launch("lanczos step"))) return st;
       if (prec == SEEMPS_PREC_MIXED && cycle == 0 && j == 0) {
         double* ab = hp + 2;
@@ -747,7 +755,7 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
         if (ab[1] > fp32_start * fmax(eps23, fabs(ab[0]))) mv_prec = SEEMPS_PREC_FP32;
       }
       if (check) {
-        SEEMPS_HIP(hipStreamSynchronize(st_));
+        if ((st = wait_host_flag(host_flag(hp), ticket, st_))) return st;
         if (hp[1] <= tol * fmax(eps23, fabs(hp[0]))) {
           kd_eff = kd;
           break;
@@ -760,7 +768,7 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
     hipLaunchKernelGGL(lz_unit, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, nbk, pn0, w.V, w.V,
                        (double2*)evec, w.sc);
     if ((st = check_launch("lz_unit"))) return st;
-    SEEMPS_HIP(hipStreamSynchronize(st_));
+    if ((st = wait_host_flag(host_flag(hp), ticket, st_))) return st;
     theta = hp[0];
     resid = hp[1];
     const double scale = fmax(eps23, fabs(theta));
@@ -781,6 +789,7 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
       break;
     }
   }
+  SEEMPS_HIP(hipStreamSynchronize(st_));
   if (stats) {
     stats[0] = theta;
     stats[1] = resid;

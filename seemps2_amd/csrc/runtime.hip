@@ -68,6 +68,32 @@ void* pinned_stage(size_t bytes) {
   return buf;
 }
 
+uint64_t next_ticket() {
+  static thread_local uint64_t n = 0;
+  return ++n;
+}
+
+// Spins on the flag (a wait for the stream takes some 8 us more: end of kernel,
+// signal, wake-up; a DMRG sweep waits every second Lanczos step).  The stream is
+// asked now and then, so that a failed launch or a fault ends the wait.
+int wait_host_flag(uint64_t* flag, uint64_t ticket, hipStream_t stream) {
+  for (;;) {
+    for (int i = 0; i < 20000; ++i) {
+      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return SEEMPS_OK;
+      __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();  // not an error of the launches to come
+      continue;
+    }
+    if (e != hipSuccess) SEEMPS_HIP(e);
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == ticket) return SEEMPS_OK;
+    set_error("a kernel ended without its result");
+    return SEEMPS_ERR_RUNTIME;
+  }
+}
+
 int device_info(DeviceInfo* info) {
   // One cache entry per device; the library is used from one process per GPU.
   static thread_local int cached_dev = -1;

@@ -186,7 +186,8 @@ template <bool STAGED>
 __global__ __launch_bounds__(1024) void sort_truncate(SvdShape s, SvdWork w, double* S,
                                                       int64_t* D_dev, int method, double tol,
                                                       int64_t max_bond, double* spill,
-                                                      SplitResult* host) {
+                                                      SplitResult* host, uint64_t* flag,
+                                                      uint64_t ticket) {
   extern __shared__ double lds[];
   __shared__ int64_t sD;
   __shared__ int s_tiny;
@@ -231,6 +232,7 @@ __global__ __launch_bounds__(1024) void sort_truncate(SvdShape s, SvdWork w, dou
   if (tid == 0) {
     host->tiny = s_tiny;
     for (int i = 0; i < 3; ++i) host->status[i] = w.ctrl->info[i];
+    host_publish(flag, ticket);
   }
 }
 
@@ -327,6 +329,8 @@ int svd_split_impl(int64_t m, int64_t n, const double2* A, int mode, int method,
   SplitResult* res = (SplitResult*)hp;
   void* res_dev = nullptr;
   SEEMPS_HIP(hipHostGetDevicePointer(&res_dev, res, 0));
+  const uint64_t ticket = next_ticket();
+  *host_flag(hp) = 0;
   const SvdShape s = split_shape(m, n, di.num_cu);
   SplitWork x;
   split_carve(s, work, &x);
@@ -349,12 +353,13 @@ int svd_split_impl(int64_t m, int64_t n, const double2* A, int mode, int method,
   if (s.ncolp <= SORT_LDS)
     hipLaunchKernelGGL(sort_truncate<true>, dim3(1), dim3(1024), 2 * s.ncolp * sizeof(double), st_,
                        s, w, x.S, x.D, method, tolerance, max_bond, (double*)nullptr,
-                       (SplitResult*)res_dev);
+                       (SplitResult*)res_dev, host_flag(res_dev), ticket);
   else
     hipLaunchKernelGGL(sort_truncate<false>, dim3(1), dim3(1024), 0, st_, s, w, x.S, x.D, method,
-                       tolerance, max_bond, (double*)w.part, (SplitResult*)res_dev);
+                       tolerance, max_bond, (double*)w.part, (SplitResult*)res_dev,
+                       host_flag(res_dev), ticket);
   if ((st = check_launch("sort_truncate"))) return st;
-  SEEMPS_HIP(hipStreamSynchronize(st_));
+  if ((st = wait_host_flag(host_flag(hp), ticket, st_))) return st;
   const SplitResult got = *res;
   if (got.status[2] || !got.status[1] || getenv("SEEMPS_SVD_PROFILE")) {
     if ((st = svd_read_ctrl(work, (int)((char*)w.ctrl - (char*)work), info, st_))) return st;
