@@ -50,7 +50,7 @@ int64_t split_carve(const SvdShape& s, void* base, SplitWork* out) {
   x.w.W = (double2*)take(s.ncolp * s.len * 16);
   x.w.V = (double2*)take(s.ncolp * s.ncolp * 16);
   x.w.part = (double2*)take(2 * s.P * RMAX * PW * PW * 16);
-  x.w.sync = (unsigned int*)take((s.P + s.P * s.R) * 4);
+  x.w.sync = (unsigned int*)take(sync_words(s) * 4);
   x.w.colnrm = (double*)take(s.ncol * 8);
   x.w.colperm = (int*)take(s.ncol * 4);
   x.w.sigma = (double*)take(s.ncolp * 8);
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void load_sorted(SvdShape s, const double2* __
     if (s.transposed) v.y = -v.y;
     dst[r] = v;
   }
-  for (int64_t e = c * 256 + threadIdx.x; e < s.P + s.P * s.R; e += (int64_t)gridDim.x * 256)
+  for (int64_t e = c * 256 + threadIdx.x; e < sync_words(s); e += (int64_t)gridDim.x * 256)
     w.sync[e] = 0u;
   if (c == 0) {
     total = block_sum256(total, red);

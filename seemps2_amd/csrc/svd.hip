@@ -82,7 +82,7 @@ __host__ __device__ inline int inner_top_of(const SvdShape& s) {
   X(W, s.ncolp * s.len, double2)                                      \
   X(V, s.ncolp * s.ncolp, double2)                                    \
   X(part, 2 * s.P * RMAX * PW * PW, double2)                          \
-  X(sync, s.P + s.P * s.R, unsigned int)                              \
+  X(sync, sync_words(s), unsigned int)                                \
   X(colnrm, s.use_qr ? s.ncol : 0, double)                            \
   X(colperm, s.use_qr ? s.ncol : 0, int)                              \
   X(sigma, s.ncolp, double)                                           \
@@ -187,7 +187,7 @@ __global__ void init_v_ctrl(SvdShape s, SvdWork w) {
     const int64_t c = e / s.ncolp, r = e % s.ncolp;
     w.V[e] = make_double2((c == r && c < s.ncol) ? 1.0 : 0.0, 0.0);
   }
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < s.P + s.P * s.R;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < sync_words(s);
        e += (int64_t)gridDim.x * blockDim.x)
     w.sync[e] = 0u;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -287,6 +287,37 @@ __device__ bool wait_counters(Ctrl* ctrl, const unsigned int* c0, const unsigned
     *s_flag = ok;
   }
   // the loads that follow must stay behind the counter's
+  asm volatile("" ::: "memory");
+  __syncthreads();
+  return *s_flag != 0;
+}
+
+// Bounded wait of a step: counters c[i0] and c[i1] at `target`, and the n < 62
+// counters from c[guard] on at `guard_target`; a lane of the first wavefront each.
+__device__ bool wait_step(Ctrl* ctrl, const unsigned int* c, int64_t i0, int64_t i1,
+                          unsigned int target, int64_t guard, int64_t n,
+                          unsigned int guard_target, int* s_flag) {
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const unsigned int* mine = &c[lane == 0 ? i0 : lane == 1 ? i1 : lane < n + 2 ? guard + lane - 2 : i0];
+    const unsigned int want = lane >= 2 && lane < n + 2 ? guard_target : target;
+    unsigned long long spins = 0;
+    int ok = 1;
+    while (!__all(__hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want)) {
+      if (__hip_atomic_load(&ctrl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        ok = 0;
+        break;
+      }
+      if (++spins > SPIN_LIMIT) {
+        if (lane == 0) atomicExch(&ctrl->abort, 1u);
+        ok = 0;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    if (lane == 0) *s_flag = ok;
+  }
   asm volatile("" ::: "memory");
   __syncthreads();
   return *s_flag != 0;
@@ -449,9 +480,9 @@ __device__ __forceinline__ void rotate_columns(double2& x, double2& y, double rd
   y = cfma(sp, x0, rscale(cs, y));
 }
 
-// Level H on L.G and the tiles, on every wavefront of the workgroup; rec
-// receives its H x NP rotations.  Ends with a barrier.
-template <int H>
+// Level H on L.G and the tiles (ONE: the first only), on every wavefront of
+// the workgroup; rec receives its H x NP rotations.  Ends with a barrier.
+template <int H, bool ONE>
 __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, double tiny2) {
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (wv < 4) {
@@ -496,6 +527,8 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
     L.G[a * GP + d] = ad;
     L.G[b * GP + c] = bc;
     L.G[b * GP + d] = bd;
+  } else if (ONE && wv >= 8) {
+    for (int k = 0; k < H; ++k) __syncthreads();
   } else {
     const int w = wv & 3, which = wv >= 8;
     double2* tile = L.tile[which];
@@ -548,6 +581,7 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
 
 // Inner sweeps: level 16 (cross) or the levels from top down to 1.  Returns the
 // number of rounds of the last one, whose rotations L.rec holds.
+template <bool ONE>
 __device__ int inner_rounds(PairLds& L, double tol, double tiny2, int sweeps, bool cross, int top) {
   const double tol2 = tol * tol;
   Rot* rec = L.rec;
@@ -555,23 +589,23 @@ __device__ int inner_rounds(PairLds& L, double tol, double tiny2, int sweeps, bo
   for (int sw = 0; sw < sweeps; ++sw) {
     n = 0;
     if (top == 16) {
-      inner_level<16>(L, rec + n * NP, tol2, tiny2);
+      inner_level<16, ONE>(L, rec + n * NP, tol2, tiny2);
       n += 16;
       if (cross) continue;
     }
     if (top >= 8) {
-      inner_level<8>(L, rec + n * NP, tol2, tiny2);
+      inner_level<8, ONE>(L, rec + n * NP, tol2, tiny2);
       n += 8;
     }
     if (top >= 4) {
-      inner_level<4>(L, rec + n * NP, tol2, tiny2);
+      inner_level<4, ONE>(L, rec + n * NP, tol2, tiny2);
       n += 4;
     }
     if (top >= 2) {
-      inner_level<2>(L, rec + n * NP, tol2, tiny2);
+      inner_level<2, ONE>(L, rec + n * NP, tol2, tiny2);
       n += 2;
     }
-    inner_level<1>(L, rec + n * NP, tol2, tiny2);
+    inner_level<1, ONE>(L, rec + n * NP, tol2, tiny2);
     n += 1;
   }
   return n;
@@ -629,9 +663,12 @@ __device__ __forceinline__ void gram_store(double2* dst, GramShare q, d4 acc) {
     d[2 * ((q.ti * 16 + lk + 4 * r) * GP + q.tj * 16 + li)] = acc[r];
 }
 
-// Rows of V that chunk r rotates; one tile of them rotates along with W's.
+// Rows of V that chunk r of W rotates; one tile of them rotates along with W's.
+template <bool VSEP>
 __device__ __forceinline__ bool v_rows(const SvdShape& s, const SvdWork& w, int64_t r, int64_t* v0,
                                        int64_t* v1) {
+  *v0 = *v1 = 0;
+  if (VSEP) return false;  // V has workgroups of its own
   const int64_t rcv = ceil_div(s.ncolp, s.R);
   *v0 = r * rcv;
   *v1 = min(s.ncolp, *v0 + rcv);
@@ -640,15 +677,16 @@ __device__ __forceinline__ bool v_rows(const SvdShape& s, const SvdWork& w, int6
 
 // Phase A for item (p, r): the Gram matrix of rows [r0, r1) of the pair's
 // columns; the last tile of the rows stays in LDS, with V's.  R > 1: into dst
-// (PW x PW, i <= j only), to be summed over the chunks; else the two halves are
-// left in L.G and L.G2.
+// (PW x PW, i <= j only), to be summed over the chunks or read by V's workgroups;
+// with R = 1 the two halves are left in L.G and L.G2 as well.
+template <bool VSEP>
 __device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r,
                              int64_t r0, int64_t r1, double2* __restrict__ dst, PairLds& L) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const GramShare q = gram_share(wv);
   d4 c = {0.0, 0.0, 0.0, 0.0};
   int64_t v0, v1;
-  const bool v_live = v_rows(s, w, r, &v0, &v1);
+  const bool v_live = v_rows<VSEP>(s, w, r, &v0, &v1);
   constexpr int PER = (PW + JT / 64 - 1) / (JT / 64);  // columns of a tile per wavefront
   double2 vt[PER];
   for (int64_t rb = r0; rb == r0 || rb < r1; rb += RT) {
@@ -674,7 +712,7 @@ __device__ void partial_gram(const SvdShape& s, const SvdWork& w, int64_t bi, in
   }
   gram_store(q.half ? L.G2 : L.G, q, c);
   __syncthreads();
-  if (s.R == 1) return;
+  if (s.R == 1 && !VSEP) return;
   const auto out = shared_rsrc(dst, PW * PW);
   for (int e = threadIdx.x; e < PW * PW; e += JT) {
     const int i = e / PW, j = e % PW;
@@ -718,7 +756,7 @@ __device__ void replay(double2* __restrict__ M, int64_t ld, int64_t bi, int64_t 
 __device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj, int64_t r,
                        int64_t r0, int64_t r1, PairLds& L) {
   if (s.R == 1) {
-    partial_gram(s, w, bi, bj, r, r0, r1, nullptr, L);
+    partial_gram<false>(s, w, bi, bj, r, r0, r1, nullptr, L);
     return;
   }
   __syncthreads();
@@ -727,12 +765,13 @@ __device__ void reload(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t 
     load_tile(w.W, s.len, bi, bj, last, (int)(r1 - last), L.tile[0]);
   }
   int64_t v0, v1;
-  if (v_rows(s, w, r, &v0, &v1)) load_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
+  if (v_rows<false>(s, w, r, &v0, &v1)) load_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
 }
 
 // Phases B + C for item (p, r): G = sum of the R partials at src (R > 1), the
 // pair's off-diagonal measure (r == 0) into *off_slot, inner Jacobi, rotation of
-// this chunk's rows of W and V.  prof/pt/t0: phase timing of workgroup 0.
+// this chunk's rows of W and V (r >= R: chunk r - R of V's, its tile in LDS).  prof/pt/t0: phase timing of workgroup 0.
+template <bool VSEP>
 __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int64_t bj,
                             int64_t r, const double2* __restrict__ src,
                             unsigned long long* off_slot, double tol, double tiny2,
@@ -746,7 +785,7 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
     const int i = e / PW, j = e % PW;
     if (i > j) continue;
     double2 g;
-    if (s.R == 1) {
+    if (s.R == 1 && (!VSEP || r == 0)) {
       g = cadd(L.G[i * GP + j], L.G2[i * GP + j]);
     } else {
       g = make_double2(0.0, 0.0);
@@ -790,12 +829,17 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
   // already orthogonal to tolerance: no rotation is applied to this pair
   if (pair_off <= tol) return;
   int64_t v0, v1;
-  const bool v_live = v_rows(s, w, r, &v0, &v1);
-  const int n = inner_rounds(L, tol, tiny2, inner_sweeps, cross, inner_top_of(s));
+  const bool v_live = v_rows<VSEP>(s, w, r, &v0, &v1);
+  const int n = inner_rounds<VSEP>(L, tol, tiny2, inner_sweeps, cross, inner_top_of(s));
   if (prof) {
     const long long t1 = now_ticks();
     pt[3] += t1 - *t0;
     *t0 = t1;
+  }
+  if (VSEP && r >= s.R) {
+    const int64_t v0 = (r - s.R) * RT;
+    store_tile(w.V, s.ncolp, bi, bj, v0, (int)min((int64_t)RT, s.ncolp - v0), L.tile[0]);
+    return;
   }
   // the tile in LDS is the chunk's last one
   const int64_t r0 = r * rc, r1 = min(s.len, r0 + rc);
@@ -806,7 +850,7 @@ __device__ void pair_update(const SvdShape& s, const SvdWork& w, int64_t bi, int
   }
   if (v_live)
     store_tile(w.V, s.ncolp, bi, bj, v0, (int)(v1 - v0), L.tile[1]);
-  else if (w.V)
+  else if (w.V && !VSEP)
     replay(w.V, s.ncolp, bi, bj, v0, v1, n, cross, inner_top_of(s), L);
   if (prof) {
     const long long t1 = now_ticks();
@@ -846,8 +890,15 @@ __device__ inline void local_item(int64_t b, int64_t G, int64_t R, int64_t* p, i
 // Grams (pair counter), and a workgroup starts a step once the two pairs that
 // held its blocks in the previous step have rotated its row chunk (chunk step
 // counters).  One grid barrier per sweep reduces the convergence measure.
+// VSEP (LOCAL, VS > 0): the rows of V are rotated by VS more workgroups per pair, which
+// take the Gram matrix from W's and solve it like them.  An inner round is bound by
+// the instructions of three wavefronts a SIMD (G, a tile of W, one of V), so V on
+// other CUs shortens it; V's workgroups follow W's by a step or so and hold them up
+// only if they fall two behind (the partial Grams alternate between two buffers) or
+// at the end.  They read the convergence measure but are not counted in the barrier.
+// An inner round 0.52 -> 0.44 us (64 columns).
 // !LOCAL: items are strided over the grid, with two grid barriers per step.
-template <bool LOCAL>
+template <bool LOCAL, bool VSEP>
 __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double tol,
                                                  int max_sweeps) {
   __shared__ PairLds L;
@@ -861,11 +912,13 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
   const int64_t steps = s.nb - 1;
   const int inner_sweeps = inner_sweeps_of(s);
   const double tiny2 = w.ctrl->tiny2;
+  const int64_t RA = s.R + (VSEP ? s.VS : 0);  // workgroups of a pair
   const size_t part_stride = (size_t)s.P * RMAX * PW * PW;
   unsigned int* pair_ctr = w.sync;
   unsigned int* chunk_ctr = w.sync + s.P;
   unsigned int barrier_no = 0;
-  const unsigned int G_ = gridDim.x;
+  const unsigned int G_ = LOCAL ? (unsigned int)items : gridDim.x;  // arrivals at the barrier
+  bool v_side = false;
   int sweep = 0;
   int converged = 0;
   double off_prev = 1.0e300;
@@ -883,32 +936,45 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
       if (prof) t0 = now_ticks();
       if (LOCAL) {
         int64_t p, r;
-        local_item(blockIdx.x, gridDim.x, s.R, &p, &r);
+        local_item(blockIdx.x, gridDim.x, RA, &p, &r);
+        v_side = VSEP && r >= s.R;
         int64_t bi, bj;
         pair_blocks(s.nb, k, p, &bi, &bj);
         if (g > 0) {
           const int64_t kp = (k == 0) ? steps - 1 : k - 1;
           const int64_t oi = block_owner(s.nb, kp, bi), oj = block_owner(s.nb, kp, bj);
-          if (!wait_counters(w.ctrl, &chunk_ctr[oi * s.R + r], &chunk_ctr[oj * s.R + r],
-                             (unsigned int)g, &L.flag))
-            goto aborted;
+          // (VSEP) and V's chunks have read the partial Grams of step g - 2
+          const bool ok =
+              VSEP ? wait_step(w.ctrl, chunk_ctr, oi * RA + r, oj * RA + r, (unsigned int)g,
+                               p * RA + s.R, v_side ? 0 : s.VS, (unsigned int)(g - 1), &L.flag)
+                   : wait_counters(w.ctrl, &chunk_ctr[oi * RA + r], &chunk_ctr[oj * RA + r],
+                                   (unsigned int)g, &L.flag);
+          if (!ok) goto aborted;
         }
         if (prof) {
           const long long t1 = now_ticks();
           pt[5] += t1 - t0;
           t0 = t1;
         }
-        partial_gram(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
-                     part + (p * RMAX + r) * PW * PW, L);
+        if (v_side) {
+          const int64_t v0 = (r - s.R) * RT;
+          load_tile(w.V, s.ncolp, bi, bj, v0, (int)min((int64_t)RT, s.ncolp - v0), L.tile[0]);
+        } else {
+          partial_gram<VSEP>(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
+                             part + (p * RMAX + r) * PW * PW, L);
+        }
         if (prof) {
           const long long t1 = now_ticks();
           pt[0] += t1 - t0;
           t0 = t1;
         }
         if (s.R > 1) {
-          signal_add(&pair_ctr[p]);
+          if (!v_side) signal_add(&pair_ctr[p]);
           if (!wait_counters(w.ctrl, &pair_ctr[p], nullptr, (unsigned int)((g + 1) * s.R),
                              &L.flag))
+            goto aborted;
+        } else if (VSEP && v_side) {  // the only chunk of W does not stop to publish its Gram matrix
+          if (!wait_counters(w.ctrl, &chunk_ctr[p * RA], nullptr, (unsigned int)(g + 1), &L.flag))
             goto aborted;
         }
         if (prof) {
@@ -916,16 +982,16 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           pt[1] += t1 - t0;
           t0 = t1;
         }
-        pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                    inner_sweeps, cross, L, prof, pt, &t0);
-        signal_set(&chunk_ctr[p * s.R + r], (unsigned int)(g + 1));
+        pair_update<VSEP>(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
+                          inner_sweeps, cross, L, prof, pt, &t0);
+        signal_set(&chunk_ctr[p * RA + r], (unsigned int)(g + 1));
       } else {
         for (int64_t it = blockIdx.x; it < items && s.R > 1; it += G_) {
           const int64_t p = it / s.R, r = it % s.R;
           int64_t bi, bj;
           pair_blocks(s.nb, k, p, &bi, &bj);
-          partial_gram(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
-                       part + (p * RMAX + r) * PW * PW, L);
+          partial_gram<false>(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc),
+                              part + (p * RMAX + r) * PW * PW, L);
         }
         if (prof) {
           const long long t1 = now_ticks();
@@ -945,16 +1011,23 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           // the chunk's last tile (and, R = 1, its Gram matrix) again: L has
           // held other items since
           reload(s, w, bi, bj, r, r * rc, min(s.len, r * rc + rc), L);
-          pair_update(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
-                      inner_sweeps, cross, L, prof, pt, &t0);
+          pair_update<false>(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
+                             inner_sweeps, cross, L, prof, pt, &t0);
         }
         if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
         if (prof) pt[5] += now_ticks() - t0;
       }
     }
     if (LOCAL) {
-      // all pairs' measures of this sweep are in *off_slot after the barrier
-      if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
+      // all pairs' measures of this sweep are in *off_slot after the barrier.  Slot
+      // (sweep + 1) % 3 is not reset before V's workgroups have read sweep - 2's: at the
+      // end of sweep - 1 they had all finished its first step (steps >= 3).
+      ++barrier_no;
+      if (v_side) {
+        if (!wait_counters(w.ctrl, &w.ctrl->barrier, nullptr, barrier_no * G_, &L.flag)) goto aborted;
+      } else if (!grid_barrier(w.ctrl, barrier_no * G_, &L.flag)) {
+        goto aborted;
+      }
     }
     {
       const unsigned long long bits =
@@ -1217,7 +1290,7 @@ int cooperative_grid(int64_t items, int* grid) {
   if (occ_dev != di.device) {
     int o = 0;
     SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &o, (const void*)svd_jacobi<true>, JT, 0));
+        &o, (const void*)svd_jacobi<true, false>, JT, 0));
     occ = o;
     occ_dev = di.device;
   }
@@ -1264,6 +1337,12 @@ void jacobi_shape(SvdShape* s, int num_cu) {
   if (R > RMAX) R = RMAX;
   if (R < 1) R = 1;
   s->R = R;
+  // V's rows to workgroups of their own as long as all of them take a quarter of the
+  // CUs (256 columns); with more, the waits between them cost what the shorter rounds
+  // give.  A square matrix, us, V apart / along with W: 64 columns 653 / 680, 128
+  // 1549 / 1707, 256 3640 / 3842, 320 5674 / 5667, 416 8378 / 8158, 512 9976 / 9237.
+  const int64_t vs = ceil_div(s->ncolp, RT);
+  s->VS = nb > 2 && 4 * s->P * (R + vs) <= num_cu ? vs : 0;
   // Inner solves: every block's own pairs are visited at the first step of a
   // sweep (each block meets one partner there); with cross_inner the later
   // steps rotate only the pairs across the two blocks (16 rounds instead of
@@ -1282,9 +1361,15 @@ void jacobi_shape(SvdShape* s, int num_cu) {
   s->cross_inner = s->nb > 2 ? inner_mode : 0;
 }
 
-int jacobi_enqueue(const SvdShape& s, const SvdWork& w, hipStream_t stream) {
+int jacobi_enqueue(const SvdShape& shape, const SvdWork& w, hipStream_t stream) {
+  SvdShape s = shape;
   int st, grid = 1;
-  if ((st = cooperative_grid(s.P * s.R, &grid))) return st;
+  if (!w.V) s.VS = 0;
+  if ((st = cooperative_grid(s.P * (s.R + s.VS), &grid))) return st;
+  if (grid < s.P * (s.R + s.VS)) {
+    s.VS = 0;
+    if ((st = cooperative_grid(s.P * s.R, &grid))) return st;
+  }
   // Relative orthogonality target: a few times above the rounding floor of the
   // measured Gram entries (~sqrt(len) eps), so that rounding alone cannot keep
   // the measure above it.
@@ -1295,7 +1380,9 @@ int jacobi_enqueue(const SvdShape& s, const SvdWork& w, hipStream_t stream) {
   const double M_ = (double)s.lenA, N_ = (double)s.ncol;
   TimedLaunch timed("svd_jacobi", stream, 4.0 * (6.0 * M_ * N_ * N_ + 16.0 * N_ * N_ * N_));
   // one work item per workgroup when they all fit: local step ordering
-  const void* fn = grid == s.P * s.R ? (const void*)svd_jacobi<true> : (const void*)svd_jacobi<false>;
+  const void* fn = grid < s.P * s.R ? (const void*)svd_jacobi<false, false>
+                   : s.VS > 0        ? (const void*)svd_jacobi<true, true>
+                                     : (const void*)svd_jacobi<true, false>;
   if (grid == 1) {  // nothing to be resident with
     SEEMPS_HIP(hipLaunchKernel(fn, dim3(1), dim3(JT), args, 0, stream));
     return SEEMPS_OK;

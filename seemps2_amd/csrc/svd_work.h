@@ -29,7 +29,8 @@ struct SvdShape {
   int64_t lenA, ncol;   // working matrix B: ncol columns of length lenA
   int64_t len;          // Jacobi column length (ncol with QR, lenA without)
   int64_t nb, ncolp;    // blocks (even), padded column count
-  int64_t P, R;         // pairs per step, row chunks
+  int64_t P, R;         // pairs per step, row chunks of W
+  int64_t VS;           // row chunks of V with workgroups of their own (0: W's rotate V too)
   int transposed;       // 1 if B = A^H
   int use_qr;
   int cross_inner;      // inner solves after a sweep's first step: cross-block pairs only
@@ -43,7 +44,7 @@ struct SvdWork {
   double2* W;     // ncolp x len
   double2* V;     // ncolp x ncolp
   double2* part;  // 2 x P x RMAX x PW x PW (partial Grams, by step parity)
-  unsigned int* sync;  // P pair arrival counters, then P x R chunk step counters
+  unsigned int* sync;  // P pair arrival counters, then P x (R + VS) chunk step counters
   double* colnrm;  // ncol squared column norms of B (QR path)
   int* colperm;    // ncol: B's columns by decreasing norm (QR path)
   double* sigma;  // ncolp
@@ -51,6 +52,7 @@ struct SvdWork {
   Ctrl* ctrl;
 };
 
+__host__ __device__ inline int64_t sync_words(const SvdShape& s) { return s.P + s.P * (s.R + s.VS); }
 inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 // Blocks, pairs and row chunks of a Jacobi on s.ncol columns of length s.len

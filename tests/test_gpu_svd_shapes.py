@@ -84,3 +84,25 @@ def test_svd_beyond_the_register_tiles(K, n):
     assert rel((U * S) @ VH, A) < tol
     assert np.abs(U.conj().T @ U - np.eye(n)).max() < tol
     assert np.abs(VH @ VH.conj().T - np.eye(n)).max() < tol
+
+
+# V's rows on workgroups of their own: one and more row chunks, a last partial chunk,
+# the last size that has them and the first that has not; all pairs, no pair and only
+# some pairs to rotate
+@pytest.mark.parametrize("n", [49, 64, 65, 129, 200, 256, 257, 272])
+@pytest.mark.parametrize("kind", ["full", "diagonal", "rank"])
+def test_svd_v_apart(K, n, kind):
+    rng = np.random.default_rng(n)
+    if kind == "diagonal":
+        A = np.diag(np.linspace(1.0, 2.0, n)[rng.permutation(n)]) + 0j
+    else:
+        r = n if kind == "full" else n // 3
+        A = crandn(rng, n, r) * np.exp(-20.0 / r * np.arange(r)) @ crandn(rng, r, n)
+        A /= np.linalg.norm(A)
+    U, S, VH = K.svd(K.as_dev(A))
+    U, S, VH = K.to_numpy(U), S.cpu().numpy(), K.to_numpy(VH)
+    assert rel((U * S) @ VH, A) < 1e-12
+    assert np.abs(U.conj().T @ U - np.eye(n)).max() < 1e-12
+    assert np.abs(VH @ VH.conj().T - np.eye(n)).max() < 1e-12
+    s_ref = np.linalg.svd(A, compute_uv=False)
+    assert np.abs(S - s_ref).max() < 5e-13 * s_ref[0]
