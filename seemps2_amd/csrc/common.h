@@ -130,6 +130,8 @@ int zgemm(int opA, int opB, int64_t M, int64_t N, int64_t K, double2 alpha, cons
           int prec = SEEMPS_PREC_FP64);
 // Split-K GEMM over caller scratch (ws holds splitk_workspace(M, N, K) elements);
 // falls back to zgemm when splitting does not pay or ws is too small.
+// Whether an FP64 product runs on 16 x 16 tiles of four wavefronts each.
+bool gemm_on_small_tiles(int opA, int opB, int64_t M, int64_t N, int64_t K);
 int zgemm_ws(int opA, int opB, int64_t M, int64_t N, int64_t K, double2 alpha, const void* A,
              int64_t lda, const void* B, int64_t ldb, double2 beta, void* C, int64_t ldc,
              double2* ws, int64_t ws_elems, hipStream_t stream, int prec = SEEMPS_PREC_FP64);

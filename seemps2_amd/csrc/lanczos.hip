@@ -8,6 +8,7 @@
 #include <cmath>
 
 #include "common.h"
+#include "gemm_direct.h"
 #include "jacobi_inner.h"
 #include "wave.h"
 
@@ -70,11 +71,13 @@ struct LzScalars {
 constexpr int LZ_KREG = 24;
 constexpr int LZ_THREADS = 256;
 
+constexpr int LZ_BLOCKS = 256;
+
 // Blocks of the orthogonalisation launches: an element per thread up to one
 // block per CU, so that a short vector is spread over as many CUs as it can use.
 inline int lz_blocks(int64_t n) {
   int64_t b = ceil_div(n, (int64_t)LZ_THREADS);
-  if (b > 256) b = 256;
+  if (b > LZ_BLOCKS) b = LZ_BLOCKS;
   if (b < 1) b = 1;
   return (int)b;
 }
@@ -188,12 +191,41 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth1(int64_t n, int k,
   lz_store_partials<KR>(acc, k, nrm, part, pn0);
 }
 
-// Pass 2: h = sum of pass-1 partials (h_{k-1} is kept); w -= V h; then the
+// Pass 1 in the last product of H v, out = x2 R^T on 16 x 16 tiles: a thread of the
+// finished tile holds one element of w, as in lz_orth1, and a tile stands for a
+// block.  Saves the launch and the reading of w: at n = 36864 the product and the
+// pass took 5.7 + 3.8 us, together 7.3.
+template <int KR>
+__global__ __launch_bounds__(LZ_THREADS) void lz_product_dots(
+    int64_t M, int64_t N, int64_t K, const double2* __restrict__ x2, const double2* __restrict__ R,
+    double2* __restrict__ w, int k, const double2* __restrict__ V, double2* __restrict__ part,
+    double* __restrict__ pn0) {
+  extern __shared__ double2 lds[];
+  const int64_t tiles_n = ceil_div(N, (int64_t)16);
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double2 x = make_double2(0.0, 0.0);
+  int64_t i = 0;
+  direct::tile<SEEMPS_OP_N, SEEMPS_OP_T, 1, 4, true>(
+      M, N, K, x2, K, R, K, tile / tiles_n * 16, tile % tiles_n * 16, wv, lds,
+      [&](int64_t m, int64_t n, double2 out) {
+        i = m * N + n;
+        x = out;
+        w[i] = x;
+      });
+  double2 v[KR], acc[KR];
+  lz_column<KR>(M * N, k, i, V, v);
+#pragma unroll
+  for (int j = 0; j < KR; ++j) acc[j] = cmulc(v[j], x);
+  lz_store_partials<KR>(acc, k, cabs2(x), part, pn0);
+}
+
+// Pass 2: h = sum of the nb_in pass-1 partials (h_{k-1} is kept); w -= V h; then the
 // block sums of conj(V_j) w (part_out) and |w|^2 (pn1) of the updated w.
 template <int KR>
 __global__ __launch_bounds__(LZ_THREADS) void lz_orth2(int64_t n, int k,
                                                        const double2* __restrict__ V,
-                                                       double2* __restrict__ w,
+                                                       double2* __restrict__ w, int nb_in,
                                                        const double2* __restrict__ part_in,
                                                        double2* __restrict__ part_out,
                                                        double* __restrict__ pn1,
@@ -205,7 +237,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth2(int64_t n, int k,
   lz_column<KR>(n, k, min(i, n - 1), V, v);
   if (threadIdx.x < LZ_KREG) hs[threadIdx.x] = make_double2(0.0, 0.0);
   __syncthreads();
-  lz_load_coeffs(k, gridDim.x, part_in, hs);
+  lz_load_coeffs(k, nb_in, part_in, hs);
   __syncthreads();
   if (blockIdx.x == 0 && threadIdx.x == 0) s->h = hs[k - 1];
   double2 acc[KR];
@@ -350,7 +382,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
                                                        const double2* __restrict__ V,
                                                        double2* __restrict__ w,
                                                        const double2* __restrict__ part_in,
-                                                       const double* __restrict__ pn0,
+                                                       int nb0, const double* __restrict__ pn0,
                                                        const double* __restrict__ pn1,
                                                        LzScalars* __restrict__ s, uint64_t ritz,
                                                        double* __restrict__ out) {
@@ -365,7 +397,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
   const double prev = j > 0 ? s->beta[j - 1] : 0.0, scale_prev = j > 0 ? s->scl[j - 1] : 0.0;
   const int brk_prev = j > 0 ? s->brk[j - 1] : 0;
   const int kd_prev = s->kd;
-  const double n0 = lz_wave_sum(nb, pn0), n1 = lz_wave_sum(nb, pn1);
+  const double n0 = lz_wave_sum(nb0, pn0), n1 = lz_wave_sum(nb, pn1);
   if (threadIdx.x < LZ_KREG) hs[threadIdx.x] = make_double2(0.0, 0.0);
   __syncthreads();
   const bool second = !(n1 >= 0.5 * n0);
@@ -509,9 +541,9 @@ int64_t eig_bytes_full(int64_t chiL, int64_t c, int64_t d1, int64_t d2, int64_t 
   b += al256((m + 1) * n * 16);
   b += al256(chiL * c * d1 * d2 * chiR * 16);
   b += al256(chiL * d1 * d2 * w2 * chiR * 16);
-  b += al256(LZ_KREG * lz_blocks(n) * 16);
-  b += al256(LZ_KREG * lz_blocks(n) * 16);
-  b += al256(2 * lz_blocks(n) * 8);
+  b += al256(LZ_KREG * LZ_BLOCKS * 16);
+  b += al256(LZ_KREG * LZ_BLOCKS * 16);
+  b += al256(2 * LZ_BLOCKS * 8);
   b += al256(matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR) * 16);
   b += al256(sizeof(LzScalars));
   return b;
@@ -529,11 +561,11 @@ EigWork eig_carve(void* work, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   w.x2 = (double2*)p;
   p += al256(chiL * d1 * d2 * w2 * chiR * 16);
   w.part = (double2*)p;
-  p += al256(LZ_KREG * lz_blocks(n) * 16);
+  p += al256(LZ_KREG * LZ_BLOCKS * 16);
   w.part2 = (double2*)p;
-  p += al256(LZ_KREG * lz_blocks(n) * 16);
+  p += al256(LZ_KREG * LZ_BLOCKS * 16);
   w.pnorm = (double*)p;
-  p += al256(2 * lz_blocks(n) * 8);
+  p += al256(2 * LZ_BLOCKS * 8);
   w.ks = (double2*)p;
   p += al256(matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR) * 16);
   w.sc = (LzScalars*)p;
@@ -549,6 +581,21 @@ unsigned grid_for(int64_t n) {
 
 }  // namespace
 
+// x2[a, ko, lo, d, f] = sum L[a,c,b] Hm[(c,k,l),(ko,lo,d)] v[b,k,l,f]
+static int two_site_half(int64_t a, int64_t c, int64_t b, int64_t d1, int64_t d2, int64_t w2,
+                         int64_t f, const double2* L, const double2* Hm, const double2* v,
+                         double2* x1, double2* x2, double2* ks, int64_t ks_elems,
+                         hipStream_t stream, int prec) {
+  int st;
+  // x1[(a,c), (k,l,f)] = L[(a,c), b] v[b, (k,l,f)]
+  if ((st = zgemm_ws(SEEMPS_OP_N, SEEMPS_OP_N, a * c, d1 * d2 * f, b, make_double2(1.0, 0.0), L, b,
+                     v, d1 * d2 * f, make_double2(0.0, 0.0), x1, d1 * d2 * f, ks, ks_elems, stream,
+                     prec)))
+    return st;
+  // x2[a, (ko,lo,d), f] = sum_{(c,k,l)} x1[a, (c,k,l), f] Hm[(c,k,l), (ko,lo,d)]
+  return zlocal_impl(a, c * d1 * d2, f, d1 * d2 * w2, 1, x1, Hm, x2, 0, stream);
+}
+
 // out[a, ko, lo, g] = sum L[a,c,b] Hm[(c,k,l),(ko,lo,d)] v[b,k,l,f] R[g,d,f]
 int two_site_matvec_impl(int64_t a, int64_t c, int64_t b, int64_t d1, int64_t d2, int64_t w2,
                          int64_t f, int64_t g, const double2* L, const double2* Hm,
@@ -557,12 +604,8 @@ int two_site_matvec_impl(int64_t a, int64_t c, int64_t b, int64_t d1, int64_t d2
                          int prec) {
   int st;
   const double2 one = make_double2(1.0, 0.0), zero = make_double2(0.0, 0.0);
-  // x1[(a,c), (k,l,f)] = L[(a,c), b] v[b, (k,l,f)]
-  if ((st = zgemm_ws(SEEMPS_OP_N, SEEMPS_OP_N, a * c, d1 * d2 * f, b, one, L, b, v, d1 * d2 * f,
-                     zero, x1, d1 * d2 * f, ks, ks_elems, stream, prec)))
+  if ((st = two_site_half(a, c, b, d1, d2, w2, f, L, Hm, v, x1, x2, ks, ks_elems, stream, prec)))
     return st;
-  // x2[a, (ko,lo,d), f] = sum_{(c,k,l)} x1[a, (c,k,l), f] Hm[(c,k,l), (ko,lo,d)]
-  if ((st = zlocal_impl(a, c * d1 * d2, f, d1 * d2 * w2, 1, x1, Hm, x2, 0, stream))) return st;
   // out[(a,ko,lo), g] = x2[(a,ko,lo), (d,f)] R[g, (d,f)]^T
   return zgemm_ws(SEEMPS_OP_N, SEEMPS_OP_T, a * d1 * d2, g, w2 * f, one, x2, w2 * f, R, w2 * f,
                   zero, out, g, ks, ks_elems, stream, prec);
@@ -639,35 +682,56 @@ extern "C" int64_t seemps_eigensolve_workspace(int64_t chiL, int64_t c, int64_t 
 
 namespace {
 
-// Orthogonalisation of wv = H V[k-1] against V[0..k), its norm and scalars.
+// The last product of wv = H V[k-1] (x2 in w.x2), its orthogonalisation against
+// V[0..k), norm and scalars.
+struct LzProduct {
+  int64_t M, N, K;
+  const double2* R;
+  int prec;
+  int64_t ks_elems;
+};
+
 template <int KR>
-void lz_step_kr(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
-                uint64_t ritz, double* out, hipStream_t s) {
+int lz_step_kr(const LzProduct& pr, int k, int nb, const EigWork& w, double2* wv, double* pn0,
+               double* pn1, uint64_t ritz, double* out, hipStream_t s) {
+  const int64_t n = pr.M * pr.N, tiles = ceil_div(pr.M, (int64_t)16) * ceil_div(pr.N, (int64_t)16);
   const double orth = 8.0 * n * k;
-  {
+  int nb_in = nb;
+  if (pr.prec == SEEMPS_PREC_FP64 && tiles <= LZ_BLOCKS &&
+      gemm_on_small_tiles(SEEMPS_OP_N, SEEMPS_OP_T, pr.M, pr.N, pr.K)) {
+    nb_in = (int)tiles;
+    TimedLaunch timed("lz_product_dots", s, 8.0 * n * pr.K + orth);
+    hipLaunchKernelGGL(lz_product_dots<KR>, dim3(nb_in), dim3(LZ_THREADS), 4 * 4 * 64 * 16, s,
+                       pr.M, pr.N, pr.K, w.x2, pr.R, wv, k, w.V, w.part, pn0);
+  } else {
+    const int st = zgemm_ws(SEEMPS_OP_N, SEEMPS_OP_T, pr.M, pr.N, pr.K, make_double2(1.0, 0.0),
+                            w.x2, pr.K, pr.R, pr.K, make_double2(0.0, 0.0), wv, pr.N, w.ks,
+                            pr.ks_elems, s, pr.prec);
+    if (st) return st;
     TimedLaunch timed("lz_orth1", s, orth);
     hipLaunchKernelGGL(lz_orth1<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part,
                        pn0);
   }
   {
     TimedLaunch timed("lz_orth2", s, 2.0 * orth);
-    hipLaunchKernelGGL(lz_orth2<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part,
-                       w.part2, pn1, w.sc);
+    hipLaunchKernelGGL(lz_orth2<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, nb_in,
+                       w.part, w.part2, pn1, w.sc);
   }
   TimedLaunch timed("lz_orth3", s, orth);
-  hipLaunchKernelGGL(lz_orth3<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part2, pn0,
-                     pn1, w.sc, ritz, out);
+  hipLaunchKernelGGL(lz_orth3<KR>, dim3(nb), dim3(LZ_THREADS), 0, s, n, k, w.V, wv, w.part2, nb_in,
+                     pn0, pn1, w.sc, ritz, out);
+  return check_launch("lanczos step");
 }
 
-void lz_step(int64_t n, int k, int nb, const EigWork& w, double2* wv, double* pn0, double* pn1,
-             uint64_t ritz, double* out, hipStream_t s) {
+int lz_step(const LzProduct& pr, int k, int nb, const EigWork& w, double2* wv, double* pn0,
+            double* pn1, uint64_t ritz, double* out, hipStream_t s) {
   switch ((k + 3) / 4) {
-    case 1: return lz_step_kr<4>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
-    case 2: return lz_step_kr<8>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
-    case 3: return lz_step_kr<12>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
-    case 4: return lz_step_kr<16>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
-    case 5: return lz_step_kr<20>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
-    default: return lz_step_kr<24>(n, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 1: return lz_step_kr<4>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 2: return lz_step_kr<8>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 3: return lz_step_kr<12>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 4: return lz_step_kr<16>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    case 5: return lz_step_kr<20>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
+    default: return lz_step_kr<24>(pr, k, nb, w, wv, pn0, pn1, ritz, out, s);
   }
 }
 
@@ -694,9 +758,10 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   const double2* H_ = (const double2*)Hm;
   const double2* R_ = (const double2*)R;
   const int nbk = lz_blocks(n);
+  const int64_t ks_elems = matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR);
   int st;
   double* pn0 = w.pnorm;
-  double* pn1 = w.pnorm + nbk;
+  double* pn1 = w.pnorm + LZ_BLOCKS;
   // V[0] = v0 / ||v0||
   hipLaunchKernelGGL(lz_combine, dim3(nbk), dim3(LZ_THREADS), 0, st_, n, 0, (double2*)v0,
                      w.sc->y, pn0);
@@ -733,10 +798,8 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
     for (int64_t j = 0; j < m; ++j) {
       double2* vj = w.V + j * n;
       double2* wv = w.V + (j + 1) * n;
-      if ((st = two_site_matvec_impl(chiL, c, chiL, d1, d2, w2, chiR, chiR, L_, H_, R_, vj, wv,
-                                     w.x1, w.x2, w.ks,
-                                     matvec_ks_elems(chiL, c, chiL, d1, d2, w2, chiR, chiR),
-                                     st_, mv_prec)))
+      if ((st = two_site_half(chiL, c, chiL, d1, d2, w2, chiR, L_, H_, vj, w.x1, w.x2, w.ks,
+                              ks_elems, st_, mv_prec)))
         return st;
       ++matvecs;
       if (mv_prec == SEEMPS_PREC_FP32) ++matvecs32;
@@ -745,8 +808,10 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
       const bool check = early && mv_prec == SEEMPS_PREC_FP64 && kd < m && kd >= first_check &&
                          (kd - first_check) % check_every == 0;
       if (check || kd == m) ticket = next_ticket();
-      lz_step(n, (int)kd, nbk, w, wv, pn0, pn1, check || kd == m ? ticket : 0, hp_dev, st_);
-      if ((st = check_launch("lanczos step"))) return st;
+      const LzProduct last{chiL * d1 * d2, chiR, w2 * chiR, R_, mv_prec, ks_elems};
+      if ((st = lz_step(last, (int)kd, nbk, w, wv, pn0, pn1, check || kd == m ? ticket : 0, hp_dev,
+                        st_)))
+        return st;
       if (prec == SEEMPS_PREC_MIXED && cycle == 0 && j == 0) {
         double* ab = hp + 2;
         SEEMPS_HIP(hipMemcpyAsync(&ab[0], &w.sc->alpha[0], 8, hipMemcpyDeviceToHost, st_));

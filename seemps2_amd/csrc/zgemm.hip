@@ -499,6 +499,13 @@ int dispatch(int prec, int opA, int opB, int64_t batch, hipStream_t stream, int6
 
 }  // namespace
 
+bool gemm_on_small_tiles(int opA, int opB, int64_t M, int64_t N, int64_t K) {
+  DeviceInfo info;
+  if (device_info(&info)) return false;
+  const Direct d = choose_direct(opA, opB, M, N, K, info.num_cu);
+  return d.F == 1 && d.KS == 4;
+}
+
 // Number of K slices zgemm_ws uses for (M, N, K) (1 = no split).
 int64_t splitk_slices(int64_t M, int64_t N, int64_t K) {
   // tuning knob: tile count from which no split is made (SEEMPS_SPLITK_TILES);
