@@ -165,8 +165,10 @@ __device__ __forceinline__ void lz_column(int64_t n, int k, int64_t i,
 // last-level cache.  So a thread takes one element and asks for all its basis
 // entries at once (KR >= k of them, a multiple of four, in registers; testing
 // j < k load by load serialises them), sums go through DPP, and partials lie so
-// that blocks read them back coalesced.  n = 36864, k <= 20: 38 us a step in
-// four launches of four elements a thread -> LZ_TIME.
+// that blocks read them back coalesced.  A step at n = 36864, averaged over k = 1..20:
+// 46.6 us in four launches of four elements a thread and a fifth for the Ritz pair of
+// some steps, now 15.7 (passes 3.8, 5.1 and 6.8), and 13.5 with the first pass in the
+// last product of H v.
 //
 // Pass 1: part = block sums of conj(V_j) w; pn0 = block sums of |w|^2.
 template <int KR>

@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256, tile_occupancy(TM, TN, G3)) void zgemm_kernel(
 // limits products of few tiles is the chain of staging and barriers that this leaves
 // out: 64^3 5.6 -> 3.1 us (a launch is 2.2), 256 x 400 x 200 15.2 -> 7.0.  Of large
 // ones the loads are the limit of 16 x 16 tiles, the matrix cores that of 32 x 32
-// (2048 x 2048 x 512 at 75 TFLOP/s, a large library product at 72).
+// (1024 x 2048 x 2048 at 78 TFLOP/s, a large library product at 72).
 template <int OPA, int OPB, int F, int KS>
 __global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, int64_t K,
                                                         double2 alpha,
@@ -330,6 +330,18 @@ __global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, in
       });
 }
 
+// SEEMPS_GEMM_TILE = 64x64 or 32x32 fixes the staged tile (a tuning knob); else -1.
+int forced_tile() {
+  static const int forced = [] {
+    const char* e = getenv("SEEMPS_GEMM_TILE");
+    if (!e) return -1;
+    if (!strcmp(e, "64x64")) return (int)TILE_64x64;
+    if (!strcmp(e, "32x32")) return (int)TILE_32x32;
+    return -1;
+  }();
+  return forced;
+}
+
 // Tile shape for an M x N output in `batch` slices on `num_cu` CUs.  The
 // 64 x 64 tile (three workgroups per CU) is the faster one per output element
 // once every CU holds four or more of them; below that the 32 x 32 tile (five
@@ -338,16 +350,8 @@ __global__ __launch_bounds__(64 * KS) void zgemm_direct(int64_t M, int64_t N, in
 // the LDS and memory latencies.  Measured with four products on the matvec
 // and environment GEMMs of chi = 128 and 256 (25-35 % faster with the small
 // tile) and on a 2048 x 2048 x 512 product (6 % slower with it).
-// SEEMPS_GEMM_TILE = 64x64 or 32x32 fixes the shape (a tuning knob).
 int choose_tile(int64_t M, int64_t N, int64_t batch, int num_cu) {
-  static const int forced = [] {
-    const char* e = getenv("SEEMPS_GEMM_TILE");
-    if (!e) return -1;
-    if (!strcmp(e, "64x64")) return (int)TILE_64x64;
-    if (!strcmp(e, "32x32")) return (int)TILE_32x32;
-    return -1;
-  }();
-  if (forced >= 0) return forced;
+  if (forced_tile() >= 0) return forced_tile();
   const int64_t cu = num_cu > 0 ? num_cu : 256;
   const int64_t tiles64 = ceil_div(M, 64) * ceil_div(N, 64) * batch;
   return tiles64 >= 4 * cu ? TILE_64x64 : TILE_32x32;
@@ -374,10 +378,12 @@ bool gemm_scheme_3m() {
 //   1280 512 256 (640)         36.9   30.0   28.4   36.1
 //   512 512 512 (256)          27.8   22.3   22.2   54.7
 //   1024 1024 1024 (1024)     142.8  176.0  121.4  123.0
-//   2048 2048 512 (4096)      280.1  330.6  233.6  228.3
+//   1024 2048 2048 (2048)     514.5  661.2  437.8  443.0
 //   1500 1100 300 (1645)       74.8   78.9   71.0   69.9
 //   1024 1024 64 (1024)        13.4   16.4   14.8   14.8
 //   1280 1024 256 (1280)       49.3   58.7   51.1   58.7
+// (Outputs of four 64 x 64 tiles a CU keep that tile and its four real products:
+// 2048 2048 512 takes 280.1 there against 228.3 with three.)
 // Few tiles: 16 x 16 ones for four times the waves.  From a tile for each CU:
 // 32 x 32 ones, which ask half the loads, where whole rounds of the CUs come out
 // at least four fifths full, and one wave a tile once every SIMD has its own.
@@ -397,8 +403,8 @@ bool rows_in_k(int opA, int opB) {
 }
 
 Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_cu) {
-  static const bool off = getenv("SEEMPS_GEMM_TILE") != nullptr;  // the knob names staged tiles
-  if (off || !gemm_scheme_3m()) return {0, 0};
+  if (forced_tile() >= 0 || !gemm_scheme_3m()) return {0, 0};
+  if (choose_tile(M, N, 1, num_cu) == TILE_64x64) return {0, 0};  // four products
   const int64_t cu = num_cu > 0 ? num_cu : 256, simd = 4 * cu;
   const int64_t t = ceil_div(M, 32) * ceil_div(N, 32);
   auto full = [&](int64_t units) { return 5 * t >= 4 * units * ceil_div(t, units); };
