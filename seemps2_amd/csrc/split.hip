@@ -67,7 +67,7 @@ struct SplitResult {
   int64_t D;
   double err;
   int tiny;                 // a kept singular value is negligible
-  int status[3];            // ctrl->info: sweeps, converged, aborted
+  int status[3];            // of the Jacobi: sweeps, converged, aborted
 };
 
 // Squared norms of the columns of B: of A's rows (adj, a wavefront each) ...
@@ -231,7 +231,9 @@ __global__ __launch_bounds__(1024) void sort_truncate(SvdShape s, SvdWork w, dou
   __syncthreads();
   if (tid == 0) {
     host->tiny = s_tiny;
-    for (int i = 0; i < 3; ++i) host->status[i] = w.ctrl->info[i];
+    host->status[0] = w.ctrl->info[0];
+    host->status[1] = w.ctrl->info[1];
+    host->status[2] = (int)w.ctrl->abort;
     host_publish(flag, ticket);
   }
 }

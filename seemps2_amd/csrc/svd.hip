@@ -949,7 +949,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
                                p * RA + s.R, v_side ? 0 : s.VS, (unsigned int)(g - 1), &L.flag)
                    : wait_counters(w.ctrl, &chunk_ctr[oi * RA + r], &chunk_ctr[oj * RA + r],
                                    (unsigned int)g, &L.flag);
-          if (!ok) goto aborted;
+          if (!ok) return;
         }
         if (prof) {
           const long long t1 = now_ticks();
@@ -972,10 +972,10 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           if (!v_side) signal_add(&pair_ctr[p]);
           if (!wait_counters(w.ctrl, &pair_ctr[p], nullptr, (unsigned int)((g + 1) * s.R),
                              &L.flag))
-            goto aborted;
+            return;
         } else if (VSEP && v_side) {  // the only chunk of W does not stop to publish its Gram matrix
           if (!wait_counters(w.ctrl, &chunk_ctr[p * RA], nullptr, (unsigned int)(g + 1), &L.flag))
-            goto aborted;
+            return;
         }
         if (prof) {
           const long long t1 = now_ticks();
@@ -998,7 +998,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           pt[0] += t1 - t0;
           t0 = t1;
         }
-        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
+        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) return;
         if (prof) {
           const long long t1 = now_ticks();
           pt[1] += t1 - t0;
@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
           pair_update<false>(s, w, bi, bj, r, part + p * RMAX * PW * PW, off_slot, tol, tiny2,
                              inner_sweeps, cross, L, prof, pt, &t0);
         }
-        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) goto aborted;
+        if (!grid_barrier(w.ctrl, (++barrier_no) * G_, &L.flag)) return;
         if (prof) pt[5] += now_ticks() - t0;
       }
     }
@@ -1024,9 +1024,9 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
       // end of sweep - 1 they had all finished its first step (steps >= 3).
       ++barrier_no;
       if (v_side) {
-        if (!wait_counters(w.ctrl, &w.ctrl->barrier, nullptr, barrier_no * G_, &L.flag)) goto aborted;
+        if (!wait_counters(w.ctrl, &w.ctrl->barrier, nullptr, barrier_no * G_, &L.flag)) return;
       } else if (!grid_barrier(w.ctrl, barrier_no * G_, &L.flag)) {
-        goto aborted;
+        return;
       }
     }
     {
@@ -1054,9 +1054,6 @@ __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double t
     w.ctrl->info[1] = converged;
     for (int i = 0; i < 6; ++i) w.ctrl->prof[i] = pt[i];
   }
-  return;
-aborted:
-  if (blockIdx.x == 0 && tid == 0) w.ctrl->info[2] = 1;
 }
 
 // sigma_c = ||w_c||.
@@ -1531,7 +1528,7 @@ int ctrl_status(const Ctrl& h, int32_t* info) {
     for (int i = 0; i < h.info[0] && i < 16; ++i) fprintf(stderr, " %.1e", h.offhist[i]);
     fprintf(stderr, "\n");
   }
-  if (h.info[2]) {
+  if (h.abort) {
     set_error("svd: grid barrier timed out (cooperative residency lost)");
     return SEEMPS_ERR_RUNTIME;
   }

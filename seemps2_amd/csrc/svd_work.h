@@ -15,9 +15,9 @@ constexpr int RMAX = 16;        // max row chunks per pair
 
 struct Ctrl {
   unsigned int barrier;       // grid barrier arrivals
-  unsigned int abort;         // set when a barrier wait timed out
+  unsigned int abort;         // set by any workgroup whose wait timed out
   unsigned long long off[3];  // per-sweep max normalised off-diagonal (as bits), slot sweep % 3
-  int info[4];                // sweeps, converged, aborted, unused
+  int info[4];                // sweeps, converged (written by workgroup 0), unused
   long long prof[8];          // wall-clock ticks of workgroup 0 per phase
   double frob2;               // ||W||_F^2 (invariant under the rotations)
   double tiny2;               // squared norm below which a column is negligible
@@ -73,6 +73,8 @@ __host__ __device__ inline double negligible2(int64_t len, double frob2) {
 int complete_enqueue(const SvdWork& w, double2* base, int64_t sk, int64_t sx, int conj, int64_t r,
                      int64_t len, const int64_t* kmax, hipStream_t stream);
 // Status and message of a finished Jacobi from a host copy of its control block.
+// `abort` decides over `info`: V's own workgroups are not counted in the last
+// barrier, so a wait of theirs may run out after workgroup 0 left as converged.
 int ctrl_status(const Ctrl& h, int32_t* info);
 
 // Truncation rule on the descending spectrum ss by one thread: the reference's
