@@ -29,24 +29,31 @@ namespace {
 
 struct Reflector {
   double beta;
-  double2 d, tau;  // alpha - beta, tau
+  double2 d, tau;  // (alpha - beta) up, tau
+  double up;       // v = up [alpha - beta; x]
   bool any;        // false: H = I
 };
 
-// A column of squared norm below 1e-300 (the squares lose their digits there)
-// gets no reflector; NaN does, and spreads.
+// In a column whose squares come near the smallest normal number, v is scaled up by
+// a power of two, so that tau (about 1 / |v|^2) stays finite.  NaN gets a reflector,
+// and spreads.
 __device__ __forceinline__ Reflector make_reflector(double2 alpha, double xnorm2) {
   Reflector h;
   h.beta = alpha.x;
   h.d = h.tau = make_double2(0.0, 0.0);
-  const double s = cabs2(alpha) + xnorm2;
-  h.any = !(xnorm2 == 0.0 && alpha.y == 0.0) && !(s < 1e-300);
+  double s = cabs2(alpha) + xnorm2;
+  h.any = !(xnorm2 == 0.0 && alpha.y == 0.0) && s != 0.0;
+  const bool tiny = s < 1e-290;
+  h.up = tiny ? 0x1p500 : 1.0;
   if (h.any) {
+    s = (s * h.up) * h.up;
+    alpha = make_double2(alpha.x * h.up, alpha.y * h.up);
     const double r = jac::rsqrt_nr(s), sg = (alpha.x >= 0.0) ? -1.0 : 1.0;
     h.beta = sg * (s * r);
     h.d = make_double2(alpha.x - h.beta, alpha.y);
     const double q = jac::rcp_nr(cabs2(h.d)), ib = -sg * r;  // 1 / |d|^2, -1 / beta
     h.tau = make_double2((h.d.x * ib) * q, (h.d.y * ib) * q);
+    h.beta *= tiny ? 0x1p-500 : 1.0;
   }
   return h;
 }
@@ -122,6 +129,12 @@ __global__ __launch_bounds__(64 * NW) void qr_panel(double2* __restrict__ A, int
           d[k] = wave::sum2(d[k]);
       }
       const Reflector h = make_reflector(alpha, nn);
+      if (h.up != 1.0) {
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) x[r] = make_double2(x[r].x * h.up, x[r].y * h.up);
+#pragma unroll
+        for (int k = 0; k < CPW; ++k) d[k] = make_double2(d[k].x * h.up, d[k].y * h.up);
+      }
 #pragma unroll
       for (int r = 0; r < RPT; ++r)
         if (lane + 64 * r == j) x[r] = h.d;  // x is v from here on
@@ -319,7 +332,9 @@ __global__ __launch_bounds__(1024) void qr_panel_long(double2* __restrict__ A, i
     const Reflector h = make_reflector(col[c], block_sum(acc, red).x);
     __syncthreads();  // every thread has read col[c]
     for (int64_t r = j0 + threadIdx.x; r < len; r += blockDim.x) {
-      v[r] = (r < c) ? make_double2(0.0, 0.0) : (r == c) ? h.d : col[r];
+      v[r] = (r < c)    ? make_double2(0.0, 0.0)
+             : (r == c) ? h.d
+                        : make_double2(col[r].x * h.up, col[r].y * h.up);
       if (r == c) col[r] = make_double2(h.beta, 0.0);
     }
     if (threadIdx.x == 0) tau[c] = h.tau;

@@ -106,3 +106,20 @@ def test_svd_v_apart(K, n, kind):
     assert np.abs(VH @ VH.conj().T - np.eye(n)).max() < 1e-12
     s_ref = np.linalg.svd(A, compute_uv=False)
     assert np.abs(S - s_ref).max() < 5e-13 * s_ref[0]
+
+
+# Column norms whose squares lie near the smallest normal number (1e-152 squared times a
+# few): register panels with and without trailing columns, a panel in memory, a column,
+# a rank of one.  The singular values of such a matrix are not resolved (the squares of
+# its Gram matrix underflow), its product is, to the bound of the chain above.
+@pytest.mark.parametrize("m,n,r", [(8, 1, 1), (2, 2, 1), (40, 30, 30), (30, 40, 30), (100, 100, 100),
+                                   (700, 20, 20), (1100, 20, 20)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_split_of_tiny_matrices(K, m, n, r, mode):
+    rng = np.random.default_rng(m + n)
+    A = crandn(rng, m, r) @ crandn(rng, r, n) / np.sqrt(r)
+    scale = 2.0 ** -505  # exact
+    Ad, Bd, D, _, _ = K.svd_split(K.as_dev(A * scale), m, n, mode, 0, 0.0, min(m, n))
+    out = K.to_numpy(Ad) @ K.to_numpy(Bd) / scale
+    assert D == min(m, n)
+    assert rel(out, A) < 1e-12
