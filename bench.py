@@ -268,8 +268,9 @@ def chosen_form_breakdown(trace_csv, top=15):
 PMC_COPY_ELEMS = 4096 * 4096   # complex128 elements of the calibration copy (256 MiB)
 PMC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                            "dmrg_chi256_pmc_traffic.md")
-PMC_KERNELS = ("zgemm_kernel", "polar_svd", "polar_persistent", "svd_jacobi", "zlocal_kernel",
-               "lz_orth1", "lz_orth2", "lz_orth3", "splitk_reduce")
+PMC_KERNELS = ("zgemm_kernel", "zgemm_direct", "grouped_zgemm_kernel", "splitk_reduce",
+               "polar_persistent", "svd_jacobi", "qr_panel", "qr_reflect", "zlocal_kernel",
+               "lz_product_dots", "lz_orth1", "lz_orth2", "lz_orth3")
 
 
 def pmc_workload(QF, H, strategy, chi, direction):
@@ -467,7 +468,8 @@ def pmc_mfma(directory):
 
 
 # library timing names whose launches appear under another name in rocprof
-ROCPROF_NAMES = {"polar_svd": "polar_persistent"}
+ROCPROF_NAMES = {"polar_svd": "polar_persistent", "zgemm_kernel_fp32": "zgemm_kernel",
+                 "grouped_zgemm": "grouped_zgemm_kernel"}
 
 
 STATS_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
@@ -577,10 +579,11 @@ def timed_sweeps(QF, strategy, direction, steps, chi, precision="fp64"):
 
 
 # HIP-event timing inside the timed sweeps: the candidates for the dominant
-# kernel of either form (the complex GEMM, the rotation-iteration SVD of the
+# kernel of either form (the complex GEMMs, staged, direct and with the
+# Gram-Schmidt dots of the Lanczos step, the rotation-iteration SVD of the
 # sketched splits, the block Jacobi SVD of the full splits); --kernel-timing
 # times others, e.g. "*" for every instrumented launch
-TIMED_KERNELS = "zgemm_kernel,polar_svd,svd_jacobi"
+TIMED_KERNELS = "zgemm_kernel,zgemm_direct,lz_product_dots,polar_svd,svd_jacobi"
 METRIC = "two-site bond updates/s at chi=256; speedup vs plain FP64 GPU at <=1e-9 rel err"
 
 

@@ -482,8 +482,10 @@ int dispatch(int prec, int opA, int opB, int64_t batch, hipStream_t stream, int6
   // the tile index runs along grid.x (at most 2^31 - 1 workgroups)
   SEEMPS_CHECK_ARG(ceil_div(M, 32) * ceil_div(N, 32) < (int64_t)INT32_MAX,
                    "zgemm: output too large");
-  TimedLaunch timed(prec == SEEMPS_PREC_FP32 ? "zgemm_kernel_fp32" : "zgemm_kernel", stream,
-                    flops);
+  TimedLaunch timed(prec == SEEMPS_PREC_FP32 ? "zgemm_kernel_fp32"
+                    : direct.F               ? "zgemm_direct"
+                                             : "zgemm_kernel",
+                    stream, flops);
 #define SEEMPS_GEMM_CASE(x, y)                                                              \
   if (opA == x && opB == y) {                                                               \
     if (direct.F) {                                                                         \

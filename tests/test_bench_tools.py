@@ -151,3 +151,31 @@ def test_committed_profiles_parse(bench):
     assert flops is not None and flops > 0
     plain_bytes, _ = bench.read_traffic("svd_jacobi", "plain")
     assert plain_bytes > traffic
+
+
+def test_counter_passes_cover_the_instrumented_kernels(bench):
+    """Every launch that the library times with a flop count is in the counter
+    tables under its rocprofv3 name, and the kernels that can dominate a sweep
+    are timed in it; a product kernel has a timing name of its own."""
+    import re
+
+    timed = set()
+    for src in sorted((ROOT / "seemps2_amd" / "csrc").glob("*.hip")):
+        for stmt in re.findall(r"TimedLaunch timed\(([^;]*);", src.read_text()):
+            if not re.search(r",\s*0\.0\)$", stmt.strip()):
+                timed.update(re.findall(r'"(\w+)"', stmt))
+    assert {"zgemm_kernel", "zgemm_direct", "lz_product_dots", "svd_jacobi"} <= timed
+    missing = {bench.ROCPROF_NAMES.get(k, k) for k in timed} - set(bench.PMC_KERNELS)
+    assert not missing
+    assert {"zgemm_kernel", "zgemm_direct", "lz_product_dots", "polar_svd",
+            "svd_jacobi"} <= set(bench.TIMED_KERNELS.split(","))
+
+
+def test_traffic_of_a_kernel_without_a_record(bench, tmp_path, monkeypatch):
+    """A profile taken before a kernel existed gives no figure for it."""
+    rec = {"forms": {"chosen": {"zgemm_kernel": {"traffic_bytes": 7, "fp64_mfma_flops": 3}}}}
+    path = tmp_path / "pmc.md"
+    path.write_text("```json\n" + json.dumps(rec) + "\n```\n")
+    monkeypatch.setattr(bench, "PMC_PROFILE", str(path))
+    assert bench.read_traffic("zgemm_kernel", "chosen") == (7, 3)
+    assert bench.read_traffic("zgemm_direct", "chosen") == (None, None)
