@@ -368,49 +368,89 @@ bool gemm_scheme_3m() {
 }
 
 // How an FP64 product without a batch runs: the direct kernel with (F, KS), or
-// staged through LDS (F = 0).  t counts 32 x 32 tiles; a tile of four waves fills
-// one CU, so t / 256 CUs says how evenly the work divides.  Times in us, staged
-// (with split-K where it applied) against 1,4 / 2,4 / 2,1:
-//   M N K (t)                staged    1,4    2,4    2,1
-//   64 64 64 (4)                5.6    3.1    5.4    9.4
-//   256 400 200 (104)          15.2    7.0   11.2   23.4
-//   640 512 512 (320)          32.7   26.6   34.5   56.6
-//   1280 512 256 (640)         36.9   30.0   28.4   36.1
-//   512 512 512 (256)          27.8   22.3   22.2   54.7
-//   1024 1024 1024 (1024)     142.8  176.0  121.4  123.0
-//   1024 2048 2048 (2048)     514.5  661.2  437.8  443.0
-//   1500 1100 300 (1645)       74.8   78.9   71.0   69.9
-//   1024 1024 64 (1024)        13.4   16.4   14.8   14.8
-//   1280 1024 256 (1280)       49.3   58.7   51.1   58.7
-// (Outputs of four 64 x 64 tiles a CU keep that tile and its four real products:
-// 2048 2048 512 takes 280.1 there against 228.3 with three.)
-// Few tiles: 16 x 16 ones for four times the waves.  From a tile for each CU:
-// 32 x 32 ones, which ask half the loads, where whole rounds of the CUs come out
-// at least four fifths full, and one wave a tile once every SIMD has its own.
-// Many tiles that leave a round part empty, and short K, stay staged.  So do few
-// tiles with both operands contiguous along a long K: a load of theirs touches
-// sixteen rows, and splitting K over more CUs wins (64 x 64 x 1024 NT 12.4 against
-// 16.7, 64 x 2048 x 2048 NT 46.9 / 59.1; 1024 x 256 x 1280 NT alone 54.7 / 53.2
-// but 2.5 us slower within a matvec; shorter K win, 512 x 128 x 640 NT 15.5 /
-// 11.7, as NN and HN at any K, 64 x 64 x 4096 HN 33.8 / 32.7).
+// staged through LDS (F = 0).
 struct Direct {
   int F, KS;
 };
 
-// op(A)'s rows and op(B)'s columns both contiguous along K
-bool rows_in_k(int opA, int opB) {
-  return (opA == SEEMPS_OP_N || opA == SEEMPS_OP_C) && (opB == SEEMPS_OP_T || opB == SEEMPS_OP_H);
-}
+// op(A)'s rows (op(B)'s columns) contiguous along K
+inline bool a_along_k(int op) { return op == SEEMPS_OP_N || op == SEEMPS_OP_C; }
+inline bool b_along_k(int op) { return op == SEEMPS_OP_T || op == SEEMPS_OP_H; }
 
+// The rule takes a product to the direct kernel where it is the faster one.  What
+// decides: how many operands run along K (g: a load of theirs touches sixteen rows),
+// the tiles against the CUs (a tile of four waves fills one) and K.  us, staged (with
+// split-K where it applies) / direct 1,4 / 2,4 / 2,1:
+//   op M N K                 staged    1,4    2,4    2,1
+//   NN 64 64 64                 6.2    3.6    5.8    9.9
+//   NN 64 64 4096              34.6   37.8  108.7  389.5
+//   HN 64 64 4096              33.8   33.4  108.7  396.5
+//   HN 640 512 256             24.7   14.5   22.1   29.9
+//   NT 128 128 768             12.1   13.9   35.1   78.6
+//   NT 512 512 512             29.9   34.2   28.7   54.7
+//   NT 512 512 768             36.7   46.0   37.7   79.1
+//   NT 700 700 768             70.6   91.6   59.6   87.5
+//   NT 960 960 1000           137.5  214.2  133.6  154.9
+//   NN 900 900 16               7.6   14.4   18.0    7.8
+//   NN 900 900 256             42.9   37.0   49.4   40.7
+//   NN 1200 1100 333           79.7   76.7   93.3   85.4
+//   NN 1024 1024 1024         168.4  186.3  152.4  151.0
+// (Outputs of four 64 x 64 tiles a CU keep that tile and its four real products:
+// 2048 2048 512 takes 280.1 there against 228.3 with three.)
+// Over 17600 shapes (M, N from 8 to 2500, K from 8 to 12000, the four pairs of
+// contiguous directions, sizes odd and even) the choice takes 1.28 times less than
+// staging everything, 1 % more than the best of the four each time; 0.4 % of them
+// are more than 3 % slower than staged.
 Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_cu) {
   if (forced_tile() >= 0 || !gemm_scheme_3m()) return {0, 0};
   if (choose_tile(M, N, 1, num_cu) == TILE_64x64) return {0, 0};  // four products
+  constexpr int64_t ANY = INT64_MAX, NEVER = INT64_MAX;
   const int64_t cu = num_cu > 0 ? num_cu : 256, simd = 4 * cu;
   const int64_t t = ceil_div(M, 32) * ceil_div(N, 32);
-  auto full = [&](int64_t units) { return 5 * t >= 4 * units * ceil_div(t, units); };
-  if (t >= simd) return full(simd) && t * K >= 128 * simd ? Direct{2, 1} : Direct{0, 0};
-  if (rows_in_k(opA, opB) && K >= 1024) return {0, 0};
-  return t >= cu && full(cu) ? Direct{2, 4} : Direct{1, 4};
+  const int64_t t16 = ceil_div(M, 16) * ceil_div(N, 16);
+  const int g = (int)a_along_k(opA) + (int)b_along_k(opB);
+
+  // 32 x 32, K over four waves: up to four rounds of the CUs, the last five sixths
+  // full or more.  Half the loads of 16 x 16 tiles, so the sooner the more operands
+  // run along K.
+  const int64_t r = ceil_div(t, cu);
+  if (r <= 4 && 6 * t >= 5 * cu * r) {
+    static const int64_t from[3][4] = {{64, 1600, NEVER, NEVER},
+                                       {200, 1024, 1024, 1024},
+                                       {200, 200, 200, 850}};
+    const bool split = g == 2 && r == 1 && K >= 720;  // split-K spreads it over more CUs
+    if (K >= from[g][r - 1] && !split) return {2, 4};
+  }
+  // 32 x 32, a wave a tile: rounds of the SIMDs four fifths full
+  const int64_t rs = ceil_div(t, simd);
+  if (t > 3 * cu && 5 * t >= 4 * simd * rs) {
+    static const int64_t from[3][2] = {{48, 48}, {256, 100}, {NEVER, 160}};
+    return K >= from[g][rs > 1] ? Direct{2, 1} : Direct{0, 0};
+  }
+  // 16 x 16, K over four waves, for few tiles or rounds left part empty by 32 x 32:
+  // up to a K from which staging, its loads coalesced and K split over more CUs,
+  // wins; that comes sooner where the last round is less than half full.  Tiles that
+  // reach past an edge cost the staged kernel bounds tests, the direct one nothing.
+  const int64_t u = ceil_div(t16, cu);
+  if (u > 14) return {0, 0};
+  const bool edge = M % 32 != 0 || N % 32 != 0;
+  // tiles: up to cu/8, cu/2, cu; 2, 3 and 4 rounds, less and more than half full;
+  // 6 rounds, 14
+  static const int64_t upto[3][11] = {
+      {2700, 6000, ANY, 3500, 8000, 2700, 6000, 1600, 6000, 4000, 1600},
+      {1800, 3500, ANY, 1280, 2000, 850, 2000, 1280, 1600, 1000, 850},
+      {500, 600, 1000, 320, 512, 320, 400, 0, 0, 0, 0}};
+  static const int64_t upto_edge[3][3] = {{ANY, ANY, ANY}, {4000, ANY, ANY}, {720, 720, 1500}};
+  const int i = u == 1   ? (8 * t16 <= cu ? 0 : 2 * t16 <= cu ? 1 : 2)
+                : u <= 4 ? (int)(2 * u - 1) + (2 * t16 >= (2 * u - 1) * cu)
+                         : (u <= 6 ? 9 : 10);
+  const int64_t hi = !edge   ? upto[g][i]
+                     : i < 3 ? upto_edge[g][i]
+                             : upto[g][i] + upto[g][i] / 2;
+  // with many tiles a short K does not pay for the prologue of each
+  int64_t lo = i < 3 ? 1 : t16 / (g == 2 ? (edge ? 16 : 8) : (edge ? 24 : 12));
+  if ((g == 2 || (g == 1 && i >= 3)) && lo < 17) lo = 17;
+  return lo <= K && K <= hi ? Direct{1, 4} : Direct{0, 0};
 }
 
 template <int OPA, int OPB>

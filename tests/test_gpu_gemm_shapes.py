@@ -100,3 +100,37 @@ def test_grouped_gemm_edges(tile, count, opA, opB):
     gg.launch()
     for Cd, ref in zip(outs, refs):
         assert np.array_equal(K.to_numpy(Cd), ref)
+
+
+# Both sides of the lines between the direct and the staged kernel (256 CUs): few tiles
+# and a long K, aligned and past an edge; whole and part-empty rounds of the CUs and of
+# the SIMDs; a K too short for many tiles; both operands along K.
+@pytest.mark.parametrize("opA,opB,M,N,K_,direct", [
+    (0, 0, 64, 64, 1024, True), (0, 0, 64, 64, 8192, False), (2, 0, 64, 64, 2048, True),
+    (0, 0, 33, 40, 8192, False), (2, 0, 33, 40, 8192, True), (0, 1, 128, 128, 512, True),
+    (0, 1, 128, 128, 768, False), (0, 1, 512, 512, 512, True), (0, 1, 512, 512, 768, False),
+    (0, 1, 272, 1000, 256, False), (0, 1, 272, 1000, 768, False), (3, 2, 700, 700, 768, True),
+    (2, 0, 640, 512, 256, True), (0, 0, 900, 900, 16, False), (0, 0, 900, 900, 256, True),
+    (1, 1, 1024, 1000, 300, True), (1, 0, 1100, 1000, 60, False), (1, 0, 1100, 1000, 333, False),
+    (1, 0, 700, 640, 333, True)])
+def test_gemm_route(opA, opB, M, N, K_, direct):
+    from seemps2_amd import _lib, kernels as K
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are drawn for 256 CUs")
+    rng = np.random.default_rng(M + N + K_)
+
+    def ints(r, c):
+        return rng.integers(-3, 4, (r, c)) + 1j * rng.integers(-3, 4, (r, c))
+
+    A = ints(*((K_, M) if opA in (1, 2) else (M, K_)))
+    B = ints(*((N, K_) if opB in (1, 2) else (K_, N)))
+    a, b = K.as_dev(A), K.as_dev(B)
+    _lib.timing_enable("zgemm_kernel,zgemm_direct")
+    try:
+        out = K.to_numpy(K.gemm(a, b, opA, opB))
+        ran = [k for k, r in _lib.timing_records().items() if r["launches"]]
+    finally:
+        _lib.timing_enable(None)
+    assert ran == ["zgemm_direct" if direct else "zgemm_kernel"]
+    assert np.array_equal(out, OPS[opA](A) @ OPS[opB](B))
