@@ -27,6 +27,10 @@
 namespace seemps {
 namespace {
 
+__device__ __forceinline__ double2 rscale(double f, double2 x) {
+  return make_double2(f * x.x, f * x.y);
+}
+
 struct Reflector {
   double beta;
   double2 d, tau;  // (alpha - beta) up, tau
@@ -131,9 +135,9 @@ __global__ __launch_bounds__(64 * NW) void qr_panel(double2* __restrict__ A, int
       const Reflector h = make_reflector(alpha, nn);
       if (h.up != 1.0) {
 #pragma unroll
-        for (int r = 0; r < RPT; ++r) x[r] = make_double2(x[r].x * h.up, x[r].y * h.up);
+        for (int r = 0; r < RPT; ++r) x[r] = rscale(h.up, x[r]);
 #pragma unroll
-        for (int k = 0; k < CPW; ++k) d[k] = make_double2(d[k].x * h.up, d[k].y * h.up);
+        for (int k = 0; k < CPW; ++k) d[k] = rscale(h.up, d[k]);
       }
 #pragma unroll
       for (int r = 0; r < RPT; ++r)
@@ -287,7 +291,7 @@ __global__ __launch_bounds__(64) void qr_reflect(double2* __restrict__ Y, int64_
 // ---- columns longer than the registers hold (more than 64 REG_RPT rows) ------
 
 constexpr int REG_RPT = 16;
-constexpr int LONG_NB = 16;
+constexpr int LONG_NB = 8;
 
 __device__ double2 block_sum(double2 v, double2* red) {
   v = wave::sum2(v);
@@ -316,42 +320,123 @@ __device__ void long_reflect(double2* __restrict__ y, const double2* __restrict_
   }
 }
 
-// Panel of nb columns from j0 on, columns in memory, one workgroup.
-__global__ __launch_bounds__(1024) void qr_panel_long(double2* __restrict__ A, int64_t len,
-                                                      int64_t j0, int nb,
-                                                      double2* __restrict__ tau,
-                                                      double2* __restrict__ Vall) {
-  __shared__ double2 red[16];
-  for (int j = 0; j < nb; ++j) {
-    const int64_t c = j0 + j;
-    double2* col = A + c * len;
-    double2* v = Vall + c * len;
-    __syncthreads();
-    double2 acc = make_double2(0.0, 0.0);
-    for (int64_t r = c + 1 + threadIdx.x; r < len; r += blockDim.x) acc.x += cabs2(col[r]);
-    const Reflector h = make_reflector(col[c], block_sum(acc, red).x);
-    __syncthreads();  // every thread has read col[c]
-    for (int64_t r = j0 + threadIdx.x; r < len; r += blockDim.x) {
-      v[r] = (r < c)    ? make_double2(0.0, 0.0)
-             : (r == c) ? h.d
-                        : make_double2(col[r].x * h.up, col[r].y * h.up);
-      if (r == c) col[r] = make_double2(h.beta, 0.0);
+// Panel of nb <= NB columns from j0 on, columns in memory, one workgroup.  A thread
+// keeps the same rows throughout.  Step j: one pass applies reflector j to the later
+// columns and forms, from the values in hand, the norm of column j + 1 below its
+// diagonal and its dot products with the columns after it; a wavefront then derives
+// reflector j + 1 and the factors of the next pass.  Two barriers a column.  Bound by
+// what one CU moves, so panels are narrow: 16 columns of 4096 rows take 134 us in two
+// of eight (and 50 on the reflectors in between), 205 in one of sixteen, and took 501
+// with a pass for every dot product and every update.
+constexpr int LONG_THREADS = 512;
+
+template <int NB>
+struct LongLds {
+  double2 red[LONG_THREADS / 64][NB];  // wavefronts' sums: |x|^2 of the next column, x^H a_k
+  double2 row[NB];                     // the next column's diagonal row
+  double2 f[NB];                       // -conj(tau) v^H a_k
+  Reflector h;
+};
+
+// Steps J, J + 1, .. of the panel (P, V: its columns of A and of Vall); J = -1 only
+// forms the sums of column 0.
+template <int NB, int J>
+__device__ __forceinline__ void long_steps(double2* __restrict__ P, double2* __restrict__ V,
+                                           int64_t len, int64_t j0, int nb,
+                                           double2* __restrict__ tau, LongLds<NB>& L) {
+  constexpr int NW = LONG_THREADS / 64, T = NB - 1 - J;  // columns after column J
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t c = j0 + J;
+  const bool any = J >= 0 && L.h.any;
+  double2 acc[T];
+#pragma unroll
+  for (int k = 0; k < T; ++k) acc[k] = make_double2(0.0, 0.0);
+  for (int64_t r = j0 + threadIdx.x; r < len; r += LONG_THREADS) {
+    double2 v = make_double2(0.0, 0.0);
+    if (J >= 0) {
+      double2* x = P + J * len + r;
+      if (r >= c) v = r == c ? L.h.d : rscale(L.h.up, *x);
+      V[J * len + r] = v;
+      if (r == c) *x = make_double2(L.h.beta, 0.0);
+      if (r < c) continue;
     }
-    if (threadIdx.x == 0) tau[c] = h.tau;
-    if (!h.any) continue;
-    __syncthreads();
-    for (int jj = j + 1; jj < nb; ++jj)
-      long_reflect(A + (j0 + jj) * len, v, c, len, make_double2(h.tau.x, -h.tau.y), red);
+    double2 a[T];
+    double2* const p = P + (J + 1) * len + r;
+#pragma unroll
+    for (int k = 0; k < T; ++k) a[k] = p[min(k, nb - 2 - J) * len];
+    if (any) {
+#pragma unroll
+      for (int k = 0; k < T; ++k) a[k] = cfma(L.f[J + 1 + k], v, a[k]);
+#pragma unroll
+      for (int k = 0; k < T; ++k)
+        if (k < nb - 1 - J) p[k * len] = a[k];
+    }
+    if (r == c + 1) {
+#pragma unroll
+      for (int k = 0; k < T; ++k) L.row[J + 1 + k] = a[k];
+    } else if (r > c + 1) {
+      acc[0].x += cabs2(a[0]);
+#pragma unroll
+      for (int k = 1; k < T; ++k) acc[k] = cfmac(a[0], a[k], acc[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < T; k += 2) {
+    if (k + 1 < T)
+      wave::sum4(acc[k], acc[k + 1 < T ? k + 1 : k]);
+    else
+      acc[k] = wave::sum2(acc[k]);
+    if (lane == 0) {
+      L.red[wv][J + 1 + k] = acc[k];
+      if (k + 1 < T) L.red[wv][J + 2 + k] = acc[k + 1 < T ? k + 1 : k];
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const int k = min(max(lane, J + 1), NB - 1);
+    double2 t = make_double2(0.0, 0.0);
+    for (int q = 0; q < NW; ++q) t = cadd(t, L.red[q][k]);
+    const Reflector h = make_reflector(L.row[J + 1], wave::bcast(t.x, J + 1));
+    // v^H a_k = conj(d) a_k[c + 1] + up x^H a_k
+    if (lane > J + 1 && lane < NB)
+      L.f[k] = cmul(make_double2(-h.tau.x, h.tau.y), cfmac(h.d, L.row[k], rscale(h.up, t)));
+    if (lane == 0) {
+      L.h = h;
+      tau[c + 1] = h.tau;
+    }
+  }
+  __syncthreads();
+  if constexpr (J + 2 < NB) {
+    if (J + 2 < nb) long_steps<NB, J + 1>(P, V, len, j0, nb, tau, L);
+  }
+}
+
+template <int NB>
+__global__ __launch_bounds__(LONG_THREADS) void qr_panel_long(double2* __restrict__ A, int64_t len,
+                                                              int64_t j0, int nb,
+                                                              double2* __restrict__ tau,
+                                                              double2* __restrict__ Vall) {
+  __shared__ LongLds<NB> L;
+  long_steps<NB, -1>(A + j0 * len, Vall + j0 * len, len, j0, nb, tau, L);
+  // the last column: its reflector
+  const int64_t c = j0 + nb - 1;
+  for (int64_t r = j0 + threadIdx.x; r < len; r += LONG_THREADS) {
+    double2* x = A + c * len + r;
+    Vall[c * len + r] = r < c    ? make_double2(0.0, 0.0)
+                        : r == c ? L.h.d
+                                 : rscale(L.h.up, *x);
+    if (r == c) *x = make_double2(L.h.beta, 0.0);
   }
 }
 
 // Reflectors j0 .. j1 - 1 (adjoint, ascending) or j1 - 1 .. j0 on one column
-// of Y per workgroup, in memory.
-__global__ __launch_bounds__(256) void qr_reflect_long(double2* __restrict__ Y, int64_t len,
-                                                       int64_t j0, int64_t j1, int forward,
-                                                       const double2* __restrict__ tau,
-                                                       const double2* __restrict__ Vall) {
-  __shared__ double2 red[4];
+// of Y per workgroup, in memory.  16 reflectors on 16 columns of 20000 rows: 587 us
+// with 256 threads, 259 with 1024; up to 4096 rows the barriers of 256 are the shorter.
+__global__ __launch_bounds__(1024) void qr_reflect_long(double2* __restrict__ Y, int64_t len,
+                                                        int64_t j0, int64_t j1, int forward,
+                                                        const double2* __restrict__ tau,
+                                                        const double2* __restrict__ Vall) {
+  __shared__ double2 red[16];
   double2* y = Y + (int64_t)blockIdx.x * len;
   for (int64_t q = 0; q < j1 - j0; ++q) {
     const int64_t j = forward ? j0 + q : j1 - 1 - q;
@@ -391,7 +476,8 @@ int panel(int r, double2* A, int64_t len, int64_t j0, int nb, double2* tau, doub
   else if (r == 16)
     SEEMPS_PANEL(8, 16, 1);
   else
-    hipLaunchKernelGGL(qr_panel_long, dim3(1), dim3(1024), 0, stream, A, len, j0, nb, tau, Vall);
+    hipLaunchKernelGGL(nb <= 4 ? qr_panel_long<4> : qr_panel_long<LONG_NB>,
+                       dim3(1), dim3(LONG_THREADS), 0, stream, A, len, j0, nb, tau, Vall);
 #undef SEEMPS_PANEL
   return check_launch("qr_panel");
 }
@@ -420,8 +506,8 @@ int reflect(double2* Y, int64_t len, int64_t ny, int64_t r0, int64_t j0, int64_t
     case 8: SEEMPS_REFLECT(8); break;
     case 16: SEEMPS_REFLECT(16); break;
     default:
-      hipLaunchKernelGGL(qr_reflect_long, dim3((unsigned)ny), dim3(256), 0, stream, Y, len, j0, j1,
-                         (int)FORWARD, tau, Vall);
+      hipLaunchKernelGGL(qr_reflect_long, dim3((unsigned)ny), dim3(len > 4096 ? 1024 : 256), 0,
+                         stream, Y, len, j0, j1, (int)FORWARD, tau, Vall);
   }
 #undef SEEMPS_REFLECT
   return check_launch("qr_reflect");

@@ -81,20 +81,22 @@ __global__ __launch_bounds__(256) void row_norms(int64_t rows, int64_t cols,
   acc = wave::sum(acc);
   if ((threadIdx.x & 63) == 0) nrm[r] = acc;
 }
-// ... or of A's columns (64 to a workgroup, the rows over its wavefronts).
-__global__ __launch_bounds__(1024) void column_norms(int64_t rows, int64_t cols,
+// ... or of A's columns (cw = 16, 32 or 64 to a workgroup; the rows over
+// its wavefronts and their 64 / cw groups of lanes).
+__global__ __launch_bounds__(1024) void column_norms(int64_t rows, int64_t cols, int cw,
                                                      const double2* __restrict__ A,
                                                      double* __restrict__ nrm) {
-  __shared__ double red[16][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t c = blockIdx.x * 64 + lane;
+  __shared__ double red[1024];
+  const int64_t c = (int64_t)blockIdx.x * cw + (threadIdx.x & (cw - 1));
   double acc = 0.0;
-  if (c < cols)
-    for (int64_t r = wv; r < rows; r += 16) acc += cabs2(A[r * cols + c]);
-  red[wv][lane] = acc;
+  if (c < cols) {
+#pragma unroll 4
+    for (int64_t r = threadIdx.x / cw; r < rows; r += 1024 / cw) acc += cabs2(A[r * cols + c]);
+  }
+  red[threadIdx.x] = acc;
   __syncthreads();
-  if (wv == 0 && c < cols) {
-    for (int q = 1; q < 16; ++q) acc += red[q][lane];
+  if ((int)threadIdx.x < cw && c < cols) {
+    for (int q = cw; q < 1024; q += cw) acc += red[q + threadIdx.x];
     nrm[c] = acc;
   }
 }
@@ -340,9 +342,12 @@ int svd_split_impl(int64_t m, int64_t n, const double2* A, int mode, int method,
   if (s.transposed)
     hipLaunchKernelGGL(row_norms, dim3((unsigned)ceil_div(m, 4)), dim3(256), 0, st_, m, n, A,
                        w.colnrm);
-  else
-    hipLaunchKernelGGL(column_norms, dim3((unsigned)ceil_div(n, 64)), dim3(1024), 0, st_, m, n, A,
-                       w.colnrm);
+  else {
+    int cw = 64;
+    while (cw > 16 && cw / 2 >= n) cw /= 2;
+    hipLaunchKernelGGL(column_norms, dim3((unsigned)ceil_div(n, cw)), dim3(1024), 0, st_, m, n, cw,
+                       A, w.colnrm);
+  }
   if ((st = check_launch("split norms"))) return st;
   hipLaunchKernelGGL(load_sorted, dim3((unsigned)s.ncol), dim3(256), 0, st_, s, A, w);
   if ((st = check_launch("load_sorted"))) return st;

@@ -123,3 +123,24 @@ def test_split_of_tiny_matrices(K, m, n, r, mode):
     out = K.to_numpy(Ad) @ K.to_numpy(Bd) / scale
     assert D == min(m, n)
     assert rel(out, A) < 1e-12
+
+
+# Columns beyond the registers: panels of one, up to four and up to eight columns and
+# their remainders, the reflectors on workgroups of 256 and (from 4097 rows) of 1024
+# threads; few enough columns for the norms' lanes to share a row.
+@pytest.mark.parametrize("m,n", [(1025, 1), (1025, 4), (1030, 5), (1600, 8), (1601, 9),
+                                 (24, 1030), (4097, 12), (5000, 40), (1100, 70)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_split_long_columns(K, m, n, mode):
+    rng = np.random.default_rng(m * 1000 + n)
+    r = min(m, n)
+    A = crandn(rng, m, r) * np.exp(-20.0 / r * np.arange(r)) @ crandn(rng, r, n)
+    A /= np.linalg.norm(A)
+    Ad, Bd, D, _, sd = K.svd_split(K.as_dev(A), m, n, mode, 0, 0.0, r, want_s=True)
+    Ad, Bd = K.to_numpy(Ad), K.to_numpy(Bd)
+    assert D == r
+    assert rel(Ad @ Bd, A) < 1e-12
+    iso = Ad.conj().T @ Ad if mode == 0 else Bd @ Bd.conj().T
+    assert np.abs(iso - np.eye(r)).max() < 1e-12
+    s_ref = np.linalg.svd(A, compute_uv=False)
+    assert np.abs(sd.cpu().numpy() - s_ref).max() < 5e-13 * s_ref[0]
