@@ -387,8 +387,8 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
 // what it has (the second index's diagonal entry comes with that pair's
 // rotation), everyone applies it after the barrier.
 //
-// A round takes 0.51 us, two thirds of it instruction issue (48 FP64
-// operations a thread in either role, the rotation's chain of 45); with G and
+// A round takes 0.52 us, two thirds of it instruction issue (48 FP64
+// operations a thread in either role, the rotation's chain of 55); with G and
 // the tile in LDS it took 1.07 us, LDS traffic (100 KB a round).
 constexpr int JT = 768;            // threads
 constexpr int TP = RT + 1;         // padded tile column (complex)
@@ -438,12 +438,27 @@ struct PairLds {
   int flag;
 };
 
+// 1/sqrt(x) and 1/x to a few ulp by one step of third order on the hardware's
+// estimate (about 5e-8): two dependent operations shorter than jac::rsqrt_nr and
+// rcp_nr, but an ulp low at x = 1, where those are exact.
+__device__ __forceinline__ double rsqrt_short(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double rcp_short(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+
 // Rotation that annihilates c = G_ab; identity when the pair is orthogonal to
 // tol or either column negligible.  t = tan(angle), the smaller root of
-// t^2 + 2 tau t - 1 = 0, comes from the hardware's reciprocal and square root
-// estimates (relative error about 1e-7): an angle that far off leaves 1e-7 of
-// G_ab, which the next sweep removes.  cs and |s| are refined to a few ulp, so
-// the rotation is unitary whatever t is.
+// t^2 + 2 tau t - 1 = 0, to a few ulp (from the unrefined estimates it was good to
+// 1e-8, a round 0.01 us shorter, and left that much of G_ab to the next sweep).
+// cs = 1/sqrt(1 + t^2) must be unbiased where it is close to one (jac::rsqrt_nr is):
+// an ulp lost in each of the hundreds of small rotations of a column adds up
+// (1.4e-14 against 8.9e-15 on 64 columns).
 __device__ __forceinline__ Rot pair_rotation(double gaa, double gbb, double2 c, double tol2,
                                              double tiny2) {
   Rot q;
@@ -452,10 +467,10 @@ __device__ __forceinline__ Rot pair_rotation(double gaa, double gbb, double2 c, 
   q.s = make_double2(0.0, 0.0);
   const double s2 = cabs2(c);
   const bool any = s2 > 0.0 && gaa > tiny2 && gbb > tiny2 && s2 > (tol2 * gaa) * gbb;
-  const double tau = (gbb - gaa) * (0.5 * __builtin_amdgcn_rsq(s2));
+  const double tau = (gbb - gaa) * (0.5 * rsqrt_short(s2));
   const double at = fmin(fabs(tau), 1e150);
   const double u = fma(at, at, 1.0);
-  const double t = copysign(__builtin_amdgcn_rcp(fma(u, __builtin_amdgcn_rsq(u), at)), tau);
+  const double t = copysign(rcp_short(fma(u, rsqrt_short(u), at)), tau);
   const double cs = jac::rsqrt_nr(fma(t, t, 1.0)), r = jac::rsqrt_nr(s2);
   const double sn = t * cs * r;
   if (any) {
@@ -896,7 +911,7 @@ __device__ inline void local_item(int64_t b, int64_t G, int64_t R, int64_t* p, i
 // other CUs shortens it; V's workgroups follow W's by a step or so and hold them up
 // only if they fall two behind (the partial Grams alternate between two buffers) or
 // at the end.  They read the convergence measure but are not counted in the barrier.
-// An inner round 0.52 -> 0.44 us (64 columns).
+// An inner round 0.53 -> 0.45 us (64 columns).
 // !LOCAL: items are strided over the grid, with two grid barriers per step.
 template <bool LOCAL, bool VSEP>
 __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double tol,

@@ -144,3 +144,27 @@ def test_split_long_columns(K, m, n, mode):
     assert np.abs(iso - np.eye(r)).max() < 1e-12
     s_ref = np.linalg.svd(A, compute_uv=False)
     assert np.abs(sd.cpu().numpy() - s_ref).max() < 5e-13 * s_ref[0]
+
+
+@pytest.mark.parametrize("c", [0.1, 0.3, 0.5, 0.7, 1.0, 1.6])
+def test_one_rotation_is_exact(K, c):
+    """Columns that are orthogonal but for one pair: a sweep meets that pair once, and
+    a rotation whose angle is good to rounding leaves it orthogonal to far below the
+    1e-9 from which the next sweep is the last.  An angle off by 1e-8 takes three."""
+    import ctypes
+
+    from seemps2_amd._lib import check, lib, ptr, stream, workspace
+
+    n, a, b = 64, 3, 40
+    rng = np.random.default_rng(11)
+    R = np.diag(np.linspace(3.0, 1.0, n)) + 0j
+    R[a, b] = c
+    A = K.as_dev(np.linalg.qr(crandn(rng, n, n))[0] @ R)
+    U, VH = K.empty(n, n), K.empty(n, n)
+    S = torch.empty(n, dtype=torch.float64, device=A.device)
+    wp, wn = workspace.get(lib.seemps_svd_workspace(n, n))
+    info = (ctypes.c_int32 * 2)()
+    check(lib.seemps_zgesvd(n, n, ptr(A), n, ptr(U), ptr(S), ptr(VH), wp, wn, info, stream()))
+    assert list(info) == [2, 1]
+    s_ref = np.linalg.svd(R, compute_uv=False)
+    assert np.abs(S.cpu().numpy() - s_ref).max() < 5e-13 * s_ref[0]
