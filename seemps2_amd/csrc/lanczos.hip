@@ -62,7 +62,6 @@ struct LzScalars {
   double y[64];
   double2 h;        // first-pass coefficient of the last basis vector
   int kd;           // effective Krylov dimension of the cycle
-  int broken;       // breakdown seen in this cycle
   double scl[64];   // running max |alpha| + |beta| after step j (breakdown reference)
   int brk[64];      // breakdown seen up to step j
 };
@@ -435,7 +434,6 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_orth3(int64_t n, int k,
     s->beta[j] = brk ? 0.0 : beta;
     s->scl[j] = ref;
     s->brk[j] = brk;
-    s->broken = brk;
     s->kd = kd_new;
   }
   if (!ritz) return;
@@ -503,10 +501,7 @@ __global__ __launch_bounds__(LZ_THREADS) void lz_unit(int64_t n, int nb,
                                                       LzScalars* __restrict__ s) {
   const double nn = sqrt(fmax(lz_wave_sum(nb, pn), 0.0));
   const double inv = (nn > 0.0) ? 1.0 / nn : 0.0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    s->broken = 0;
-    s->kd = 0;
-  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) s->kd = 0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const double2 t = x[i], u = make_double2(t.x * inv, t.y * inv);

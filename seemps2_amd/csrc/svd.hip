@@ -1294,26 +1294,25 @@ __global__ void truncate_kernel(int64_t N, const double* __restrict__ s, int met
   truncation_rule(N, ss, method, tol, max_bond, D_out, err_out);
 }
 
-int cooperative_grid(int64_t items, int* grid) {
+// Kernel of each variant, and the workgroups of it that can be resident at once.
+const void* jacobi_kernel(int variant) {
+  return variant == JACOBI_V_APART ? (const void*)svd_jacobi<true, true>
+         : variant == JACOBI_LOCAL ? (const void*)svd_jacobi<true, false>
+                                   : (const void*)svd_jacobi<false, false>;
+}
+int resident_workgroups(int64_t* lim) {
   DeviceInfo di;
   int st = device_info(&di);
   if (st) return st;
-  static thread_local int occ_dev = -1, occ = 0;
+  static thread_local int occ_dev = -1, occ[3];
   if (occ_dev != di.device) {
-    int o = 0;
-    SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &o, (const void*)svd_jacobi<true, false>, JT, 0));
-    occ = o;
+    for (int v = 0; v < 3; ++v) {
+      occ[v] = 0;
+      SEEMPS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ[v], jacobi_kernel(v), JT, 0));
+    }
     occ_dev = di.device;
   }
-  int64_t lim = (int64_t)occ * di.num_cu;
-  if (lim < 1) {
-    set_error("svd: kernel cannot be resident on this device");
-    return SEEMPS_ERR_RUNTIME;
-  }
-  int64_t g = items < lim ? items : lim;
-  if (g > 1024) g = 1024;
-  *grid = (int)g;
+  for (int v = 0; v < 3; ++v) lim[v] = (int64_t)occ[v] * di.num_cu;
   return SEEMPS_OK;
 }
 
@@ -1373,15 +1372,33 @@ void jacobi_shape(SvdShape* s, int num_cu) {
   s->cross_inner = s->nb > 2 ? inner_mode : 0;
 }
 
+bool jacobi_plan(int64_t P, int64_t R, int64_t VS, const int64_t* lim, int* variant, int* grid) {
+  // an item a workgroup where they all fit: local step ordering
+  const int64_t apart = P * (R + VS), local = P * R;
+  if (VS > 0 && apart <= lim[JACOBI_V_APART]) {
+    *variant = JACOBI_V_APART;
+    *grid = (int)apart;
+  } else if (local <= lim[JACOBI_LOCAL]) {
+    *variant = JACOBI_LOCAL;
+    *grid = (int)local;
+  } else {
+    *variant = JACOBI_STRIDED;
+    *grid = (int)(local < lim[JACOBI_STRIDED] ? local : lim[JACOBI_STRIDED]);
+  }
+  return *grid >= 1;
+}
+
 int jacobi_enqueue(const SvdShape& shape, const SvdWork& w, hipStream_t stream) {
   SvdShape s = shape;
-  int st, grid = 1;
   if (!w.V) s.VS = 0;
-  if ((st = cooperative_grid(s.P * (s.R + s.VS), &grid))) return st;
-  if (grid < s.P * (s.R + s.VS)) {
-    s.VS = 0;
-    if ((st = cooperative_grid(s.P * s.R, &grid))) return st;
+  int64_t lim[3];
+  int st, variant, grid;
+  if ((st = resident_workgroups(lim))) return st;
+  if (!jacobi_plan(s.P, s.R, s.VS, lim, &variant, &grid)) {
+    set_error("svd: kernel cannot be resident on this device");
+    return SEEMPS_ERR_RUNTIME;
   }
+  if (variant != JACOBI_V_APART) s.VS = 0;
   // Relative orthogonality target: a few times above the rounding floor of the
   // measured Gram entries (~sqrt(len) eps), so that rounding alone cannot keep
   // the measure above it.
@@ -1391,10 +1408,7 @@ int jacobi_enqueue(const SvdShape& shape, const SvdWork& w, hipStream_t stream) 
   // nominal SVD flops (complex): 4 * (6 M N^2 + 16 N^3), M >= N
   const double M_ = (double)s.lenA, N_ = (double)s.ncol;
   TimedLaunch timed("svd_jacobi", stream, 4.0 * (6.0 * M_ * N_ * N_ + 16.0 * N_ * N_ * N_));
-  // one work item per workgroup when they all fit: local step ordering
-  const void* fn = grid < s.P * s.R ? (const void*)svd_jacobi<false, false>
-                   : s.VS > 0        ? (const void*)svd_jacobi<true, true>
-                                     : (const void*)svd_jacobi<true, false>;
+  const void* fn = jacobi_kernel(variant);
   if (grid == 1) {  // nothing to be resident with
     SEEMPS_HIP(hipLaunchKernel(fn, dim3(1), dim3(JT), args, 0, stream));
     return SEEMPS_OK;

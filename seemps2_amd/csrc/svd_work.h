@@ -58,6 +58,12 @@ inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 // Blocks, pairs and row chunks of a Jacobi on s.ncol columns of length s.len
 // (set by the caller, as s.use_qr), at most one workgroup per CU.
 void jacobi_shape(SvdShape* s, int num_cu);
+// Forms of the Jacobi kernel: V's rows on workgroups of their own, one work item a
+// workgroup, items strided over the grid.
+enum JacobiVariant { JACOBI_V_APART = 0, JACOBI_LOCAL = 1, JACOBI_STRIDED = 2 };
+// The form and its grid for P pairs of R row chunks (and VS of V's), when lim[v]
+// workgroups of form v can be resident at once; false if no grid can.
+bool jacobi_plan(int64_t P, int64_t R, int64_t VS, const int64_t* lim, int* variant, int* grid);
 // Sweeps on w.W (and w.V unless it is null) until converged; w.ctrl reset and
 // its tiny2 set beforehand, w.sync zero.
 int jacobi_enqueue(const SvdShape& s, const SvdWork& w, hipStream_t stream);
