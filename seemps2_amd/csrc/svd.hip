@@ -387,9 +387,10 @@ __device__ __forceinline__ int64_t block_owner(int64_t nb, int64_t k, int64_t x)
 // what it has (the second index's diagonal entry comes with that pair's
 // rotation), everyone applies it after the barrier.
 //
-// A round takes 0.52 us, two thirds of it instruction issue (48 FP64
-// operations a thread in either role, the rotation's chain of 55); with G and
-// the tile in LDS it took 1.07 us, LDS traffic (100 KB a round).
+// A round takes 0.51 us, two thirds of it instruction issue (48 FP64
+// operations a thread in either role, the rotation's chain of 45); with G and
+// the tile in LDS it took 1.07 us, LDS traffic (100 KB a round).  G's rounds are
+// not unrolled: in fours the 64 x 64 split took 634 us for 625 (more spills).
 constexpr int JT = 768;            // threads
 constexpr int TP = RT + 1;         // padded tile column (complex)
 constexpr int NP = PW / 2;         // pairs a round
@@ -453,9 +454,9 @@ __device__ __forceinline__ double rcp_short(double x) {
 }
 
 // Rotation that annihilates c = G_ab; identity when the pair is orthogonal to
-// tol or either column negligible.  t = tan(angle), the smaller root of
-// t^2 + 2 tau t - 1 = 0, to a few ulp (from the unrefined estimates it was good to
-// 1e-8, a round 0.01 us shorter, and left that much of G_ab to the next sweep).
+// tol or either column negligible.  With d = G_bb - G_aa the tangent is
+// t = w |c|, w = 2 sign(d) / (|d| + sqrt(d^2 + 4 |c|^2)) (the smaller root of
+// t^2 + d t / |c| - 1 = 0), so |c| itself is not needed; all to a few ulp.
 // cs = 1/sqrt(1 + t^2) must be unbiased where it is close to one (jac::rsqrt_nr is):
 // an ulp lost in each of the hundreds of small rotations of a column adds up
 // (1.4e-14 against 8.9e-15 on 64 columns).
@@ -465,17 +466,15 @@ __device__ __forceinline__ Rot pair_rotation(double gaa, double gbb, double2 c, 
   q.cs = 1.0;
   q.gbb = gbb;
   q.s = make_double2(0.0, 0.0);
-  const double s2 = cabs2(c);
+  const double s2 = cabs2(c), d = gbb - gaa;
   const bool any = s2 > 0.0 && gaa > tiny2 && gbb > tiny2 && s2 > (tol2 * gaa) * gbb;
-  const double tau = (gbb - gaa) * (0.5 * rsqrt_short(s2));
-  const double at = fmin(fabs(tau), 1e150);
-  const double u = fma(at, at, 1.0);
-  const double t = copysign(rcp_short(fma(u, rsqrt_short(u), at)), tau);
-  const double cs = jac::rsqrt_nr(fma(t, t, 1.0)), r = jac::rsqrt_nr(s2);
-  const double sn = t * cs * r;
+  const double h = fma(d, d, 4.0 * s2);
+  const double w = copysign(2.0 * rcp_short(fma(h, rsqrt_short(h), fabs(d))), d);
+  const double tc = w * s2;  // t |c|
+  const double cs = jac::rsqrt_nr(fma(w, tc, 1.0)), sn = w * cs;
   if (any) {
     q.cs = cs;
-    q.gbb = fma(t, s2 * r, gbb);
+    q.gbb = gbb + tc;
     q.s = make_double2(c.x * sn, c.y * sn);
   }
   return q;
@@ -508,7 +507,7 @@ __device__ __forceinline__ void inner_level(PairLds& L, Rot* rec, double tol2, d
     double2 ac = L.G[a * GP + c], ad = L.G[a * GP + d];
     double2 bc = L.G[b * GP + c], bd = L.G[b * GP + d];
     double gbb = bd.x;
-#pragma unroll 4
+#pragma unroll 1
     for (int k = 0; k < H; ++k) {
       Rot* rot = rec + k * NP;
       const Rot own = pair_rotation(ac.x, gbb, ad, tol2, tiny2);
@@ -911,7 +910,7 @@ __device__ inline void local_item(int64_t b, int64_t G, int64_t R, int64_t* p, i
 // other CUs shortens it; V's workgroups follow W's by a step or so and hold them up
 // only if they fall two behind (the partial Grams alternate between two buffers) or
 // at the end.  They read the convergence measure but are not counted in the barrier.
-// An inner round 0.53 -> 0.45 us (64 columns).
+// An inner round 0.52 -> 0.44 us (64 columns).
 // !LOCAL: items are strided over the grid, with two grid barriers per step.
 template <bool LOCAL, bool VSEP>
 __global__ __launch_bounds__(JT) void svd_jacobi(SvdShape s, SvdWork w, double tol,
