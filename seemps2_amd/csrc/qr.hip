@@ -38,27 +38,32 @@ struct Reflector {
   bool any;        // false: H = I
 };
 
-// In a column whose squares come near the smallest normal number, v is scaled up by
-// a power of two, so that tau (about 1 / |v|^2) stays finite.  NaN gets a reflector,
-// and spreads.
+// None for a column of squared norm below 1e-300 (tau, about 1 / |v|^2, nears the
+// largest number there); NaN gets one, and spreads.
 __device__ __forceinline__ Reflector make_reflector(double2 alpha, double xnorm2) {
   Reflector h;
   h.beta = alpha.x;
   h.d = h.tau = make_double2(0.0, 0.0);
-  double s = cabs2(alpha) + xnorm2;
-  h.any = !(xnorm2 == 0.0 && alpha.y == 0.0) && s != 0.0;
-  const bool tiny = s < 1e-290;
-  h.up = tiny ? 0x1p500 : 1.0;
+  h.up = 1.0;
+  const double s = cabs2(alpha) + xnorm2;
+  h.any = !(xnorm2 == 0.0 && alpha.y == 0.0) && !(s < 1e-300);
   if (h.any) {
-    s = (s * h.up) * h.up;
-    alpha = make_double2(alpha.x * h.up, alpha.y * h.up);
     const double r = jac::rsqrt_nr(s), sg = (alpha.x >= 0.0) ? -1.0 : 1.0;
     h.beta = sg * (s * r);
     h.d = make_double2(alpha.x - h.beta, alpha.y);
     const double q = jac::rcp_nr(cabs2(h.d)), ib = -sg * r;  // 1 / |d|^2, -1 / beta
     h.tau = make_double2((h.d.x * ib) * q, (h.d.y * ib) * q);
-    h.beta *= tiny ? 0x1p-500 : 1.0;
   }
+  return h;
+}
+
+// The reflector of such a column, v scaled up by a power of two.  Asked for where
+// make_reflector gave none, so that the other columns do not pay for it (a test of the
+// norm and a scale in that chain made the panels 5 % slower).
+__device__ __forceinline__ Reflector tiny_reflector(double2 alpha, double xnorm2) {
+  Reflector h = make_reflector(rscale(0x1p500, alpha), (xnorm2 * 0x1p500) * 0x1p500);
+  h.beta *= 0x1p-500;
+  h.up = 0x1p500;
   return h;
 }
 
@@ -132,8 +137,9 @@ __global__ __launch_bounds__(64 * NW) void qr_panel(double2* __restrict__ A, int
         else
           d[k] = wave::sum2(d[k]);
       }
-      const Reflector h = make_reflector(alpha, nn);
-      if (h.up != 1.0) {
+      Reflector h = make_reflector(alpha, nn);
+      if (!h.any) {
+        h = tiny_reflector(alpha, nn);
 #pragma unroll
         for (int r = 0; r < RPT; ++r) x[r] = rscale(h.up, x[r]);
 #pragma unroll
@@ -396,7 +402,10 @@ __device__ __forceinline__ void long_steps(double2* __restrict__ P, double2* __r
     const int k = min(max(lane, J + 1), NB - 1);
     double2 t = make_double2(0.0, 0.0);
     for (int q = 0; q < NW; ++q) t = cadd(t, L.red[q][k]);
-    const Reflector h = make_reflector(L.row[J + 1], wave::bcast(t.x, J + 1));
+    const double2 alpha = L.row[J + 1];
+    const double nn = wave::bcast(t.x, J + 1);
+    Reflector h = make_reflector(alpha, nn);
+    if (!h.any) h = tiny_reflector(alpha, nn);
     // v^H a_k = conj(d) a_k[c + 1] + up x^H a_k
     if (lane > J + 1 && lane < NB)
       L.f[k] = cmul(make_double2(-h.tau.x, h.tau.y), cfmac(h.d, L.row[k], rscale(h.up, t)));
