@@ -168,3 +168,38 @@ def test_one_rotation_is_exact(K, c):
     assert list(info) == [2, 1]
     s_ref = np.linalg.svd(R, compute_uv=False)
     assert np.abs(S.cpu().numpy() - s_ref).max() < 5e-13 * s_ref[0]
+
+
+@pytest.mark.parametrize("n", [4090, 4100])
+def test_split_long_spectrum(K, n):
+    """The sort and the truncation on spectra that just fit LDS and that do not."""
+    d = torch.linspace(2.0, 1.0, n, dtype=torch.float64, device="cuda")
+    p = torch.from_numpy(np.random.default_rng(n).permutation(n)).cuda()
+    A = torch.diag(d[p]).to(torch.complex128)
+    Ad, Bd, D, err2, s = K.svd_split(A, n, n, 0, 2, 0.0, 2000, want_s=True)
+    assert D == 2000
+    assert float((s - d[:2000]).abs().max()) < 1e-14
+    assert abs(err2 - float((d[2000:] ** 2).sum())) < 1e-11 * err2
+    # entries at most 2, each off by a few ulp
+    assert float((Ad.mH @ Ad - torch.eye(D, device="cuda")).abs().max()) < 1e-14
+    assert float(((Ad @ Bd) - torch.diag(torch.where(d[p] >= d[1999], d[p], 0.0))).abs().max()) < 1e-14
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("m,n", [(3, 2), (16, 16), (40, 30), (70, 90), (1100, 9)])
+def test_split_spreads_nan(K, m, n, bad):
+    """A value that is no number ends in an error or in the result, in every mode and
+    rule, never in factors that look right."""
+    from scipy.linalg import LinAlgError
+
+    A = crandn(np.random.default_rng(m), m, n)
+    A[m // 2, n // 2] = bad
+    for mode in (0, 1):
+        for method in range(4):
+            try:
+                Ad, Bd, D, err2, _ = K.svd_split(K.as_dev(A), m, n, mode, method, 1e-10, 7)
+            except LinAlgError:
+                continue
+            assert 1 <= D <= min(m, n)
+            finite = np.isfinite(K.to_numpy(Ad)).all() and np.isfinite(K.to_numpy(Bd)).all()
+            assert not (finite and np.isfinite(err2)), (mode, method)
