@@ -96,11 +96,11 @@ def parse():
 # (label, M, N, K, opA, opB): the products of a chi=256 (and 128) sweep
 GEMM_SHAPES = [
     ("matvec L.v, chi=256", 1280, 1024, 256, 0, 0),
-    ("matvec second product, chi=256 (split-K)", 1024, 256, 1280, 0, 0),
+    ("matvec second product, op (N, T), chi=256", 1024, 256, 1280, 0, 1),
     ("environment, op (C, N), chi=256", 256, 1280, 512, 3, 0),
     ("environment, chi=256", 1280, 512, 256, 0, 0),
     ("matvec L.v, chi=128", 640, 512, 128, 0, 0),
-    ("matvec second product, chi=128 (split-K)", 512, 128, 640, 0, 0),
+    ("matvec second product, op (N, T), chi=128", 512, 128, 640, 0, 1),
     ("sketch product", 512, 272, 512, 0, 0),
     ("large square", 2048, 2048, 512, 0, 0),
 ]
@@ -123,7 +123,7 @@ def gemm_shapes(reps=100):
         B = torch.randn((N, Kd) if ob in (1, 2) else (Kd, N), dtype=torch.complex128,
                         device="cuda", generator=gen)
         C = K.gemm(A, B, oa, ob)
-        ref = (A.conj() if oa == 3 else A) @ B
+        ref = (A.conj() if oa == 3 else A) @ (B.mT.contiguous() if ob == 1 else B)
         err = ((C - ref).abs().max() / ref.abs().max()).item()
         torch.cuda.synchronize()
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

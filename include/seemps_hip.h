@@ -9,7 +9,9 @@
  *     MPS environments rho[bra, ket], MPO environments L/R[bra, mpo, ket].
  *   - `stream` is a hipStream_t (NULL = default stream).  All work is enqueued on
  *     it; entry points that must return a size to the host (the kept bond
- *     dimension D, eigensolver statistics) synchronise that stream once.
+ *     dimension D, eigensolver statistics) wait for it: for the stream, or for a
+ *     flag that the kernel with the result sets in pinned memory, with the work
+ *     that follows it (the factors) still on the stream when they return.
  *   - Scratch memory is caller-provided (`work`, `work_bytes`); the library never
  *     allocates persistent device memory.  `*_workspace()` gives the bytes needed.
  *   - Return value: SEEMPS_OK or an error code; seemps_last_error() describes it.

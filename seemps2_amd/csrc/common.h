@@ -128,10 +128,10 @@ int zgemm(int opA, int opB, int64_t M, int64_t N, int64_t K, double2 alpha, cons
           int64_t lda, int64_t sA, const void* B, int64_t ldb, int64_t sB, double2 beta, void* C,
           int64_t ldc, int64_t sC, int64_t batch, hipStream_t stream,
           int prec = SEEMPS_PREC_FP64);
-// Split-K GEMM over caller scratch (ws holds splitk_workspace(M, N, K) elements);
-// falls back to zgemm when splitting does not pay or ws is too small.
 // Whether an FP64 product runs on 16 x 16 tiles of four wavefronts each.
 bool gemm_on_small_tiles(int opA, int opB, int64_t M, int64_t N, int64_t K);
+// Split-K GEMM over caller scratch (ws holds splitk_workspace(M, N, K) elements);
+// falls back to zgemm when splitting does not pay or ws is too small.
 int zgemm_ws(int opA, int opB, int64_t M, int64_t N, int64_t K, double2 alpha, const void* A,
              int64_t lda, const void* B, int64_t ldb, double2 beta, void* C, int64_t ldc,
              double2* ws, int64_t ws_elems, hipStream_t stream, int prec = SEEMPS_PREC_FP64);

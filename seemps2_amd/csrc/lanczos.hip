@@ -1,6 +1,7 @@
 // DMRG two-site effective Hamiltonian: operator build, matvec and a Lanczos
 // eigensolver whose Krylov recurrence, tridiagonal eigensolve and Ritz vector
-// stay on the device (one host synchronisation per restart cycle).
+// stay on the device (the host waits for the residual at the end of a restart cycle
+// and, for large operators, at every second step).
 //
 // Replaces QuadraticForm.two_site_operator (src/seemps/operators/quadratic.py:
 // 187-237) and the scipy eigsh / ARPACK call of _diagonalize_two_site
@@ -785,9 +786,9 @@ int eigensolve_impl(int prec, int64_t chiL, int64_t c, int64_t d1, int64_t d2, i
   const double fp32_floor = 1e-5, fp32_start = 1e-4;
   double last_resid = HUGE_VAL;
   // In FP64 cycles the Ritz residual is also tested after steps 4, 6, 8, ...
-  // (one single-block tridiagonal solve and a synchronisation each), so that a
-  // warm start stops well before ncv products; only for operators large enough
-  // that a product outweighs the check.
+  // (a tridiagonal solve at the end of the step's last launch and a wait for its
+  // flag each), so that a warm start stops well before ncv products; only for
+  // operators large enough that a product outweighs the check.
   const bool early = n >= 8192;
   const int64_t first_check = 4, check_every = 2;
   for (cycle = 0; cycle < maxiter; ++cycle) {

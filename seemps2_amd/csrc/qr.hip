@@ -8,12 +8,12 @@
 // rows below are scratch), tau, and the reflectors explicitly: row c of Vall
 // (length len) is v_c, zeros above row c included.
 //
-// Both kernels keep columns in registers, one column's rows spread over the 64
-// lanes of a wavefront, so a dot product is a few FMAs per lane and one
-// wavefront reduction (wave.h).  A panel is one workgroup of 16 wavefronts
+// Up to 1024 rows both kernels keep columns in registers, one column's rows spread
+// over the 64 lanes of a wavefront, so a dot product is a few FMAs per lane and one
+// wavefront reduction (wave.h).  A panel is one workgroup of eight wavefronts
 // with one barrier per column; the trailing columns then take the panel's
 // reflectors one after the other in one launch, every column by itself (no
-// compact-WY factor, no GEMMs).
+// compact-WY factor, no GEMMs).  Longer columns stay in memory.
 //
 // Reflector convention: H = I - tau v v^H with H^H [alpha; x] = [beta; 0], beta
 // real of the sign opposite to Re alpha, v = [alpha - beta; x] (not scaled to a
@@ -463,9 +463,8 @@ inline int rows_per_lane(int64_t L) {
 }
 
 // Panel width of a register panel with r rows per lane: 64 columns up to 128
-// rows, 32 up to 256, 16 up to 512 (four, two, one columns on each of 16
-// wavefronts), 8 beyond (16 rows of two columns a lane do not fit the registers
-// of a full workgroup).
+// rows, 32 up to 256, 16 up to 512, 8 beyond (eight, four, two, one columns on
+// each of eight wavefronts: what the registers hold).
 inline int panel_width(int r) { return r <= 2 ? 64 : r <= 4 ? 32 : r <= 8 ? 16 : 8; }
 
 int panel(int r, double2* A, int64_t len, int64_t j0, int nb, double2* tau, double2* Vall,
