@@ -399,7 +399,7 @@ inline bool b_along_k(int op) { return op == SEEMPS_OP_T || op == SEEMPS_OP_H; }
 // 2048 2048 512 takes 280.1 there against 228.3 with three.)
 // Over 17600 shapes (M, N from 8 to 2500, K from 8 to 12000, the four pairs of
 // contiguous directions, sizes odd and even) the choice takes 1.28 times less than
-// staging everything, 1 % more than the best of the four each time; 0.4 % of them
+// staging everything, 0.8 % more than the best of the four each time; 0.5 % of them
 // are more than 3 % slower than staged.
 Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_cu) {
   if (forced_tile() >= 0 || !gemm_scheme_3m()) return {0, 0};
@@ -444,13 +444,18 @@ Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_
   const int i = u == 1   ? (8 * t16 <= cu ? 0 : 2 * t16 <= cu ? 1 : 2)
                 : u <= 4 ? (int)(2 * u - 1) + (2 * t16 >= (2 * u - 1) * cu)
                          : (u <= 6 ? 9 : 10);
+  // A load along K touches sixteen rows.  Rows a whole number of 128-byte lines long
+  // fall on few of the cache's sets (NT 144 134 704: 13.2 us staged, 12.7 direct);
+  // others bear twice the K (700: 13.3, 10.3; 804: 14.3, 11.5).
+  const bool apart = g > 0 && K % 8 != 0;
   const int64_t hi = !edge   ? upto[g][i]
                      : i < 3 ? upto_edge[g][i]
                              : upto[g][i] + upto[g][i] / 2;
   // with many tiles a short K does not pay for the prologue of each
   int64_t lo = i < 3 ? 1 : t16 / (g == 2 ? (edge ? 16 : 8) : (edge ? 24 : 12));
-  if ((g == 2 || (g == 1 && i >= 3)) && lo < 17) lo = 17;
-  return lo <= K && K <= hi ? Direct{1, 4} : Direct{0, 0};
+  if (apart && i >= 3) lo = lo * 2 / 3;
+  if (((g == 2 && !apart) || (g > 0 && i >= 3)) && lo < 17) lo = 17;
+  return lo <= K && (apart ? (K + 1) / 2 : K) <= hi ? Direct{1, 4} : Direct{0, 0};
 }
 
 template <int OPA, int OPB>

@@ -104,7 +104,8 @@ def test_grouped_gemm_edges(tile, count, opA, opB):
 
 # Both sides of the lines between the direct and the staged kernel (256 CUs): few tiles
 # and a long K, aligned and past an edge; whole and part-empty rounds of the CUs and of
-# the SIMDs; a K too short for many tiles; both operands along K.
+# the SIMDs; a K too short for many tiles; both operands along K,
+# their rows whole cache lines apart or not.
 @pytest.mark.parametrize("opA,opB,M,N,K_,direct", [
     (0, 0, 64, 64, 1024, True), (0, 0, 64, 64, 8192, False), (2, 0, 64, 64, 2048, True),
     (0, 0, 33, 40, 8192, False), (2, 0, 33, 40, 8192, True), (0, 1, 128, 128, 512, True),
@@ -112,7 +113,8 @@ def test_grouped_gemm_edges(tile, count, opA, opB):
     (0, 1, 272, 1000, 256, False), (0, 1, 272, 1000, 768, False), (3, 2, 700, 700, 768, True),
     (2, 0, 640, 512, 256, True), (0, 0, 900, 900, 16, False), (0, 0, 900, 900, 256, True),
     (1, 1, 1024, 1000, 300, True), (1, 0, 1100, 1000, 60, False), (1, 0, 1100, 1000, 333, False),
-    (1, 0, 700, 640, 333, True)])
+    (1, 0, 700, 640, 333, True), (0, 1, 144, 134, 804, True), (0, 1, 144, 134, 800, False),
+    (0, 1, 512, 160, 636, True), (0, 1, 512, 160, 640, False)])
 def test_gemm_route(opA, opB, M, N, K_, direct):
     from seemps2_amd import _lib, kernels as K
 
