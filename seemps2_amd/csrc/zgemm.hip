@@ -454,7 +454,7 @@ Direct choose_direct(int opA, int opB, int64_t M, int64_t N, int64_t K, int num_
   // with many tiles a short K does not pay for the prologue of each
   int64_t lo = i < 3 ? 1 : t16 / (g == 2 ? (edge ? 16 : 8) : (edge ? 24 : 12));
   if (apart && i >= 3) lo = lo * 2 / 3;
-  if (((g == 2 && !apart) || (g > 0 && i >= 3)) && lo < 17) lo = 17;
+  if ((g == 2 || (g == 1 && i >= 3)) && lo < 17) lo = 17;
   return lo <= K && (apart ? (K + 1) / 2 : K) <= hi ? Direct{1, 4} : Direct{0, 0};
 }
 
